@@ -176,6 +176,30 @@ int lsk_rmsnorm_linear_bf16(const void* w_packed, int layout_id, int N, int K,
                             int epilogue, const void* residual, int ldr,
                             void* hip_stream);
 
+/* y[M][K] = bf16((x[m][k] * r[m]) * norm_weight[k]), r[m] = 1 / sqrt(mean_k
+ * x[m][k]^2 + eps) in fp32: the RMSNorm in front of a projection of more rows
+ * than lsk_rmsnorm_linear_bf16 takes.  M >= 1; K a multiple of 512 up to
+ * 4096; x at row stride ldx >= K (a multiple of 8), y contiguous; x, y and
+ * norm_weight 16-byte aligned.  Replaces F.rms_norm of
+ * src/leanstack/runtime/qwen_explicit.py:621-628. */
+int lsk_rmsnorm_bf16(const void* x, int M, int K, int ldx, const void* norm_weight, float eps, void* y,
+                     void* hip_stream);
+
+/* The q and k heads of B * T raw QKV rows ([n_q*d | n_kv*d | n_kv*d] bf16, row
+ * stride ld, rows of one batch consecutive): per-head RMSNorm over d with
+ * q_norm_weight / k_norm_weight and eps, then rotate-half RoPE with row
+ * (b, t) of cos / sin ([d/2] bf16 at b * rope_batch_stride + t *
+ * rope_row_stride elements; stride 0 broadcasts), with a bf16 rounding after
+ * each step as the reference's torch ops round, into q_out [B][n_q][T][d] and
+ * k_out [B][n_kv][T][d].  The v heads are left where they are.  d must be 128;
+ * ld and the rope strides multiples of 8; every pointer 16-byte aligned.
+ * Replaces the norms, RoPE and transposes of
+ * src/leanstack/runtime/qwen_explicit.py:749-770 and :788-806 (RoPE :690-716). */
+int lsk_qk_norm_rope_bf16(const void* qkv, int B, int T, int ld, int n_q, int n_kv, int head_dim,
+                          const void* q_norm_weight, const void* k_norm_weight, float eps,
+                          const void* cos, const void* sin, long long rope_batch_stride,
+                          long long rope_row_stride, void* q_out, void* k_out, void* hip_stream);
+
 /* Device workspace of lsk_decode_attention_bf16 for n_kv kv heads of
  * n_q / n_kv q heads and caches of max_seq_len rows (0 if the geometry is not
  * supported).  Needed once more than 128 rows are attended. */

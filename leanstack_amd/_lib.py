@@ -64,6 +64,13 @@ _SIGNATURES: dict[str, tuple[type | None, list]] = {
         [_c_void, _c_int, _c_int, _c_int, _c_void, _c_int, _c_int, _c_void, ctypes.c_float, _c_void, _c_int, _c_int,
          _c_void, _c_int, _c_void],
     ),
+    "lsk_rmsnorm_bf16": (
+        _c_int, [_c_void, _c_int, _c_int, _c_int, _c_void, ctypes.c_float, _c_void, _c_void]),
+    "lsk_qk_norm_rope_bf16": (
+        _c_int,
+        [_c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void, ctypes.c_float, _c_void, _c_void,
+         ctypes.c_longlong, ctypes.c_longlong, _c_void, _c_void, _c_void],
+    ),
     "lsk_attention_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int]),
     "lsk_decode_attention_bf16": (
         _c_int,

@@ -23,7 +23,7 @@ INCLUDE = REPO_ROOT / "include"
 BUILD_DIR = PACKAGE_DIR / "_build"
 LIBRARY = PACKAGE_DIR / "libleanstack_amd.so"
 
-SOURCES = ("abi.cpp", "host_rules.cpp", "decode.hip", "skinny.hip", "gemm.hip", "stack.hip", "attention.hip",
+SOURCES = ("abi.cpp", "host_rules.cpp", "decode.hip", "skinny.hip", "gemm.hip", "stack.hip", "attention.hip", "rows.hip",
            "noalloc.hip", "probe.hip")
 OFFLOAD_ARCH = "gfx950"
 

@@ -224,6 +224,44 @@ int lsk_rmsnorm_linear_bf16(const void* w_packed, int layout_id, int N, int K, c
   return LSK_OK;
 }
 
+int lsk_rmsnorm_bf16(const void* x, int M, int K, int ldx, const void* norm_weight, float eps, void* y,
+                     void* hip_stream) {
+  lsk::clear_error();
+  if (int st = lsk::check_rmsnorm_args(x, M, K, ldx, norm_weight, eps, y)) return st;
+  hipError_t err = lsk::launch_rms_rows(x, M, K, (size_t)ldx, norm_weight, eps, y, static_cast<hipStream_t>(hip_stream));
+  if (err != hipSuccess) return hip_fail(err, "RMSNorm kernel launch");
+  return LSK_OK;
+}
+
+int lsk_qk_norm_rope_bf16(const void* qkv, int B, int T, int ld, int n_q, int n_kv, int head_dim,
+                          const void* q_norm_weight, const void* k_norm_weight, float eps, const void* cos,
+                          const void* sin, long long rope_batch_stride, long long rope_row_stride, void* q_out,
+                          void* k_out, void* hip_stream) {
+  lsk::clear_error();
+  if (int st = lsk::check_qk_rope_args(qkv, B, T, ld, n_q, n_kv, head_dim, q_norm_weight, k_norm_weight, eps, cos, sin,
+                                       rope_batch_stride, rope_row_stride, q_out, k_out))
+    return st;
+  lsk::QkRopeArgs a;
+  a.qkv = static_cast<const __bf16*>(qkv);
+  a.q_norm_w = static_cast<const __bf16*>(q_norm_weight);
+  a.k_norm_w = static_cast<const __bf16*>(k_norm_weight);
+  a.cos = static_cast<const __bf16*>(cos);
+  a.sin = static_cast<const __bf16*>(sin);
+  a.q_out = static_cast<__bf16*>(q_out);
+  a.k_out = static_cast<__bf16*>(k_out);
+  a.ld = (size_t)ld;
+  a.rope_batch = (size_t)rope_batch_stride;
+  a.rope_row = (size_t)rope_row_stride;
+  a.M = B * T;
+  a.T = T;
+  a.n_q = n_q;
+  a.n_kv = n_kv;
+  a.eps = eps;
+  hipError_t err = lsk::launch_qk_rope(a, static_cast<hipStream_t>(hip_stream));
+  if (err != hipSuccess) return hip_fail(err, "q / k head kernel launch");
+  return LSK_OK;
+}
+
 size_t lsk_attention_workspace_bytes(int n_q, int n_kv, int head_dim, int max_seq_len) {
   if (head_dim != lsk::kAttnHeadDim || n_kv < 1 || n_kv > lsk::kAttnMaxKvHeads || n_q < n_kv || n_q % n_kv != 0 ||
       !lsk::attention_group_supported(n_q / n_kv) || max_seq_len < 1 ||

@@ -41,57 +41,6 @@ constexpr int kHeadDim = kAttnHeadDim;
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
 
-__device__ __forceinline__ float bf16r(float v) { return static_cast<float>(static_cast<__bf16>(v)); }
-
-// 1 / sqrt(ss / n + eps) with the mean rounded before eps is added, as
-// torch's rms_norm computes it (contraction would fuse the two into an fma).
-__device__ __forceinline__ float inv_rms(float ss, int n, float eps) {
-#pragma clang fp contract(off)
-  return 1.0f / sqrtf(ss / static_cast<float>(n) + eps);
-}
-
-// One half of the rotate-half RoPE pair, a*c - b*s (sign = -1) or
-// a*c + b*s (sign = +1), each product rounded to bf16 before the sum, as the
-// reference's separate bf16 tensor ops round them.  Contraction is off: with
-// it the compiler fuses the first product into the sum as one fma and skips
-// that product's rounding.
-__device__ __forceinline__ __bf16 rope_half(float a, float b, float c, float s, float sign) {
-#pragma clang fp contract(off)
-  return static_cast<__bf16>(bf16r(a * c) + sign * bf16r(b * s));
-}
-
-// Wave-wide sum / max with the butterfly's pairing (xor 1, 2, 4, 8 inside a
-// 16-lane row, then (r0 + r1) + (r2 + r3) over the rows).  The in-row steps
-// are DPP moves (quad_perm [1,0,3,2], [2,3,0,1], then row_half_mirror and
-// row_mirror: after the quad steps every lane of a quad holds the quad's
-// value, so mirroring pairs each quad / half with the other one); partners
-// combine the same two values, so every lane of a row holds identical bits.
-// The rows are combined from readlanes, so all lanes get one value.
-template <int kCtrl>
-__device__ __forceinline__ float dpp(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kCtrl, 0xf, 0xf, false));
-}
-
-__device__ __forceinline__ float row_lane(float v, int lane) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-  v += dpp<0xb1>(v);
-  v += dpp<0x4e>(v);
-  v += dpp<0x141>(v);
-  v += dpp<0x140>(v);
-  return (row_lane(v, 0) + row_lane(v, 16)) + (row_lane(v, 32) + row_lane(v, 48));
-}
-
-__device__ __forceinline__ float wave_max(float v) {
-  v = fmaxf(v, dpp<0xb1>(v));
-  v = fmaxf(v, dpp<0x4e>(v));
-  v = fmaxf(v, dpp<0x141>(v));
-  v = fmaxf(v, dpp<0x140>(v));
-  return fmaxf(fmaxf(row_lane(v, 0), row_lane(v, 16)), fmaxf(row_lane(v, 32), row_lane(v, 48)));
-}
-
 struct AttnArgs {
   const __bf16* qkv;       // [n_q*d | n_kv*d | n_kv*d]
   const __bf16* q_norm_w;  // [d]
@@ -294,8 +243,8 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   for (int u = 0; u < kItems; ++u) {
     const int i = wave + kWaves * u;
     const float r = inv_rms(wave_sum(px0[u] * px0[u] + px1[u] * px1[u]), kHeadDim, a.eps);
-    const float n0 = bf16r((px0[u] * r) * pw0[u]);
-    const float n1 = bf16r((px1[u] * r) * pw1[u]);
+    const float n0 = bf16_round((px0[u] * r) * pw0[u]);
+    const float n1 = bf16_round((px1[u] * r) * pw1[u]);
     const __bf16 o0 = rope_half(n0, n1, cs, sn, -1.f);
     const __bf16 o1 = rope_half(n1, n0, cs, sn, 1.f);
     if (i < G) {

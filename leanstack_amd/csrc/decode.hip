@@ -135,13 +135,6 @@ __device__ __forceinline__ float sum_squares(bf16x8_t v) {
   return s;
 }
 
-// 1 / sqrt(ss / n + eps) with the mean rounded before eps is added, as
-// torch's rms_norm computes it (contraction would fuse the two into an fma).
-__device__ __forceinline__ float inv_rms(float ss, int n, float eps) {
-#pragma clang fp contract(off)
-  return 1.0f / sqrtf(ss / static_cast<float>(n) + eps);
-}
-
 // Lanes 0..15 hold this wave's partial sum of squares of rows 0..15; returns
 // r[lane % 16] for active rows and 0 for padding columns, summing the waves'
 // partials in wave order.  Every wave must call it.

@@ -97,6 +97,39 @@ int check_linear_args(const void* w_packed, int layout_id, int N, int K, const v
   return LSK_OK;
 }
 
+int check_rmsnorm_args(const void* x, int M, int K, int ldx, const void* norm_weight, float eps, const void* y) {
+  if (M < 1) return fail(LSK_ERR_INVALID, "M=%d must be positive", M);
+  if (K < 512 || K > 4096 || K % 512 != 0) return fail(LSK_ERR_INVALID, "K=%d must be a multiple of 512 up to 4096", K);
+  if (ldx < K || ldx % 8 != 0) return fail(LSK_ERR_INVALID, "ldx=%d must be a multiple of 8, at least K=%d", ldx, K);
+  if (x == nullptr || norm_weight == nullptr || y == nullptr) return fail(LSK_ERR_INVALID, "null device pointer");
+  if (!aligned(x, 16) || !aligned(norm_weight, 16) || !aligned(y, 16))
+    return fail(LSK_ERR_INVALID, "x, norm_weight and y must be 16-byte aligned");
+  if (!std::isfinite(eps) || eps < 0.f) return fail(LSK_ERR_INVALID, "eps=%g must be finite and >= 0", (double)eps);
+  return LSK_OK;
+}
+
+int check_qk_rope_args(const void* qkv, int B, int T, int ld, int n_q, int n_kv, int head_dim,
+                       const void* q_norm_weight, const void* k_norm_weight, float eps, const void* cos,
+                       const void* sin, long long rope_batch_stride, long long rope_row_stride, const void* q_out,
+                       const void* k_out) {
+  if (head_dim != kAttnHeadDim)
+    return fail(LSK_ERR_INVALID, "head_dim=%d: the row kernel is built for %d", head_dim, kAttnHeadDim);
+  if (n_q < 1 || n_kv < 1 || n_q > 4096 || n_kv > 4096)
+    return fail(LSK_ERR_INVALID, "n_q=%d, n_kv=%d must be 1..4096", n_q, n_kv);
+  if (B < 1 || T < 1 || (long long)B * T > 0x7fffffffLL) return fail(LSK_ERR_INVALID, "B=%d, T=%d rows", B, T);
+  if (ld < (n_q + n_kv) * head_dim || ld % 8 != 0)
+    return fail(LSK_ERR_INVALID, "ld=%d must be a multiple of 8, at least %d", ld, (n_q + n_kv) * head_dim);
+  if (rope_batch_stride < 0 || rope_row_stride < 0 || rope_batch_stride % 8 != 0 || rope_row_stride % 8 != 0)
+    return fail(LSK_ERR_INVALID, "the cos / sin strides must be multiples of 8, not negative");
+  const void* all[] = {qkv, q_norm_weight, k_norm_weight, cos, sin, q_out, k_out};
+  for (const void* p : all) {
+    if (p == nullptr) return fail(LSK_ERR_INVALID, "null device pointer");
+    if (!aligned(p, 16)) return fail(LSK_ERR_INVALID, "device pointers must be 16-byte aligned");
+  }
+  if (!std::isfinite(eps) || eps < 0.f) return fail(LSK_ERR_INVALID, "eps=%g must be finite and >= 0", (double)eps);
+  return LSK_OK;
+}
+
 int check_attention_args(const void* qkv, int n_q, int n_kv, int head_dim, const void* q_norm_weight,
                          const void* k_norm_weight, float eps, const void* cos, const void* sin, const void* k_cache,
                          const void* v_cache, int max_seq_len, float scale, const void* out) {

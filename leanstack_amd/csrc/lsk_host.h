@@ -77,6 +77,13 @@ int check_shape(int layout_id, int N, int K);
 int check_linear_args(const void* w_packed, int layout_id, int N, int K, const void* x, int M, int ldx,
                       const void* y, int ldy, int epilogue, const void* residual, int ldr);
 
+// Argument rules of lsk_rmsnorm_bf16 and lsk_qk_norm_rope_bf16.
+int check_rmsnorm_args(const void* x, int M, int K, int ldx, const void* norm_weight, float eps, const void* y);
+int check_qk_rope_args(const void* qkv, int B, int T, int ld, int n_q, int n_kv, int head_dim,
+                       const void* q_norm_weight, const void* k_norm_weight, float eps, const void* cos,
+                       const void* sin, long long rope_batch_stride, long long rope_row_stride, const void* q_out,
+                       const void* k_out);
+
 // Argument rules shared by both decode attention entry points (all but pos
 // and the workspace).
 int check_attention_args(const void* qkv, int n_q, int n_kv, int head_dim, const void* q_norm_weight,

@@ -83,6 +83,55 @@ __device__ __forceinline__ float silu_mul_bf16(float g_acc, float u_acc) {
   return bf16_round(s * u);
 }
 
+// 1 / sqrt(ss / n + eps) with the mean rounded before eps is added, as
+// torch's rms_norm computes it (contraction would fuse the two into an fma).
+__device__ __forceinline__ float inv_rms(float ss, int n, float eps) {
+#pragma clang fp contract(off)
+  return 1.0f / sqrtf(ss / static_cast<float>(n) + eps);
+}
+
+// One half of the rotate-half RoPE pair, a*c - b*s (sign = -1) or
+// a*c + b*s (sign = +1), each product rounded to bf16 before the sum, as the
+// reference's separate bf16 tensor ops round them.  Contraction is off: with
+// it the compiler fuses the first product into the sum as one fma and skips
+// that product's rounding.
+__device__ __forceinline__ __bf16 rope_half(float a, float b, float c, float s, float sign) {
+#pragma clang fp contract(off)
+  return static_cast<__bf16>(bf16_round(a * c) + sign * bf16_round(b * s));
+}
+
+// Wave-wide sum / max with the butterfly's pairing (xor 1, 2, 4, 8 inside a
+// 16-lane row, then (r0 + r1) + (r2 + r3) over the rows).  The in-row steps
+// are DPP moves (quad_perm [1,0,3,2], [2,3,0,1], then row_half_mirror and
+// row_mirror: after the quad steps every lane of a quad holds the quad's
+// value, so mirroring pairs each quad / half with the other one); partners
+// combine the same two values, so every lane of a row holds identical bits.
+// The rows are combined from readlanes, so all lanes get one value.
+template <int kCtrl>
+__device__ __forceinline__ float dpp(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kCtrl, 0xf, 0xf, false));
+}
+
+__device__ __forceinline__ float row_lane(float v, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+
+__device__ __forceinline__ float wave_sum(float v) {
+  v += dpp<0xb1>(v);
+  v += dpp<0x4e>(v);
+  v += dpp<0x141>(v);
+  v += dpp<0x140>(v);
+  return (row_lane(v, 0) + row_lane(v, 16)) + (row_lane(v, 32) + row_lane(v, 48));
+}
+
+__device__ __forceinline__ float wave_max(float v) {
+  v = fmaxf(v, dpp<0xb1>(v));
+  v = fmaxf(v, dpp<0x4e>(v));
+  v = fmaxf(v, dpp<0x141>(v));
+  v = fmaxf(v, dpp<0x140>(v));
+  return fmaxf(fmaxf(row_lane(v, 0), row_lane(v, 16)), fmaxf(row_lane(v, 32), row_lane(v, 48)));
+}
+
 // One projection of a stack program, as the kernel reads it (64 bytes).
 struct StackDesc {
   const bf16x8_t* w;
@@ -162,6 +211,23 @@ hipError_t launch_decode_attention_at(const void* qkv, int n_q, int n_kv, const 
                                       float eps, const void* cos_table, const void* sin_table, void* k_cache,
                                       void* v_cache, int s_max, const int* pos_device, float scale, void* out,
                                       void* workspace, size_t ws_bytes, hipStream_t stream);
+
+// RMSNorm of M rows of K values (row stride ldx, K = 512..4096 in steps of
+// 512) into contiguous rows of y (rows.hip).
+hipError_t launch_rms_rows(const void* x, int M, int K, size_t ldx, const void* w, float eps, void* y,
+                           hipStream_t stream);
+
+// q and k heads of M = B * T raw QKV rows [n_q*d | n_kv*d | ...] at stride ld:
+// RMSNorm, RoPE with cos / sin row (b, t) at b * rope_batch + t * rope_row,
+// written to q_out [B][n_q][T][d] and k_out [B][n_kv][T][d] (rows.hip).
+struct QkRopeArgs {
+  const __bf16 *qkv, *q_norm_w, *k_norm_w, *cos, *sin;
+  __bf16 *q_out, *k_out;
+  size_t ld, rope_batch, rope_row;
+  int M, T, n_q, n_kv;
+  float eps;
+};
+hipError_t launch_qk_rope(const QkRopeArgs& a, hipStream_t stream);
 
 // Number of scoring workgroups (= argmax partials per row) the lm_head
 // kernel uses for V vocab rows (V % 16 == 0): with NB = V / 16 row-blocks,

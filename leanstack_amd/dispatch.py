@@ -26,6 +26,7 @@ Differences from the reference, on purpose:
 
 from __future__ import annotations
 
+import math
 import os
 
 import torch
@@ -34,12 +35,37 @@ import torch.nn.functional as F
 from . import _lib, kernels
 from .layout import PackedWeight
 
-# ---------------------------------------------------------------- torch glue
-# (out of this path's scope; restated with the reference's semantics)
+# ---------------------------------------------------------------- row work
+# (what stands between the projections, with the reference's semantics: HIP
+# kernels for plain eager bfloat16 calls on the GPU, torch ops for any other)
+
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def _plain_eager(*tensors: torch.Tensor) -> bool:
+    """Whether a call on these tensors is one that a HIP kernel may stand in
+    for: bfloat16 GPU tensors of one device at 16-byte aligned addresses, and
+    nothing around the call that follows torch ops one by one (autograd, forward-mode
+    AD, functorch transforms, tracing, compilation, autocast, torch modes)."""
+    device = tensors[0].device
+    if device.type != "cuda" or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda"):
+        return False
+    c = torch._C
+    if (c._get_tracing_state() is not None or c._len_torch_dispatch_stack() or c._len_torch_function_stack()
+            or c._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0):
+        return False
+    grad = torch.is_grad_enabled()
+    return all(type(t) in _PLAIN_TYPES and t.dtype is torch.bfloat16 and t.device == device
+               and not (grad and t.requires_grad) and t.data_ptr() % 16 == 0 for t in tensors)
 
 
 def qwen_rmsnorm(hidden_states: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """F.rms_norm over the last dim (qwen_explicit.py:621-628)."""
+    k = hidden_states.shape[-1]
+    if (k % 512 == 0 and 0 < k <= kernels.RMSNORM_MAX_K and weight.shape == (k,) and isinstance(eps, float)
+            and 0.0 <= eps < math.inf and _plain_eager(hidden_states, weight) and hidden_states.is_contiguous()
+            and weight.is_contiguous()):
+        return kernels.rmsnorm_rows(hidden_states, weight, eps)
     return F.rms_norm(hidden_states, normalized_shape=(hidden_states.shape[-1],), weight=weight, eps=eps)
 
 
@@ -100,12 +126,37 @@ def _norm_gate_up(hidden_states, norm_weight, eps, gu_w: PackedWeight):
     return kernels.linear(qwen_rmsnorm(hidden_states, norm_weight, eps), gu_w, epilogue=_lib.EPI_SILU_MUL)
 
 
+def _qk_kernel_serves(qkv_states, q_proj_out_dim, k_proj_out_dim, num_attention_heads, num_key_value_heads, head_dim,
+                      q_norm_weight, k_norm_weight, cos, sin, rms_norm_eps) -> bool:
+    """Whether the q / k head kernel computes exactly what the torch ops
+    below it would for these arguments: 128-wide heads, [128] norm weights,
+    and cos / sin that broadcast over [B, T] rows as their shapes say."""
+    b, t, n = qkv_states.shape
+    return (head_dim == 128 and q_proj_out_dim == num_attention_heads * 128
+            and k_proj_out_dim == num_key_value_heads * 128 and n == q_proj_out_dim + 2 * k_proj_out_dim
+            and q_norm_weight.shape == (128,) and k_norm_weight.shape == (128,)
+            and cos.dim() == 3 and cos.shape == sin.shape and cos.stride() == sin.stride()
+            and cos.shape[0] in (1, b) and cos.shape[1] in (1, t) and cos.shape[2] == 64 and cos.stride(2) == 1
+            and cos.stride(0) % 8 == 0 and cos.stride(1) % 8 == 0
+            and isinstance(rms_norm_eps, float) and 0.0 <= rms_norm_eps < math.inf
+            and _plain_eager(qkv_states, q_norm_weight, k_norm_weight, cos, sin)
+            and q_norm_weight.is_contiguous() and k_norm_weight.is_contiguous())
+
+
 def _semantic_attention_qkv(hidden_states, qkv_proj_weight, q_proj_out_dim, k_proj_out_dim, num_attention_heads,
                             num_key_value_heads, head_dim, q_norm_weight, k_norm_weight, cos, sin, rms_norm_eps):
     """M>1 fused QKV (qwen_explicit.py:733-770): [B,T,H] -> q [B,nq,T,d], k/v [B,nkv,T,d]."""
     w = _require_packed(qkv_proj_weight, "qkv_proj_weight")
     batch_size, query_len, _ = hidden_states.shape
     qkv_states = kernels.linear(hidden_states, w)
+    if _qk_kernel_serves(qkv_states, q_proj_out_dim, k_proj_out_dim, num_attention_heads, num_key_value_heads, head_dim,
+                         q_norm_weight, k_norm_weight, cos, sin, rms_norm_eps):
+        query_states, key_states = kernels.qk_norm_rope(
+            qkv_states, q_norm_weight, k_norm_weight, rms_norm_eps, cos, sin,
+            num_attention_heads=num_attention_heads, num_key_value_heads=num_key_value_heads)
+        value_states = qkv_states[..., q_proj_out_dim + k_proj_out_dim :].view(
+            batch_size, query_len, num_key_value_heads, head_dim).transpose(1, 2)
+        return query_states, key_states, value_states
     query_states, key_states, value_states = torch.split(
         qkv_states, (q_proj_out_dim, k_proj_out_dim, k_proj_out_dim), dim=-1)
     query_states = query_states.view(batch_size, query_len, num_attention_heads, head_dim)
@@ -132,6 +183,13 @@ def _semantic_attention_qkv_vector(hidden_states, qkv_proj_weight, q_proj_out_di
 def _qkv_heads_vector(qkv_states, q_proj_out_dim, k_proj_out_dim, num_attention_heads, num_key_value_heads,
                       head_dim, q_norm_weight, k_norm_weight, cos, sin, rms_norm_eps):
     """Split a [qkv] row into heads, q/k norm and RoPE (qwen_explicit.py:788-806)."""
+    if _qk_kernel_serves(qkv_states.view(1, 1, -1), q_proj_out_dim, k_proj_out_dim, num_attention_heads,
+                         num_key_value_heads, head_dim, q_norm_weight, k_norm_weight, cos, sin, rms_norm_eps):
+        query_states, key_states = kernels.qk_norm_rope(
+            qkv_states.view(1, 1, -1), q_norm_weight, k_norm_weight, rms_norm_eps, cos, sin,
+            num_attention_heads=num_attention_heads, num_key_value_heads=num_key_value_heads)
+        return query_states, key_states, qkv_states[q_proj_out_dim + k_proj_out_dim :].view(
+            1, num_key_value_heads, 1, head_dim)
     query_states, key_states, value_states = torch.split(
         qkv_states, (q_proj_out_dim, k_proj_out_dim, k_proj_out_dim), dim=0)
     query_states = F.rms_norm(query_states.view(1, num_attention_heads, head_dim), normalized_shape=(head_dim,),

@@ -241,6 +241,71 @@ def rmsnorm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, weigh
     return out
 
 
+RMSNORM_MAX_K = 4096
+
+
+def rmsnorm_rows(x: torch.Tensor, norm_weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """rms_norm(x) over the last dim, one bf16 rounding, for contiguous
+    bfloat16 x[..., K] with K a multiple of 512 up to RMSNORM_MAX_K."""
+    k = x.shape[-1]
+    if x.dtype != torch.bfloat16 or norm_weight.dtype != torch.bfloat16 or norm_weight.shape != (k,):
+        raise ValueError(f"x and norm_weight must be bfloat16 [..., K] and [K], got {x.dtype} {tuple(x.shape)} and "
+                         f"{norm_weight.dtype} {tuple(norm_weight.shape)}")
+    if not (x.is_contiguous() and norm_weight.is_contiguous()):
+        raise ValueError("x and norm_weight must be contiguous")
+    _require_device(x, "x")
+    _require_device(norm_weight, "norm_weight")
+    dev = _one_device(x, (norm_weight, "norm_weight"))
+    out = torch.empty_like(x)
+    m = x.numel() // k if k else 0
+    if m == 0:
+        return out
+    with torch.cuda.device(dev):
+        status = _lib.load().lsk_rmsnorm_bf16(x.data_ptr(), m, k, k, norm_weight.data_ptr(), float(eps),
+                                              out.data_ptr(), stream_handle())
+    _lib.check(status, "lsk_rmsnorm_bf16")
+    return out
+
+
+def qk_norm_rope(qkv: torch.Tensor, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, eps: float,
+                 cos: torch.Tensor, sin: torch.Tensor, *, num_attention_heads: int,
+                 num_key_value_heads: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """q [B, n_q, T, d] and k [B, n_kv, T, d] of raw QKV rows [B, T, (n_q + 2 n_kv) d]
+    (contiguous bfloat16, d = 128): per-head RMSNorm and rotate-half RoPE in
+    one kernel.  cos / sin: [B or 1, T or 1, d/2] bfloat16 with equal strides,
+    rows contiguous."""
+    b, t, n = qkv.shape
+    n_q, n_kv = num_attention_heads, num_key_value_heads
+    d = n // (n_q + 2 * n_kv)
+    if not qkv.is_contiguous() or n != (n_q + 2 * n_kv) * d:
+        raise ValueError(f"qkv must be contiguous [B, T, ({n_q} + 2 * {n_kv}) * d] rows, got {tuple(qkv.shape)}")
+    for x, what in ((qkv, "qkv"), (q_norm_weight, "q_norm_weight"), (k_norm_weight, "k_norm_weight"), (cos, "cos"),
+                    (sin, "sin")):
+        _require_device(x, what)
+        if x.dtype != torch.bfloat16:
+            raise ValueError(f"{what} must be bfloat16, got {x.dtype}")
+    if q_norm_weight.shape != (d,) or k_norm_weight.shape != (d,) or not (q_norm_weight.is_contiguous()
+                                                                           and k_norm_weight.is_contiguous()):
+        raise ValueError(f"the q / k norm weights must be contiguous [{d}]")
+    if (cos.dim() != 3 or cos.shape != sin.shape or cos.stride() != sin.stride() or cos.shape[0] not in (1, b)
+            or cos.shape[1] not in (1, t) or cos.shape[2] != d // 2 or cos.stride(2) != 1):
+        raise ValueError(f"cos / sin must be [{b} or 1, {t} or 1, {d // 2}] with equal strides and contiguous rows, got "
+                         f"{tuple(cos.shape)} / {tuple(sin.shape)}")
+    dev = _one_device(qkv, (q_norm_weight, "q_norm_weight"), (k_norm_weight, "k_norm_weight"), (cos, "cos"),
+                      (sin, "sin"))
+    q = torch.empty((b, n_q, t, d), device=qkv.device, dtype=torch.bfloat16)
+    k = torch.empty((b, n_kv, t, d), device=qkv.device, dtype=torch.bfloat16)
+    if b * t == 0:
+        return q, k
+    with torch.cuda.device(dev):
+        status = _lib.load().lsk_qk_norm_rope_bf16(
+            qkv.data_ptr(), b, t, n, n_q, n_kv, d, q_norm_weight.data_ptr(), k_norm_weight.data_ptr(), float(eps),
+            cos.data_ptr(), sin.data_ptr(), cos.stride(0) if cos.shape[0] > 1 else 0,
+            cos.stride(1) if cos.shape[1] > 1 else 0, q.data_ptr(), k.data_ptr(), stream_handle())
+    _lib.check(status, "lsk_qk_norm_rope_bf16")
+    return q, k
+
+
 _attention_workspaces: dict[tuple[int, int], torch.Tensor] = {}
 
 
