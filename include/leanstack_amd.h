@@ -252,6 +252,18 @@ int lsk_decode_attention_at_bf16(const void* qkv, int n_q, int n_kv, int head_di
                                  float scale, void* out, void* workspace, size_t ws_bytes,
                                  void* hip_stream);
 
+/* Attention of one query row over rows that are already cached, for callers
+ * that append them themselves: out[n_q*d] = softmax(q K^T * scale) V over
+ * `rows` rows, q heads [n_q*d] as given (normed and rotated), k / v the rows
+ * [rows][d] of each kv head, `kv_head_stride` elements from one head to the
+ * next (a multiple of 8, at least rows * d).  Geometry limits, chunks and
+ * workspace as for lsk_decode_attention_bf16 with max_seq_len = rows.
+ * Replaces F.scaled_dot_product_attention of
+ * src/leanstack/runtime/qwen_explicit.py:894-912. */
+int lsk_gqa_attention_bf16(const void* q, int n_q, int n_kv, int head_dim, const void* k, const void* v,
+                           long long kv_head_stride, int rows, float scale, void* out, void* workspace,
+                           size_t ws_bytes, void* hip_stream);
+
 /* Greedy lm_head: out_idx[m] = argmax_v sum_k f32(W[v][k]) * f32(x[m][k]) for
  * m < M (M = 1..16), lowest index on ties.  V % 16 == 0 (whole packed
  * row-blocks; a tensor-parallel vocab shard, e.g. 151936 / 8 = 18992, has an

@@ -320,6 +320,21 @@ int lsk_decode_attention_at_bf16(const void* qkv, int n_q, int n_kv, int head_di
   return LSK_OK;
 }
 
+int lsk_gqa_attention_bf16(const void* q, int n_q, int n_kv, int head_dim, const void* k, const void* v,
+                           long long kv_head_stride, int rows, float scale, void* out, void* workspace,
+                           size_t ws_bytes, void* hip_stream) {
+  lsk::clear_error();
+  // The norm and rope arguments of the shared rules do not exist here.
+  if (int st = lsk::check_attention_args(q, n_q, n_kv, head_dim, q, q, 0.f, q, q, k, v, rows, scale, out)) return st;
+  if (kv_head_stride < (long long)rows * head_dim || kv_head_stride % 8 != 0)
+    return fail(LSK_ERR_INVALID, "kv_head_stride=%lld must be a multiple of 8, at least rows * d", kv_head_stride);
+  if (int st = check_attention_workspace(n_q, n_kv, rows, rows, workspace, ws_bytes)) return st;
+  hipError_t err = lsk::launch_gqa_attention(q, n_q, n_kv, k, v, (size_t)kv_head_stride, rows, scale, out, workspace,
+                                             ws_bytes, static_cast<hipStream_t>(hip_stream));
+  if (err != hipSuccess) return hip_fail(err, "attention kernel launch");
+  return LSK_OK;
+}
+
 namespace {
 
 // Checks and launch shared by the plain and the RMSNorm lm_head entry points.

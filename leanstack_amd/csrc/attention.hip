@@ -42,13 +42,14 @@ constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
 
 struct AttnArgs {
-  const __bf16* qkv;       // [n_q*d | n_kv*d | n_kv*d]
+  const __bf16* qkv;       // [n_q*d | n_kv*d | n_kv*d]; kGiven: the q heads, [n_q*d]
   const __bf16* q_norm_w;  // [d]
   const __bf16* k_norm_w;  // [d]
   const __bf16* cos;       // [d/2], this position
   const __bf16* sin;       // [d/2]
-  __bf16* k_cache;         // [n_kv][s_max][d], this layer
+  __bf16* k_cache;         // [n_kv][s_max][d], this layer; kGiven: [n_kv] blocks of rows, kv_stride apart
   __bf16* v_cache;
+  size_t kv_stride;        // elements from one kv head's rows to the next one's
   __bf16* out;             // [n_q*d]
   unsigned* counters;      // workspace: one arrival counter per kv head
   unsigned char* partials; // workspace: one AttnPartial slot per (kv head, chunk)
@@ -133,19 +134,27 @@ __device__ __forceinline__ void combine_chunks(const AttnArgs& a, __amdgpu_buffe
   }
 }
 
-// DYN: pos is read from device memory (a.pos_ptr), cos / sin are the whole
+// Where the rows attended come from: a decode token at a position the host
+// gives, one at a position read from device memory, or q heads and cached
+// rows given as they are (no norms, no RoPE, no append: pos is the last row).
+// kGiven takes the place of an fp32 softmax(q K^T) V in torch ops, which
+// expanded and converted the caches on every call: 9.0 us against 95 us of
+// kernels (and 13 launches) at 700 rows.
+enum AttnMode { kHostPos, kDevicePos, kGiven };
+
+// kDevicePos: pos is read from device memory (a.pos_ptr), cos / sin are the whole
 // position tables ([s_max][d/2]), and the chunk size and count follow from
 // pos here; the grid holds the most chunks max_seq_len can need and the
 // workgroups past this pos's count leave at once.  A pos outside
 // [0, s_max) leaves every buffer untouched.
-template <int G, int NU, bool DYN>
+template <int G, int NU, AttnMode MODE>
 __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs args) {
   static_assert(G >= 1 && G <= 16, "q heads per kv head are the MFMA B columns");
   constexpr int kGroups = NU;              // 16-row groups per wave
   constexpr int kRows = 16 * kWaves * NU;  // rows per workgroup at most: 128 NU
   constexpr int kMaxChunks = kAttnMaxChunks;
   AttnArgs a = args;
-  if constexpr (DYN) {
+  if constexpr (MODE == kDevicePos) {
     const int pos = *args.pos_ptr;
     if (pos < 0 || pos >= a.s_max) return;
     a.pos = pos;
@@ -170,7 +179,8 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   // row are skipped, so short contexts cost little and the waves share the
   // rows evenly.
   auto lb = [&](int u) { return 16 * (wave + kWaves * u); };
-  const bool has_new = a.pos >= row0 && a.pos < row0 + rows;
+  const bool has_new = MODE != kGiven && a.pos >= row0 && a.pos < row0 + rows;
+  const int cached = MODE == kGiven ? L : a.pos;  // rows read from the caches
 
   __shared__ __align__(16) __bf16 qs[16][kHeadDim];     // rotated q heads; rows >= G are zero
   __shared__ __align__(16) __bf16 kv_new[2][kHeadDim];  // this token's rotated k and its v
@@ -194,6 +204,12 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
 #pragma unroll
   for (int u = 0; u < kItems; ++u) {
     const int i = wave + kWaves * u;
+    if constexpr (MODE == kGiven) {
+      const __bf16* src = a.qkv + (size_t)(j * G + (i < G ? i : G - 1)) * kHeadDim;
+      px0[u] = static_cast<float>(src[lane]);
+      px1[u] = static_cast<float>(src[lane + 64]);
+      continue;
+    }
     const bool is_k = i == G;
     const int src_head = is_k ? a.n_q + j : j * G + (i < G ? i : G - 1);
     const __bf16* src = a.qkv + (size_t)src_head * kHeadDim;
@@ -203,19 +219,23 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
     pw0[u] = static_cast<float>(nw[lane]);
     pw1[u] = static_cast<float>(nw[lane + 64]);
   }
-  const float cs = static_cast<float>(a.cos[lane]);
-  const float sn = static_cast<float>(a.sin[lane]);
-  const __bf16* vsrc = a.qkv + ((size_t)a.n_q + a.n_kv + j) * kHeadDim;
-  const __bf16 v_new0 = vsrc[lane];
-  const __bf16 v_new1 = vsrc[lane + 64];
+  float cs = 0.f, sn = 0.f;
+  __bf16 v_new0 = __bf16(0.f), v_new1 = __bf16(0.f);
+  if constexpr (MODE != kGiven) {
+    cs = static_cast<float>(a.cos[lane]);
+    sn = static_cast<float>(a.sin[lane]);
+    const __bf16* vsrc = a.qkv + ((size_t)a.n_q + a.n_kv + j) * kHeadDim;
+    v_new0 = vsrc[lane];
+    v_new1 = vsrc[lane + 64];
+  }
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- cache rows of this wave (they do not depend on q).  K as MFMA A
   // fragments: group u, lane (g, c) = row lb(u) + c, dims 32kt + 8g .. +7.
   // V: lane (g, c) = dims 8c .. 8c+7 of rows lb(u) + 4i + g.  Row pos is this
   // token's (from LDS below); rows past it are not read.
-  const __bf16* kbase = a.k_cache + (size_t)j * a.s_max * kHeadDim;
-  const __bf16* vbase = a.v_cache + (size_t)j * a.s_max * kHeadDim;
+  const __bf16* kbase = a.k_cache + (size_t)j * a.kv_stride;
+  const __bf16* vbase = a.v_cache + (size_t)j * a.kv_stride;
   bf16x8_t kf[kGroups][4];
   bf16x8_t vf[kGroups][4];
 #pragma unroll
@@ -224,7 +244,7 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
       bf16x8_t v = {};
-      if (t < a.pos && lb(u) < rows)
+      if (t < cached && lb(u) < rows)
         v = *reinterpret_cast<const bf16x8_t*>(kbase + (size_t)t * kHeadDim + 32 * kt + 8 * g);
       kf[u][kt] = v;
     }
@@ -232,7 +252,7 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
     for (int i = 0; i < 4; ++i) {
       const int tv = row0 + lb(u) + 4 * i + g;
       bf16x8_t v = {};
-      if (tv < a.pos && lb(u) < rows) v = *reinterpret_cast<const bf16x8_t*>(vbase + (size_t)tv * kHeadDim + 8 * c);
+      if (tv < cached && lb(u) < rows) v = *reinterpret_cast<const bf16x8_t*>(vbase + (size_t)tv * kHeadDim + 8 * c);
       vf[u][i] = v;
     }
   }
@@ -242,6 +262,13 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
 #pragma unroll
   for (int u = 0; u < kItems; ++u) {
     const int i = wave + kWaves * u;
+    if constexpr (MODE == kGiven) {
+      if (i < G) {
+        qs[i][lane] = static_cast<__bf16>(px0[u]);
+        qs[i][lane + 64] = static_cast<__bf16>(px1[u]);
+      }
+      continue;
+    }
     const float r = inv_rms(wave_sum(px0[u] * px0[u] + px1[u] * px1[u]), kHeadDim, a.eps);
     const float n0 = bf16_round((px0[u] * r) * pw0[u]);
     const float n1 = bf16_round((px1[u] * r) * pw1[u]);
@@ -255,8 +282,8 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
       kv_new[0][lane + 64] = o1;
       kv_new[1][lane] = v_new0;
       kv_new[1][lane + 64] = v_new1;
-      __bf16* kc = a.k_cache + ((size_t)j * a.s_max + a.pos) * kHeadDim;
-      __bf16* vc = a.v_cache + ((size_t)j * a.s_max + a.pos) * kHeadDim;
+      __bf16* kc = a.k_cache + (size_t)j * a.kv_stride + (size_t)a.pos * kHeadDim;
+      __bf16* vc = a.v_cache + (size_t)j * a.kv_stride + (size_t)a.pos * kHeadDim;
       kc[lane] = o0;
       kc[lane + 64] = o1;
       vc[lane] = v_new0;
@@ -319,7 +346,10 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
 #pragma unroll
     for (int u = 0; u < kRows / 64; ++u) {
       if (64 * u >= n) break;
-      const float e = lane + 64 * u < n ? expf(sv[u] - m) : 0.f;
+      // A chunk of -inf scores only has weight 0 beside other chunks (given
+      // rows may hold any values), not the NaN of -inf - -inf.
+      const bool live = lane + 64 * u < n && !(MODE == kGiven && m == -__builtin_huge_valf());
+      const float e = live ? expf(sv[u] - m) : 0.f;
       sc[h][lane + 64 * u] = e;
       sum += e;
     }
@@ -430,39 +460,39 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   if (threadIdx.x == 0) __hip_atomic_store(a.counters + j, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int G, int NU, bool DYN = false>
+template <int G, int NU, AttnMode MODE>
 hipError_t launch_gu(const AttnArgs& a, hipStream_t stream) {
-  launch_kernel(decode_attention_kernel<G, NU, DYN>, dim3(a.n_kv * a.grid_chunks), dim3(kThreads), 0, stream, a);
+  launch_kernel(decode_attention_kernel<G, NU, MODE>, dim3(a.n_kv * a.grid_chunks), dim3(kThreads), 0, stream, a);
   return hipGetLastError();
 }
 
-template <int G>
-hipError_t launch_dyn(const AttnArgs& a, int nu, hipStream_t stream) {
+template <int G, AttnMode MODE>
+hipError_t launch_g(const AttnArgs& a, int nu, hipStream_t stream) {
   switch (nu) {
     case 1:
-      return launch_gu<G, 1, true>(a, stream);
+      return launch_gu<G, 1, MODE>(a, stream);
     case 2:
-      return launch_gu<G, 2, true>(a, stream);
+      return launch_gu<G, 2, MODE>(a, stream);
     case 3:
-      return launch_gu<G, 3, true>(a, stream);
+      return launch_gu<G, 3, MODE>(a, stream);
     case 4:
-      return launch_gu<G, 4, true>(a, stream);
+      return launch_gu<G, 4, MODE>(a, stream);
     default:
       return hipErrorInvalidValue;
   }
 }
 
-template <int G>
-hipError_t launch_g(const AttnArgs& a, int nu, hipStream_t stream) {
-  switch (nu) {
+template <AttnMode MODE>
+hipError_t launch_mode(const AttnArgs& a, int nu, hipStream_t stream) {
+  switch (a.n_q / a.n_kv) {
     case 1:
-      return launch_gu<G, 1>(a, stream);
+      return launch_g<1, MODE>(a, nu, stream);
     case 2:
-      return launch_gu<G, 2>(a, stream);
-    case 3:
-      return launch_gu<G, 3>(a, stream);
+      return launch_g<2, MODE>(a, nu, stream);
     case 4:
-      return launch_gu<G, 4>(a, stream);
+      return launch_g<4, MODE>(a, nu, stream);
+    case 8:
+      return launch_g<8, MODE>(a, nu, stream);
     default:
       return hipErrorInvalidValue;
   }
@@ -494,6 +524,7 @@ AttnArgs common_args(const void* qkv, int n_q, int n_kv, const void* q_norm_w, c
   a.n_q = n_q;
   a.n_kv = n_kv;
   a.s_max = s_max;
+  a.kv_stride = (size_t)s_max * kHeadDim;
   a.pos = 0;
   a.chunks = 1;
   a.grid_chunks = 1;
@@ -521,18 +552,20 @@ hipError_t launch_decode_attention(const void* qkv, int n_q, int n_kv, const voi
   const int nu = (rows + 127) / 128;  // 16-row groups per wave: 8 waves x 16 rows x nu cover the chunk
   a.chunks = (pos + 1 + rows - 1) / rows;
   a.grid_chunks = a.chunks;
-  switch (n_q / n_kv) {
-    case 1:
-      return launch_g<1>(a, nu, stream);
-    case 2:
-      return launch_g<2>(a, nu, stream);
-    case 4:
-      return launch_g<4>(a, nu, stream);
-    case 8:
-      return launch_g<8>(a, nu, stream);
-    default:
-      return hipErrorInvalidValue;
-  }
+  return launch_mode<kHostPos>(a, nu, stream);
+}
+
+hipError_t launch_gqa_attention(const void* q, int n_q, int n_kv, const void* k, const void* v, size_t kv_stride,
+                                int rows, float scale, void* out, void* workspace, size_t ws_bytes,
+                                hipStream_t stream) {
+  AttnArgs a = common_args(q, n_q, n_kv, nullptr, nullptr, 0.f, nullptr, nullptr, const_cast<void*>(k),
+                           const_cast<void*>(v), rows, scale, out, workspace, ws_bytes);
+  a.kv_stride = kv_stride;
+  a.pos = rows - 1;
+  const int per_chunk = attention_chunk_rows(rows);
+  a.chunks = (rows + per_chunk - 1) / per_chunk;
+  a.grid_chunks = a.chunks;
+  return launch_mode<kGiven>(a, (per_chunk + 127) / 128, stream);
 }
 
 int attention_grid_chunks(int max_seq_len) { return attention_most_chunks(max_seq_len); }
@@ -548,18 +581,7 @@ hipError_t launch_decode_attention_at(const void* qkv, int n_q, int n_kv, const 
   // Chunks never exceed the size max_seq_len rows need (the rule grows with
   // the rows attended), so that size fixes the kernel's groups per wave.
   const int nu = (attention_chunk_rows(s_max) + 127) / 128;
-  switch (n_q / n_kv) {
-    case 1:
-      return launch_dyn<1>(a, nu, stream);
-    case 2:
-      return launch_dyn<2>(a, nu, stream);
-    case 4:
-      return launch_dyn<4>(a, nu, stream);
-    case 8:
-      return launch_dyn<8>(a, nu, stream);
-    default:
-      return hipErrorInvalidValue;
-  }
+  return launch_mode<kDevicePos>(a, nu, stream);
 }
 
 }  // namespace lsk

@@ -212,6 +212,13 @@ hipError_t launch_decode_attention_at(const void* qkv, int n_q, int n_kv, const 
                                       void* v_cache, int s_max, const int* pos_device, float scale, void* out,
                                       void* workspace, size_t ws_bytes, hipStream_t stream);
 
+// softmax(q K^T scale) V of one query row per head over `rows` cached rows
+// (contiguous [rows][d] per kv head, kv_stride elements apart): the same
+// kernel without its norms, RoPE and append.
+hipError_t launch_gqa_attention(const void* q, int n_q, int n_kv, const void* k, const void* v, size_t kv_stride,
+                                int rows, float scale, void* out, void* workspace, size_t ws_bytes,
+                                hipStream_t stream);
+
 // RMSNorm of M rows of K values (row stride ldx, K = 512..4096 in steps of
 // 512) into contiguous rows of y (rows.hip).
 hipError_t launch_rms_rows(const void* x, int M, int K, size_t ldx, const void* w, float eps, void* y,

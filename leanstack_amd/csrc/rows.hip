@@ -44,7 +44,9 @@ __device__ __forceinline__ bf16x8_t norm_chunk(bf16x8_t x, bf16x8_t w, float r) 
 // One wave per row, the row in registers (NC chunks of 8 values per lane,
 // K = 512 NC), so x is read once and y written once: the bytes are the bound.
 // Four rows per workgroup keep enough waves in flight at any M; a row per
-// wave needs no LDS and no barrier.
+// wave needs no LDS and no barrier.  K = 2560: 16.2 us at 8192 rows (84 MB,
+// 5.2 TB/s, a large copy's rate; F.rms_norm 25.5 us), 3.2 us at 64 rows, where
+// the launch is what is left.
 template <int NC>
 __global__ __launch_bounds__(kRowsThreads) void rms_rows_kernel(const __bf16* __restrict__ x, size_t ldx,
                                                                 const __bf16* __restrict__ w,
@@ -73,7 +75,10 @@ __global__ __launch_bounds__(kRowsThreads) void rms_rows_kernel(const __bf16* __
 // halves of a rotation pair are in one lane and the head's sum of squares is
 // three DPP steps over the 8 lanes.  A wave takes 8 heads of one token (2 KB
 // of the QKV row); the 4 waves of a workgroup take 4 consecutive tokens of
-// the same heads, so a head's 4 output rows are 1 KB contiguous.
+// the same heads, so a head's 4 output rows are 1 KB contiguous.  Bound by
+// its bytes: 32 + 8 heads at 8192 rows (168 MB) 36 us, 4.7 TB/s, against
+// 580 us of torch's norms, products, sums and concatenations; 3-5 us at
+// 1..64 rows, against 60-80 us.
 // Grid: (ceil(M / 4), ceil((n_q + n_kv) / 8)).
 __global__ __launch_bounds__(kRowsThreads) void qk_rope_kernel(QkRopeArgs a) {
   const int lane = threadIdx.x & 63;

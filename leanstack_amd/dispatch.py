@@ -100,6 +100,25 @@ def _sdpa(query_states, key_states, value_states, attention_scale, num_key_value
     return torch.matmul(probs, v.contiguous()).to(query_states.dtype)
 
 
+def _attend_row(query_states, key_states, value_states, attention_scale, num_key_value_groups):
+    """_sdpa of one query row of one sequence in the attention kernel, as
+    [n_q * d]; None for any call it does not serve."""
+    if query_states.dim() != 4 or key_states.dim() != 4 or key_states.shape != value_states.shape:
+        return None
+    b, n_q, t, d = query_states.shape
+    n_kv, rows = key_states.shape[1], key_states.shape[2]
+    if (b == 1 and t == 1 and d == 128 and key_states.shape[0] == 1 and key_states.shape[3] == d
+            and 0 < n_kv <= 64 and num_key_value_groups in (1, 2, 4, 8) and n_q == n_kv * num_key_value_groups
+            and 0 < rows <= kernels.ATTENTION_MAX_ROWS
+            and key_states.stride()[1:] == value_states.stride()[1:] and key_states.stride(3) == 1
+            and key_states.stride(2) == d and key_states.stride(1) % 8 == 0
+            and (n_kv == 1 or key_states.stride(1) >= rows * d)
+            and isinstance(attention_scale, float) and math.isfinite(attention_scale)
+            and query_states.is_contiguous() and _plain_eager(query_states, key_states, value_states)):
+        return kernels.gqa_attention(query_states[0, :, 0], key_states[0], value_states[0], attention_scale)
+    return None
+
+
 def _require_packed(weight, what: str, layout: int = _lib.LAYOUT_MFMA16X32) -> PackedWeight:
     if not isinstance(weight, PackedWeight):
         raise ValueError(f"{what} must be a PackedWeight from the resident arena, got {type(weight).__name__}")
@@ -252,6 +271,9 @@ def _semantic_decode_attention_output(query_states, key_states, value_states, o_
                                       num_key_value_groups):
     """SDPA then o_proj over [B,T,nq*d] (qwen_explicit.py:855-883)."""
     o_w = _require_packed(o_proj_weight, "o_proj_weight")
+    attn = _attend_row(query_states, key_states, value_states, attention_scale, num_key_value_groups)
+    if attn is not None:
+        return kernels.linear(attn.view(1, 1, -1), o_w)
     attn = _sdpa(query_states, key_states, value_states, attention_scale, num_key_value_groups)
     attn = attn.transpose(1, 2).reshape(query_states.shape[0], query_states.shape[2], -1)
     return kernels.linear(attn, o_w)
@@ -261,7 +283,9 @@ def _semantic_decode_attention_output_vector(query_states, key_states, value_sta
                                              num_key_value_groups):
     """SDPA then the M=1 o_proj GEMV (qwen_explicit.py:886-913) -> [H]."""
     o_w = _require_packed(o_proj_weight, "o_proj_weight")
-    attn = _sdpa(query_states, key_states, value_states, attention_scale, num_key_value_groups)
+    attn = _attend_row(query_states, key_states, value_states, attention_scale, num_key_value_groups)
+    if attn is None:
+        attn = _sdpa(query_states, key_states, value_states, attention_scale, num_key_value_groups)
     return kernels.linear(attn.reshape(1, -1), o_w).view(-1)
 
 

@@ -388,6 +388,57 @@ def decode_attention(qkv: torch.Tensor, q_norm_weight: torch.Tensor, k_norm_weig
     return out
 
 
+ATTENTION_MAX_ROWS = 16384
+ATTENTION_COUNTER_BYTES = 256  # the part of an attention workspace that must start zeroed
+
+# Workspaces of gqa_attention by (device, stream, bytes): one size per head
+# geometry, so none is ever replaced under a call that is still running.
+_gqa_workspaces: dict[tuple[int, int, int], torch.Tensor] = {}
+
+
+def _gqa_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
+    if torch.cuda.is_current_stream_capturing():
+        # the graph's own: replays never share one with eager calls
+        workspace = torch.empty(nbytes, device=device, dtype=torch.uint8)
+        workspace[:ATTENTION_COUNTER_BYTES].zero_()
+        return workspace
+    key = (_device_index(device), stream_handle(), nbytes)
+    workspace = _gqa_workspaces.get(key)
+    if workspace is None:
+        workspace = _gqa_workspaces[key] = torch.zeros(nbytes, device=device, dtype=torch.uint8)
+    return workspace
+
+
+def gqa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float) -> torch.Tensor:
+    """softmax(q k^T * scale) v of one query row per head over rows already
+    cached: q [n_q, d] contiguous, k / v [n_kv, rows, d] with equal strides and
+    contiguous rows (a cache's written part), bfloat16, d = 128.  Returns
+    [n_q * d] bf16."""
+    n_q, d = q.shape
+    n_kv, rows, _ = k.shape
+    for t, what in ((q, "q"), (k, "k"), (v, "v")):
+        _require_device(t, what)
+        if t.dtype != torch.bfloat16:
+            raise ValueError(f"{what} must be bfloat16, got {t.dtype}")
+    if k.shape != v.shape or k.stride() != v.stride() or k.shape[2] != d or k.stride(2) != 1 or k.stride(1) != d \
+            or not q.is_contiguous():
+        raise ValueError(f"q must be contiguous [n_q, {d}] and k / v [n_kv, rows, {d}] with equal strides and "
+                         f"contiguous rows, got {tuple(q.shape)}, {tuple(k.shape)} / {tuple(v.shape)}")
+    dev = _one_device(q, (k, "k"), (v, "v"))
+    lib = _lib.load()
+    out = torch.empty((n_q * d,), device=q.device, dtype=torch.bfloat16)
+    with torch.cuda.device(dev):
+        workspace = None
+        if rows > 128:  # sized for the longest cache: one workspace as a sequence grows
+            workspace = _gqa_workspace(dev, lib.lsk_attention_workspace_bytes(n_q, n_kv, d, ATTENTION_MAX_ROWS))
+        status = lib.lsk_gqa_attention_bf16(
+            q.data_ptr(), n_q, n_kv, d, k.data_ptr(), v.data_ptr(), max(k.stride(0), rows * d), rows, float(scale),
+            out.data_ptr(), None if workspace is None else workspace.data_ptr(),
+            0 if workspace is None else workspace.numel(), stream_handle())
+    _lib.check(status, "lsk_gqa_attention_bf16")
+    return out
+
+
 class LmHeadWorkspace:
     """Device workspace of the greedy head, sized once per (M, V, K): a status
     word and the per-workgroup argmax partials.  Zero-filled here; every call

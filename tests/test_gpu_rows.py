@@ -99,3 +99,60 @@ def test_rows_keep_the_general_path(gpu):
     assert dispatch.qwen_rmsnorm(x[:0], w, EPS).shape == (0, 2560)
     dual = torch.func.jvp(lambda v: dispatch.qwen_rmsnorm(v, w, EPS), (x,), (torch.ones_like(x),))[1]
     assert dual.shape == x.shape and bool(dual.isfinite().all())
+
+
+@pytest.mark.parametrize("rows", [1, 16, 127, 128, 129, 512, 513, 700, 4096, 4097, 16384])
+@pytest.mark.parametrize("n_q,n_kv", [(32, 8), (4, 4), (8, 1), (4, 2)])
+def test_gqa_attention(gpu, rows, n_q, n_kv):
+    """Every chunk-rule regime on the written part of a longer cache (rows past
+    it hold NaN).  fp32 softmax weights sum to 1 and the output is rounded
+    once: within one bf16 step of the oracle plus 2^-14 of the largest |v|
+    (expf and the fp32 sums of up to 16384 weights)."""
+    if rows > 4097 and n_q != 32:
+        pytest.skip("one geometry at the longest cache")
+    q = activations(n_q, 128, seed=rows).view(1, n_q, 1, 128)
+    k = torch.full((1, n_kv, rows + 16, 128), float("nan"), dtype=torch.bfloat16)
+    v = k.clone()
+    k[:, :, :rows] = activations(n_kv * rows, 128, seed=2).view(1, n_kv, rows, 128)
+    v[:, :, :rows] = activations(n_kv * rows, 128, seed=3).view(1, n_kv, rows, 128)
+    dk, dv = k.to(DEV)[:, :, :rows], v.to(DEV)[:, :, :rows]
+    scale = 128 ** -0.5
+    got = dispatch._attend_row(q.to(DEV), dk, dv, scale, n_q // n_kv)
+    assert got is not None and torch.equal(got, dispatch._attend_row(q.to(DEV), dk, dv, scale, n_q // n_kv))
+    expect = ref_attention.sdpa_gqa(q, k[:, :, :rows], v[:, :, :rows], scale, n_q // n_kv).float().view(-1)
+    diff = (got.cpu().float() - expect).abs()
+    assert bool((diff <= expect.abs() * 2.0 ** -7 + 2.0 ** -14 * float(v[:, :, :rows].abs().max())).all())
+
+
+def test_gqa_attention_extremes_and_routes(gpu):
+    """Scores of -inf in a whole chunk and NaN rows behave as the torch ops;
+    shapes the kernel does not serve take them; a captured call replays."""
+    scale, rows = 128 ** -0.5, 700
+    q = activations(32, 128, seed=1).abs().view(1, 32, 1, 128).to(DEV)
+    k = activations(8 * rows, 128, seed=2).view(1, 8, rows, 128).to(DEV)
+    v = activations(8 * rows, 128, seed=3).view(1, 8, rows, 128).to(DEV)
+    k[:, 1, 128:256] = float("-inf")  # q > 0: the whole second chunk scores -inf
+    k[:, 2, 300, 5] = float("nan")
+    k[:, 3, 17] = float("inf")
+    got = dispatch._attend_row(q, k, v, scale, 4).float()
+    expect = dispatch._sdpa(q, k, v, scale, 4).view(-1).float()
+    assert torch.equal(got.isnan(), expect.isnan()) and bool(got.isnan().any()) and not bool(got.isnan().all())
+    assert float((got - expect).nan_to_num().abs().max()) <= 2.0 ** -6
+    for bad in ((q.expand(2, -1, -1, -1), k.expand(2, -1, -1, -1), v.expand(2, -1, -1, -1), scale, 4),
+                (q.expand(-1, -1, 3, -1), k, v, scale, 4), (q, k, v.clone()[..., ::2].repeat(1, 1, 1, 2)[:, :, ::1, :], scale, 2),
+                (q, k.transpose(1, 2).contiguous().transpose(1, 2), v, scale, 4), (q.float(), k, v, scale, 4),
+                (q.clone().requires_grad_(), k, v, scale, 4), (q, k[:, :, :0], v[:, :, :0], scale, 4)):
+        assert dispatch._attend_row(*bad) is None
+    k[:, 1:4] = 0.5
+    expect = dispatch._attend_row(q, k, v, scale, 4)
+    side = torch.cuda.Stream()  # no warm-up on it: the graph brings its own workspace
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = dispatch._attend_row(q, k, v, scale, 4)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        eager = dispatch._attend_row(q, k, v, scale, 4)
+        torch.cuda.synchronize()
+        assert torch.equal(out, expect) and torch.equal(eager, expect)
