@@ -109,8 +109,9 @@ int lsk_unpack_bf16(const void* packed_host, int N, int K, int layout_id, void* 
  *   weight rows per workgroup (16, 32 or 64), plan[1] = N / plan[0] row
  *   groups, plan[2] = the groups whose K range is split (all or none),
  *   plan[3] = workgroups per group (1: no split).  This is the plan of the
- *   plain and residual epilogues; a SiLU*up call takes whole gate/up pairs
- *   (32 or 64 rows) and may split differently.
+ *   plain and residual epilogues; a SiLU*up call takes units of 8 gate and 8
+ *   up rows, runs this kernel up to 128 rows at any N, and may split
+ *   differently.
  *   M > 128: plan[0] = weight rows per output block of the prefill block GEMM
  *   (256, 192 or 128), plan[1] = output blocks, plan[2] = blocks whose K
  *   range is split over several workgroups, plan[3] = workgroups (K chunks)
@@ -137,7 +138,8 @@ int lsk_linear_plan(int M, int N, int K, size_t ws_bytes, int plan[4]);
  *   M          >= 1.  M <= 16 runs the decode/verify kernel (weights streamed
  *              once, activations padded to the 16 MFMA columns); 17..128 the
  *              skinny kernel (weights streamed once, activations in groups
- *              of 16 tokens; 65..128 rows of N >= 8192 the 128x128 GEMM);
+ *              of 16 tokens; 65..128 rows of N >= 8192 without SiLU*up the
+ *              128x128 GEMM);
  *              larger M the prefill MFMA GEMM.
  *   workspace  NULL, or lsk_workspace_bytes(LSK_OP_LINEAR, M, N, K) bytes
  *              (0 bytes: no workspace is used), 256-byte aligned, zero-filled

@@ -95,7 +95,7 @@ size_t lsk_workspace_bytes(int op, int M, int N, int K) {
     if (M <= lsk::kSkinnyMaxM) {
       // the larger of the plain and the SiLU*up split (lsk_workspace_bytes
       // does not know the epilogue)
-      if (!lsk::skinny_route(M, N, K)) return 0;
+      if (!lsk::skinny_route(M, N, K, false)) return 0;
       int cus = 0;
       if (lsk::current_device_cus(&cus) != hipSuccess) return 0;
       const size_t plain = lsk::skinny_plan(M, N, K, false, cus, true).bytes;
@@ -130,7 +130,7 @@ int lsk_linear_plan(int M, int N, int K, size_t ws_bytes, int* plan) {
   // tile grid; decode slices off it ({0, 0, 0, 1}).
   if (M <= lsk::kDecodeMaxM) return LSK_OK;
   hipError_t err;
-  if (lsk::skinny_route(M, N, K)) {
+  if (lsk::skinny_route(M, N, K, false)) {
     int cus = 0;
     err = lsk::current_device_cus(&cus);
     if (err != hipSuccess) return hip_fail(err, "device CU count");
@@ -170,7 +170,7 @@ int lsk_linear_bf16(const void* w_packed, int layout_id, int N, int K, const voi
   const bool gemm_shape = N % lsk::kGemmBN == 0 && K % lsk::kGemmBK == 0;
   if (M <= lsk::kDecodeMaxM) {
     err = lsk::launch_decode_linear(w_packed, N, K, x, M, ldx, y, ldy, epi, residual, ldr, stream);
-  } else if (lsk::skinny_route(M, N, K)) {
+  } else if (lsk::skinny_route(M, N, K, epi == lsk::Epilogue::kSiluMul)) {
     int cus = 0;
     err = lsk::current_device_cus(&cus);
     if (err != hipSuccess) return hip_fail(err, "device CU count");

@@ -15,7 +15,7 @@
 //    for the M > 128 shapes with N a multiple of 256 that the wdx kernel does
 //    not take (K an odd multiple of 64).
 //  * gemm_linear_kernel, 128 x 128 blocks for the rest of the 128-row grid
-//    (65..128 rows of N >= 8192, or N a multiple of 128 with K an odd
+//    (65..128 rows of N >= 8192 without SiLU*up, or N a multiple of 128 with K an odd
 //    multiple of 64 that the 256 x 256 kernel cannot take).  Each packed 1 KB weight
 //    tile already is a v_mfma_f32_16x16x32_bf16 operand in lane order, so the
 //    weight half of every LDS stage is a straight linear copy; the activation

@@ -30,7 +30,7 @@ constexpr unsigned kSkSpinLimit = 1u << 22;
 
 // Projections of kDecodeMaxM < M <= kSkinnyMaxM rows (skinny.hip).
 constexpr int kSkinnyMaxM = 128;
-constexpr int kSkinnyWaves = 8;
+constexpr int kSkinnyWaves = 4;
 // Split-K arrival counters live in the prefill workspace's flag words (each
 // call leaves them zero), partial slots from kSkPartialsOffset.
 constexpr int kSkinnyMaxGroups = (int)((kSkPartialsOffset - kSkFlagsOffset) / 4);
@@ -264,7 +264,7 @@ struct SkinnyPlan {
 };
 int skinny_groups(int M);
 hipError_t current_device_cus(int* cus_out);
-bool skinny_route(int M, int N, int K);
+bool skinny_route(int M, int N, int K, bool silu);
 SkinnyPlan skinny_plan(int M, int N, int K, bool silu, int cus, bool has_workspace);
 // y = epilogue(x . W^T) for kDecodeMaxM < M <= kSkinnyMaxM (N % 16 == 0, or
 // N % 32 == 0 for SiLU*up; K % 32 == 0).  `workspace` (NULL: no split) must

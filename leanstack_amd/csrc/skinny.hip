@@ -1,17 +1,25 @@
-// Projections of 17..128 rows on gfx950: y[M][N] = epilogue(x[M][K] . W^T).
+// Projections of 17..128 rows on gfx950: y[M][N] = epilogue(x[M][K] . W[N][K]^T).
 //
-// At these row counts a projection is still bound by its weight bytes (the
-// arithmetic intensity is M FLOP per weight byte, under 128), so the kernel
-// keeps the decode kernels' streaming form and widens its B operand instead
-// of tiling like the prefill GEMM: every packed 1 KB weight tile is loaded
-// once, straight into registers as the A operand of
-// v_mfma_f32_16x16x32_bf16, and multiplied with ceil(M / 16) activation
-// fragments of 16 tokens each (MG groups), read from L2 next to it.
+// At these row counts a projection is still bound by the bytes that each CU
+// pulls: the weights from HBM once (the arithmetic intensity is M FLOP per
+// weight byte, under 128) and, per workgroup, the activations from L2.  A
+// workgroup owns RBW row-blocks (16 output rows each) and all tokens over one
+// K range, which its 4 wavefronts take in 64-K steps in turn.  Each wave DMAs
+// the weight tiles and activation rows of its steps into a ring of its own in
+// LDS, 2-4 steps deep (up to 160 KB in flight per CU, no registers), and
+// multiplies a step on v_mfma_f32_16x16x32_bf16 as it lands: no barrier and no
+// shared stage until the waves' partial tiles are summed through LDS, in wave
+// order.
 //
-// Work split.  A workgroup owns RBW row-blocks (16 output rows each; a
-// gate/up pair for SiLU*up) over one K range; its 8 wavefronts split that
-// range and their partial tiles are summed through LDS in wave order.  When
-// the row-blocks alone would leave CUs idle (kv/o/down-sized N), the call's
+// Activations are read 8 lanes per row, whole 128-byte lines: read as B
+// fragments straight from global memory (16 rows of 64 bytes per load, each
+// 16 bytes of it another cache access), they cost four times the accesses and
+// the weights waited behind them.  17.5 / 14.0 / 45.0 / 24.5 -> 12.9 / 10.8 /
+// 24.8 / 17.6 us for QKV / o / gate_up + SiLU*up / down at 64 rows, 32 / 24 /
+// 56 / 42 -> 18.5 / 15.4 / 37 / 25 at 128; per CU about 33 bytes/ns of weights
+// and activations together, against 27 of weights alone in the decode kernels.
+//
+// When the row-blocks alone would leave CUs idle (kv/o/down-sized N), the call's
 // workspace lets the K range of every row-block be split over S workgroups:
 // each publishes its fp32 partial with device-coherent stores and counts its
 // arrival, and the workgroup that arrives last adds the S partials in split
@@ -42,43 +50,144 @@ typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kNW = kSkinnyWaves;  // wavefronts per workgroup
 constexpr int kCoherent = 16;      // buffer cache policy: device-coherent (sc1)
+constexpr unsigned kRawBufferDword3 = 0x00020000u;
+constexpr int kLdsBytes = 160 * 1024;  // of one CU
 
 __device__ __forceinline__ f32x4_t mfma16(bf16x8_t a, bf16x8_t b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// k-tiles loaded per round: about 16 loads per wave in flight.
-template <int RBW, int MG>
-constexpr int round_tiles() {
-  return 16 / (RBW + MG) > 0 ? 16 / (RBW + MG) : 1;
+__device__ __forceinline__ u32x4_t buffer_words(const void* base, size_t bytes) {
+  const unsigned long long p = reinterpret_cast<unsigned long long>(base);
+  return u32x4_t{(unsigned)p, (unsigned)(p >> 32) & 0xffffu, (unsigned)(bytes < 0x7fffffffu ? bytes : 0x7fffffffu),
+                 kRawBufferDword3};
 }
 
-// Token groups summed per LDS round: the largest divisor of MG with
-// RBW * CG <= 8 (7 waves x 8 KB of partial tiles).
-template <int RBW, int MG>
-constexpr int sum_chunk() {
-  int c = 8 / RBW < MG ? 8 / RBW : MG;
-  while (MG % c != 0) --c;
-  return c;
+// 1 KB of global memory straight into LDS: lane l's 16 bytes at voff + soff
+// land at lds + 16 l.  In assembly, with no result register, so that the
+// compiler neither counts it nor waits for it before unrelated LDS reads (one
+// ring in one LDS array would otherwise be drained before every read); each
+// use waits for its own data (wait_steps).
+template <bool STREAM>
+__device__ __forceinline__ void dma_1k(u32x4_t rsrc, unsigned voff, unsigned soff, unsigned lds) {
+  soff = __builtin_amdgcn_readfirstlane(soff);  // wave-uniform; says so to the compiler
+  lds = __builtin_amdgcn_readfirstlane(lds);
+  if constexpr (STREAM)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds), "v"(voff),
+                 "s"(rsrc), "s"(soff)
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
+                 "s"(rsrc), "s"(soff)
+                 : "memory");
 }
 
+// Wait until at most `steps` (0..D-1, wave-uniform) steps of NL loads are in
+// flight.
+template <int NL, int D>
+__device__ __forceinline__ void wait_steps(int steps) {
+  if constexpr (D >= 4) {
+    if (steps >= 3) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * NL < 63 ? 3 * NL : 63) : "memory");
+      return;
+    }
+  }
+  if constexpr (D >= 3) {
+    if (steps == 2) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NL < 63 ? 2 * NL : 63) : "memory");
+      return;
+    }
+  }
+  if constexpr (D >= 2) {
+    if (steps == 1) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL < 63 ? NL : 63) : "memory");
+      return;
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// RBW row-blocks x MG token groups per workgroup; 64-K steps of (2 RBW + 2 MG)
+// KB, each loaded and multiplied by one wave.
+template <int RBW, int MG>
+struct Shape {
+  static constexpr int kLoads = 2 * RBW + 2 * MG;  // 1 KB loads per step
+  static constexpr int kSlot = kLoads * 1024;
+  static constexpr int kFit = kLdsBytes / (kNW * kSlot);
+  static constexpr int kDepth = kFit < 1 ? 1 : kFit > 4 ? 4 : kFit;  // steps in flight per wave
+  static constexpr int kRing = kNW * kDepth * kSlot;
+  // Row-blocks whose partial tiles of all waves fit the ring at once.
+  static constexpr int kSumRows = kRing / (kNW * MG * 1024) < RBW ? kRing / (kNW * MG * 1024) : RBW;
+  static_assert(kFit >= 1 && kSumRows >= 1, "one step per wave fits the LDS");
+};
+
+// EPI SiLU*up: a "row-block" is a unit of 8 gate rows and the 8 up rows of the
+// same outputs (half a gate/up pair of the packed layout), so units, not
+// pairs, are what the workgroups share out.
 template <int RBW, int MG, int EPI>
 __global__ __launch_bounds__(kNW * 64) void skinny_kernel(
     const bf16x8_t* __restrict__ w, const __bf16* __restrict__ x, int ldx, __bf16* __restrict__ y, int ldy,
-    const __bf16* __restrict__ residual, int ldr, int M, int KT, int S, unsigned* __restrict__ counters,
+    const __bf16* __restrict__ residual, int ldr, int M, int NB, int KT, int S, unsigned* __restrict__ counters,
     unsigned char* __restrict__ partials, unsigned partial_bytes) {
-  static_assert(EPI != static_cast<int>(Epilogue::kSiluMul) || RBW % 2 == 0,
-                "SiLU*up takes whole gate/up pairs of row-blocks");
+  using Sh = Shape<RBW, MG>;
+  constexpr bool kSilu = EPI == static_cast<int>(Epilogue::kSiluMul);
+  constexpr int D = Sh::kDepth;
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[Sh::kRing];
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int m = lane & 15;  // B-operand column = token within its group
   const int g = lane >> 4;  // K group inside a tile / output row quad
   const int grp = blockIdx.x / S;
   const int split = blockIdx.x - grp * S;
   const int rb0 = grp * RBW;
-  const int sb = (KT * split) / S, se = (KT * (split + 1)) / S;
-  const int kb = sb + ((se - sb) * wave) / kNW;
-  const int ke = sb + ((se - sb) * (wave + 1)) / kNW;
+
+  // Steps of 64 K: this split's are [ub, ue), dealt to the waves in turn, so
+  // that the four waves read neighbouring 128-byte pieces of the same rows.
+  const int units = (KT + 1) / 2;
+  const int ub = (int)((long long)units * split / S), ue = (int)((long long)units * (split + 1) / S);
+  const int n = ue - ub > wave ? (ue - ub - wave + kNW - 1) / kNW : 0;
+
+  // Weight loads: one packed tile (or the 8 + 8 rows of a unit) in A-operand
+  // order per KB.  Blocks past the last repeat it; they are never stored.
+  const int first = kSilu ? (rb0 >> 1) * 2 : rb0;  // packed row-block the buffer starts at
+  const u32x4_t wrsrc = buffer_words(w + (size_t)first * KT * 64, (size_t)(NB - first) * KT * 1024);
+  unsigned wvoff[RBW];
+#pragma unroll
+  for (int r = 0; r < RBW; ++r) {
+    const int rb = min(rb0 + r, NB - 1);
+    if constexpr (kSilu)
+      wvoff[r] = (unsigned)((rb & ~1) - first + (m >> 3)) * KT * 1024u + (g * 16 + 8 * (rb & 1) + (m & 7)) * 16u;
+    else
+      wvoff[r] = (unsigned)(rb - first) * KT * 1024u + lane * 16u;
+  }
+  // Activation loads: 8 token rows x 128 bytes (whole lines) per KB.  Row t's
+  // 16-byte chunk c is stored at position c ^ ((t >> 1) & 7) of its 128
+  // bytes, which puts the 16 lanes of a fragment read on distinct banks.
+  // Rows past M repeat row M - 1; their columns are never stored.
+  const u32x4_t xrsrc = buffer_words(x, ((size_t)(M - 1) * ldx + (size_t)KT * kTileK) * 2);
+  unsigned xrow[2 * MG];
+  const int xr = lane >> 3;
+#pragma unroll
+  for (int i = 0; i < 2 * MG; ++i) xrow[i] = (unsigned)min(8 * i + xr, M - 1) * ldx * 2u;
+  const unsigned ring0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)ring +
+                         wave * D * Sh::kSlot;
+
+  auto issue = [&](int step, int slot) {
+    const int u = ub + wave + kNW * step;
+    const bool half = 2 * u + 1 >= KT;  // odd KT: the last step has one k-tile
+    const unsigned lds = ring0 + slot * Sh::kSlot;
+#pragma unroll
+    for (int r = 0; r < RBW; ++r)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        dma_1k<true>(wrsrc, wvoff[r], (unsigned)(2 * u + (half ? 0 : h)) * 1024u, lds + (2 * r + h) * 1024);
+#pragma unroll
+    for (int i = 0; i < 2 * MG; ++i) {
+      int c = (lane & 7) ^ (((i & 1) << 2) | (xr >> 1));
+      if (half) c &= 3;
+      dma_1k<false>(xrsrc, xrow[i] + c * 16u, (unsigned)u * 128u, lds + (2 * RBW + i) * 1024);
+    }
+  };
 
   f32x4_t acc[RBW][MG];
 #pragma unroll
@@ -86,215 +195,188 @@ __global__ __launch_bounds__(kNW * 64) void skinny_kernel(
 #pragma unroll
     for (int q = 0; q < MG; ++q) acc[r][q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  // Token rows 16q + m; rows past M read row 0 (in bounds) and are masked.
-  const bf16x8_t* xr[MG];
-  unsigned keep[MG];
 #pragma unroll
-  for (int q = 0; q < MG; ++q) {
-    const int row = 16 * q + m;
-    keep[q] = row < M ? 0xffffffffu : 0u;
-    xr[q] = reinterpret_cast<const bf16x8_t*>(x + (size_t)(row < M ? row : 0) * ldx) + g;
-  }
-  const bf16x8_t* wt = w + (size_t)rb0 * KT * 64 + lane;
-
-  // Rounds of R k-tiles: every load of a round goes out before its first
-  // multiply, so each wave keeps about 16 loads in flight.
-  constexpr int R = round_tiles<RBW, MG>();
-  auto round = [&](int kt, auto n_tag) {
-    constexpr int N = decltype(n_tag)::value;
-    bf16x8_t wv[N][RBW];
-    bf16x8_t xv[N][MG];
+  for (int d = 0; d < D; ++d)
+    if (d < n) issue(d, d);
+  int slot = 0;
+  for (int i = 0; i < n; ++i) {
+    wait_steps<Sh::kLoads, D>(min(D - 1, n - 1 - i));
+    const unsigned char* buf = ring + (wave * D + slot) * Sh::kSlot;
+    bf16x8_t wv[2][RBW], xv[2][MG];
 #pragma unroll
-    for (int u = 0; u < N; ++u)
+    for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int r = 0; r < RBW; ++r) wv[u][r] = __builtin_nontemporal_load(wt + ((size_t)r * KT + kt + u) * 64);
-#pragma unroll
-    for (int u = 0; u < N; ++u)
-#pragma unroll
-      for (int q = 0; q < MG; ++q) {
-        u32x4_t v = __builtin_bit_cast(u32x4_t, xr[q][(kt + u) * 4]);
-        v &= keep[q];
-        xv[u][q] = __builtin_bit_cast(bf16x8_t, v);
-      }
-#pragma unroll
-    for (int u = 0; u < N; ++u)
-#pragma unroll
-      for (int r = 0; r < RBW; ++r)
-#pragma unroll
-        for (int q = 0; q < MG; ++q) acc[r][q] = mfma16(wv[u][r], xv[u][q], acc[r][q]);
-  };
-  int kt = kb;
-  for (; kt + R <= ke; kt += R) round(kt, std::integral_constant<int, R>{});
-  for (; kt < ke; ++kt) round(kt, std::integral_constant<int, 1>{});
-
-  // Cross-wave sum in wave order, CG token groups at a time (56 KB of LDS).
-  constexpr int CG = sum_chunk<RBW, MG>();
-  static_assert(MG % CG == 0, "token groups are summed in whole chunks");
-  __shared__ f32x4_t red[kNW - 1][RBW * CG][64];
-#pragma unroll
-  for (int c0 = 0; c0 < MG; c0 += CG) {
-    if (wave > 0) {
-#pragma unroll
-      for (int r = 0; r < RBW; ++r)
-#pragma unroll
-        for (int j = 0; j < CG; ++j) red[wave - 1][r * CG + j][lane] = acc[r][c0 + j];
-    }
-    __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-      for (int v = 0; v < kNW - 1; ++v)
-#pragma unroll
-        for (int r = 0; r < RBW; ++r)
-#pragma unroll
-          for (int j = 0; j < CG; ++j) acc[r][c0 + j] += red[v][r * CG + j][lane];
-    }
-    if (c0 + CG < MG) __syncthreads();
-  }
-  if (wave != 0) return;
-
-  if (S > 1) {
-    // Publish this split's partial, count the arrival; the last of the S
-    // splits of the row-blocks sums them in split order.  Partials cross
-    // XCDs, whose L2s are not coherent with each other: device-coherent
-    // buffer stores and loads, and the arrival only after the stores are
-    // acknowledged.
-    const __amdgpu_buffer_rsrc_t parts =
-        __builtin_amdgcn_make_buffer_rsrc(partials, (short)0, (int)partial_bytes, (int)0x00020000u);
-    constexpr unsigned kSlot = RBW * MG * 64 * 16;
-#pragma unroll
-    for (int r = 0; r < RBW; ++r)
+      for (int r = 0; r < RBW; ++r) wv[h][r] = *reinterpret_cast<const bf16x8_t*>(buf + (2 * r + h) * 1024 + lane * 16);
 #pragma unroll
       for (int q = 0; q < MG; ++q)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[r][q]), parts, lane * 16,
-                                               (unsigned)blockIdx.x * kSlot + (r * MG + q) * 1024u, kCoherent);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    unsigned old = 0;
-    if (lane == 0) old = __hip_atomic_fetch_add(counters + grp, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    old = (unsigned)__builtin_amdgcn_readfirstlane((int)old);
-    if (old != (unsigned)S - 1) return;
-    // Last arrival: every other split's partial is acknowledged.  Re-arm the
-    // counter for the next call, then add the S partials in split order, this
-    // split's own from its registers.  The others are loaded PB partials at a
-    // time (16 fragments in flight); slots past the last split are read at an
-    // offset beyond the buffer's range, which returns zeros without a memory
-    // access, and are never added.
-    if (lane == 0) __hip_atomic_store(counters + grp, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    constexpr int PB = RBW * MG >= 16 ? 1 : 16 / (RBW * MG);
-    f32x4_t mine[RBW][MG];
-#pragma unroll
-    for (int r = 0; r < RBW; ++r)
-#pragma unroll
-      for (int q = 0; q < MG; ++q) {
-        mine[r][q] = acc[r][q];
-        acc[r][q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      }
-    bool own_added = false;
-    for (int o0 = 0; o0 < S - 1; o0 += PB) {
-      f32x4_t v[PB][RBW][MG];
-#pragma unroll
-      for (int b = 0; b < PB; ++b) {
-        const int o = o0 + b;  // o-th other split in split order
-        const int sp = o < split ? o : o + 1;
-        // Out of range goes in the vector offset: the range check covers the
-        // vector and instruction offsets, not the scalar one.
-        const bool real = o < S - 1;
-        const unsigned voff = (real ? 0u : 0x80000000u) + (unsigned)lane * 16u;
-        const unsigned base = real ? (unsigned)(grp * S + sp) * kSlot : 0u;
-#pragma unroll
-        for (int r = 0; r < RBW; ++r)
-#pragma unroll
-          for (int q = 0; q < MG; ++q)
-            v[b][r][q] = __builtin_bit_cast(
-                f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(parts, voff, base + (r * MG + q) * 1024u, kCoherent));
-      }
-#pragma unroll
-      for (int b = 0; b < PB; ++b) {
-        const int o = o0 + b;
-        if (o >= S - 1) break;
-        if (!own_added && (o < split ? o : o + 1) > split) {
-#pragma unroll
-          for (int r = 0; r < RBW; ++r)
-#pragma unroll
-            for (int q = 0; q < MG; ++q) acc[r][q] += mine[r][q];
-          own_added = true;
-        }
-#pragma unroll
-        for (int r = 0; r < RBW; ++r)
-#pragma unroll
-          for (int q = 0; q < MG; ++q) acc[r][q] += v[b][r][q];
-      }
+        xv[h][q] = *reinterpret_cast<const bf16x8_t*>(buf + 2 * RBW * 1024 + (16 * q + m) * 128 +
+                                                      (((4 * h + g) ^ (m >> 1)) << 4));
     }
-    if (!own_added) {
+    // The slot's values are in registers before its next loads may land.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (i + D < n) issue(i + D, slot);
+    const bool half = 2 * (ub + wave + kNW * i) + 1 >= KT;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (h == 1 && half) break;
 #pragma unroll
       for (int r = 0; r < RBW; ++r)
 #pragma unroll
-        for (int q = 0; q < MG; ++q) acc[r][q] += mine[r][q];
+        for (int q = 0; q < MG; ++q) acc[r][q] = mfma16(wv[h][r], xv[h][q], acc[r][q]);
+    }
+    slot = slot + 1 == D ? 0 : slot + 1;
+  }
+
+  // Cross-wave sum in wave order through the drained ring, kSumRows row-blocks
+  // at a time: tile t = r MG + q is summed (and stored) by wave t % 4.
+  constexpr int kTiles = RBW * MG;
+  constexpr int kMine = (kTiles + kNW - 1) / kNW;
+  f32x4_t sum[kMine];
+#pragma unroll
+  for (int r0 = 0; r0 < RBW; r0 += Sh::kSumRows) {
+    __syncthreads();
+#pragma unroll
+    for (int r = r0; r < RBW && r < r0 + Sh::kSumRows; ++r)
+#pragma unroll
+      for (int q = 0; q < MG; ++q)
+        *reinterpret_cast<f32x4_t*>(ring + ((wave * Sh::kSumRows + r - r0) * MG + q) * 1024 + lane * 16) = acc[r][q];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) {
+      const int t = j * kNW + wave;
+      if (t < r0 * MG || t >= (r0 + Sh::kSumRows) * MG || t >= kTiles) continue;
+      const unsigned char* src = ring + (t - r0 * MG) * 1024 + lane * 16;
+      f32x4_t v = *reinterpret_cast<const f32x4_t*>(src);
+#pragma unroll
+      for (int o = 1; o < kNW; ++o) v += *reinterpret_cast<const f32x4_t*>(src + o * Sh::kSumRows * MG * 1024);
+      sum[j] = v;
     }
   }
 
-  // Lane (g, m) holds output rows 4g..4g+3 of each row-block for token
-  // 16q + m of each group q.
+  if (S > 1) {
+    // Publish this split's sums, count the arrival; the last of the S splits
+    // of the row-blocks adds them in split order.  Partials cross XCDs, whose
+    // L2s are not coherent with each other: device-coherent buffer stores and
+    // loads, and the arrival only after every wave's stores are acknowledged.
+    const __amdgpu_buffer_rsrc_t parts =
+        __builtin_amdgcn_make_buffer_rsrc(partials, (short)0, (int)partial_bytes, (int)kRawBufferDword3);
+    constexpr unsigned kPart = kTiles * 1024;
 #pragma unroll
-  for (int q = 0; q < MG; ++q) {
-    const int tok = 16 * q + m;
-    if (tok >= M) continue;
-    if constexpr (EPI == static_cast<int>(Epilogue::kSiluMul)) {
+    for (int j = 0; j < kMine; ++j) {
+      const int t = j * kNW + wave;
+      if (t < kTiles)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, sum[j]), parts, lane * 16,
+                                               (unsigned)blockIdx.x * kPart + t * 1024u, kCoherent);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* last = reinterpret_cast<int*>(ring);
+    if (threadIdx.x == 0)
+      *last = __hip_atomic_fetch_add(counters + grp, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+              (unsigned)S - 1;
+    __syncthreads();
+    if (!*last) return;
+    // Re-arm the counter for the next call, then add the S partials, this
+    // split's own from its registers, the others PB splits at a time (every load
+    // of a round goes out before the first add: a branch around an add would
+    // let the compiler sink the load into it); slots past the last split are
+    // read at an offset beyond the buffer's range, which returns zeros without
+    // a memory access.
+    if (threadIdx.x == 0) __hip_atomic_store(counters + grp, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    constexpr int PB = kMine >= 8 ? 2 : 4;
+    f32x4_t total[kMine];
 #pragma unroll
-      for (int p = 0; p < RBW / 2; ++p) {
-        const int j = (rb0 / 2 + p) * 16 + 4 * g;  // intermediate index
-        unsigned short o[4];
+    for (int j = 0; j < kMine; ++j) total[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < S; s0 += PB) {
+      f32x4_t v[PB][kMine];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = bf16_bits(silu_mul_bf16(acc[2 * p][q][i], acc[2 * p + 1][q][i]));
-        *reinterpret_cast<u32x2_t*>(y + (size_t)tok * ldy + j) =
-            u32x2_t{o[0] | ((unsigned)o[1] << 16), o[2] | ((unsigned)o[3] << 16)};
-      }
-    } else {
+      for (int b = 0; b < PB; ++b) {
+        // Out of range goes in the vector offset: the range check covers the
+        // vector and instruction offsets, not the scalar one.
+        const bool real = s0 + b < S && s0 + b != split;
+        const unsigned voff = (real ? 0u : 0x80000000u) + (unsigned)lane * 16u;
+        const unsigned base = real ? (unsigned)(grp * S + s0 + b) * kPart : 0u;
 #pragma unroll
-      for (int r = 0; r < RBW; ++r) {
-        const int n = (rb0 + r) * 16 + 4 * g;
-        unsigned short o[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float v = bf16_round(acc[r][q][i]);
-          if constexpr (EPI == static_cast<int>(Epilogue::kResidualAdd))
-            v = static_cast<float>(residual[(size_t)tok * ldr + n + i]) + v;
-          o[i] = bf16_bits(v);
+        for (int j = 0; j < kMine; ++j) {
+          const int t = min(j * kNW + wave, kTiles - 1);
+          v[b][j] = __builtin_bit_cast(
+              f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(parts, voff, base + t * 1024u, kCoherent));
         }
-        *reinterpret_cast<u32x2_t*>(y + (size_t)tok * ldy + n) =
-            u32x2_t{o[0] | ((unsigned)o[1] << 16), o[2] | ((unsigned)o[3] << 16)};
       }
+#pragma unroll
+      for (int b = 0; b < PB; ++b) {
+#pragma unroll
+        for (int j = 0; j < kMine; ++j) total[j] += s0 + b == split ? sum[j] : v[b][j];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) sum[j] = total[j];
+  }
+
+  // Lane (g, m) holds output rows 4g..4g+3 of a tile's row-block for token
+  // 16q + m; of a SiLU*up unit, g = 0, 1 gate rows and g = 2, 3 the up rows of
+  // lanes 32 below.
+#pragma unroll
+  for (int j = 0; j < kMine; ++j) {
+    const int t = j * kNW + wave;
+    if (t >= kTiles) break;
+    const int rb = rb0 + t / MG;
+    const int tok = 16 * (t % MG) + m;
+    if constexpr (kSilu) {
+      float up[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) up[i] = __shfl_xor(sum[j][i], 32);
+      if (rb >= NB || tok >= M || g >= 2) continue;
+      unsigned short o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = bf16_bits(silu_mul_bf16(sum[j][i], up[i]));
+      *reinterpret_cast<u32x2_t*>(y + (size_t)tok * ldy + rb * 8 + 4 * g) =
+          u32x2_t{o[0] | ((unsigned)o[1] << 16), o[2] | ((unsigned)o[3] << 16)};
+    } else {
+      if (rb >= NB || tok >= M) continue;
+      const int col = rb * 16 + 4 * g;
+      unsigned short o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float v = bf16_round(sum[j][i]);
+        if constexpr (EPI == static_cast<int>(Epilogue::kResidualAdd))
+          v = static_cast<float>(residual[(size_t)tok * ldr + col + i]) + v;
+        o[i] = bf16_bits(v);
+      }
+      *reinterpret_cast<u32x2_t*>(y + (size_t)tok * ldy + col) =
+          u32x2_t{o[0] | ((unsigned)o[1] << 16), o[2] | ((unsigned)o[3] << 16)};
     }
   }
 }
 
 template <int RBW, int MG, int EPI>
 hipError_t launch_cfg(const SkinnyPlan& p, const void* w, const void* x, int ldx, void* y, int ldy,
-                      const void* residual, int ldr, int M, int KT, void* workspace, hipStream_t stream) {
+                      const void* residual, int ldr, int M, int NB, int KT, void* workspace, hipStream_t stream) {
   auto* ws = static_cast<unsigned char*>(workspace);
   unsigned* counters = p.S > 1 ? reinterpret_cast<unsigned*>(ws + kSkFlagsOffset) : nullptr;
   unsigned char* partials = p.S > 1 ? ws + kSkPartialsOffset : nullptr;
   const unsigned partial_bytes = p.S > 1 ? (unsigned)(p.groups * p.S * RBW * MG * 1024) : 0u;
   launch_kernel(skinny_kernel<RBW, MG, EPI>, dim3(p.groups * p.S), dim3(kNW * 64), 0, stream,
                 static_cast<const bf16x8_t*>(w), static_cast<const __bf16*>(x), ldx, static_cast<__bf16*>(y), ldy,
-                static_cast<const __bf16*>(residual), ldr, M, KT, p.S, counters, partials, partial_bytes);
+                static_cast<const __bf16*>(residual), ldr, M, NB, KT, p.S, counters, partials, partial_bytes);
   return hipGetLastError();
 }
 
 template <int RBW, int EPI>
 hipError_t launch_rbw(const SkinnyPlan& p, const void* w, const void* x, int ldx, void* y, int ldy,
-                      const void* residual, int ldr, int M, int KT, void* workspace, hipStream_t stream) {
+                      const void* residual, int ldr, int M, int NB, int KT, void* workspace, hipStream_t stream) {
   switch (skinny_groups(M)) {
     case 2:
-      return launch_cfg<RBW, 2, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, KT, workspace, stream);
+      return launch_cfg<RBW, 2, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
     case 3:
-      return launch_cfg<RBW, 3, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, KT, workspace, stream);
+      return launch_cfg<RBW, 3, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
     case 4:
-      return launch_cfg<RBW, 4, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, KT, workspace, stream);
+      return launch_cfg<RBW, 4, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
     case 6:
-      if constexpr (RBW <= 2) return launch_cfg<RBW, 6, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, KT, workspace, stream);
+      if constexpr (RBW != 4) return launch_cfg<RBW, 6, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
       break;
     case 8:
-      if constexpr (RBW <= 2) return launch_cfg<RBW, 8, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, KT, workspace, stream);
+      if constexpr (RBW != 4) return launch_cfg<RBW, 8, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
       break;
     default:
       break;
@@ -304,12 +386,21 @@ hipError_t launch_rbw(const SkinnyPlan& p, const void* w, const void* x, int ldx
 
 template <int EPI>
 hipError_t launch_epi(const SkinnyPlan& p, const void* w, const void* x, int ldx, void* y, int ldy,
-                      const void* residual, int ldr, int M, int KT, void* workspace, hipStream_t stream) {
-  const int rbw = p.rows / kTileRows;
-  if (rbw == 4) return launch_rbw<4, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, KT, workspace, stream);
-  if (rbw == 2) return launch_rbw<2, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, KT, workspace, stream);
-  if constexpr (EPI != static_cast<int>(Epilogue::kSiluMul))
-    return launch_rbw<1, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, KT, workspace, stream);
+                      const void* residual, int ldr, int M, int NB, int KT, void* workspace, hipStream_t stream) {
+  switch (p.rows / kTileRows) {
+    case 1:
+      return launch_rbw<1, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
+    case 2:
+      return launch_rbw<2, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
+    case 4:
+      return launch_rbw<4, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
+    case 5:
+      if constexpr (EPI == static_cast<int>(Epilogue::kSiluMul))
+        return launch_rbw<5, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
+      break;
+    default:
+      break;
+  }
   return hipErrorInvalidValue;
 }
 
@@ -342,48 +433,56 @@ int skinny_groups(int M) {
 }
 
 // Whether lsk_linear_bf16 runs M rows of an [N, K] projection on the skinny
-// kernel: 17..64 rows always, 65..128 rows unless N is wide enough (>= 8192,
-// the gate_up shapes) for the 128 x 128 GEMM's blocks to fill the chip, which
-// then reads each activation fragment once per 128 weight rows instead of
-// once per 32 (measured at 128 rows: gate_up 9728 x 2560 38 against 58 us,
-// the fused 19456 x 2560 with SiLU*up 40 against 92 us).
-bool skinny_route(int M, int N, int K) {
+// kernel: 17..64 rows always; 65..128 rows unless N is wide (>= 8192) and on
+// the 128 x 128 GEMM's grid, whose blocks then fill the chip and read each
+// activation fragment once per 128 weight rows instead of once per 32 --
+// except with SiLU*up, where units of 8 outputs give every CU 80 weight rows
+// in one round (19456 x 2560 at 128 rows: 37 us, the GEMM 56 us).
+bool skinny_route(int M, int N, int K, bool silu) {
   if (M <= kDecodeMaxM || M > kSkinnyMaxM || N % kTileRows != 0 || K % kTileK != 0) return false;
   const bool gemm_grid = N % kGemmBN == 0 && K % kGemmBK == 0;
-  return M <= 64 || !gemm_grid || N < 8192;
+  return M <= 64 || !gemm_grid || N < 8192 || silu;
 }
 
-// Row-blocks per workgroup and the K split, from a sweep of every (rows, S)
-// over the Qwen3-4B projections at 17, 32, 64 and 128 rows on 256 CUs: two
-// row-blocks (one gate/up pair) per workgroup by default, since each
-// activation fragment is read once for all of them; one for narrow N (fewer
-// than 64 pairs of row-blocks) and for up to 32 rows when the row-blocks
-// alone cover every CU; four (up to 64 rows, for the registers) when two
-// would take more than one round of the CUs and four still cover half of
-// them.  With a workspace the K range is split so that the grid comes to
-// about one workgroup per CU, each split keeping at least two k-tiles per
-// wave.
+// Row-blocks per workgroup and the K split, from sweeps of (rows, S) over the
+// Qwen3-4B projections at 17, 32, 64 and 128 rows on 256 CUs.  Two row-blocks
+// per workgroup by default, since the activations are read once for all of
+// them (QKV at 32 rows: 10.0 us with two, 13.2 with one, 10.9 with four in two
+// splits; o_proj at 64 rows 10.8 with two in three splits, 17.9 with one in
+// two, 13.4 with four in six); one for narrow N (fewer than 64 pairs of
+// row-blocks) and for up to 32 rows when the row-blocks are one round of the
+// CUs by themselves; four (up to 64 rows) when two would take more than one
+// round of the CUs and four still cover half of them.  SiLU*up takes as many
+// units per workgroup as bring them to one round: five for the 1216 units of
+// 19456 rows (21.3 us at 32 rows; four, in two rounds, 28.6).  With a
+// workspace the K range is split so that the grid comes to about one
+// workgroup per CU, each split keeping at least 16 k-tiles; a second split
+// that leaves the CUs two rounds costs more than it balances (QKV at 64 rows
+// 12.8 -> 17.9 us).
 SkinnyPlan skinny_plan(int M, int N, int K, bool silu, int cus, bool has_workspace) {
   const int NB = N / kTileRows;
   const int KT = K / kTileK;
   const int mg = skinny_groups(M);
   int rbw = 2;
-  if (!silu && ((mg <= 2 && NB >= cus) || NB / 2 < 64 || NB % 2 != 0)) {
+  if (silu) {
+    // units of 8 outputs: as many per workgroup as bring them to one round
+    if (NB > 2 * cus) rbw = mg <= 4 && NB <= 4 * cus ? 4 : 5;
+  } else if ((mg <= 2 && NB >= cus && NB <= cus + cus / 8) || NB / 2 < 64 || NB % 2 != 0) {
     rbw = 1;
   } else if (mg <= 4 && NB % 4 == 0 && NB / 2 > cus && NB / 4 <= cus && 2 * (NB / 4) >= cus) {
     rbw = 4;
   }
-  const int groups = NB / rbw;
+  const int groups = (NB + rbw - 1) / rbw;
   int S = 1;
-  const int max_s = KT / (2 * kNW);
-  if (has_workspace && groups <= kSkinnyMaxGroups && max_s >= 2) {
+  const int max_s = KT / 16;
+  if (has_workspace && skinny_route(M, N, K, false) && groups <= kSkinnyMaxGroups && max_s >= 2) {
     S = (4 * cus + groups) / (4 * groups);  // floor(cus / groups + 1/4)
     if (S > max_s) S = max_s;
     if (S < 1) S = 1;
   }
   SkinnyPlan p;
   p.rows = kTileRows * rbw;
-  p.groups = NB / rbw;
+  p.groups = groups;
   p.S = S;
   p.bytes = p.S > 1 ? kSkPartialsOffset + (size_t)p.groups * p.S * rbw * mg * 1024 : 0;
   return p;
@@ -395,15 +494,16 @@ hipError_t launch_skinny_linear(const void* w, int N, int K, const void* x, int 
   const bool silu = epi == Epilogue::kSiluMul;
   SkinnyPlan p = skinny_plan(M, N, K, silu, cus, workspace != nullptr);
   if (p.S > 1 && ws_bytes < p.bytes) return hipErrorInvalidValue;  // checked by the caller
+  const int NB = N / kTileRows;
   const int KT = K / kTileK;
   switch (epi) {
     case Epilogue::kSiluMul:
-      return launch_epi<1>(p, w, x, ldx, y, ldy, residual, ldr, M, KT, workspace, stream);
+      return launch_epi<1>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
     case Epilogue::kResidualAdd:
-      return launch_epi<2>(p, w, x, ldx, y, ldy, residual, ldr, M, KT, workspace, stream);
+      return launch_epi<2>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
     case Epilogue::kNone:
     default:
-      return launch_epi<0>(p, w, x, ldx, y, ldy, residual, ldr, M, KT, workspace, stream);
+      return launch_epi<0>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
   }
 }
 
