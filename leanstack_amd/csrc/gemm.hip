@@ -4,11 +4,11 @@
 // kernels; launch_gemm_linear at the end of this file picks one:
 //
 //  * wdx::gemm_wdx_kernel, the prefill GEMM proper (M > 128, N a multiple of
-//    128 or 192, K of 128: every Qwen3-4B projection).  256 tokens x 256, 192
-//    or 128 weight rows x 64 K per stage and workgroup on
+//    128 or 192, K of 128: every Qwen3-4B projection).  Up to 256 tokens x 256,
+//    192 or 128 weight rows x 64 K per stage and workgroup on
 //    v_mfma_f32_32x32x16_bf16: weight fragments from HBM/L2 straight into
-//    registers one stage ahead, activations DMA'd into a three-buffer LDS ring
-//    two stages ahead, a counted stage barrier, the epilogue through LDS in
+//    registers one to four stages ahead, activations DMA'd into an LDS ring two
+//    to four stages ahead, a counted stage barrier, the epilogue through LDS in
 //    row order, and, with a workspace, the last partial round split along K
 //    over the idle CUs ("Split-K of the last round" below).
 //  * big::gemm256_kernel, 256 x 256 blocks with both operands staged in LDS,
@@ -483,26 +483,48 @@ hipError_t launch(const void* w, int N, int K, const void* x, int M, int ldx, vo
 // rows the same way; the 192-row blocks keep two waves across N and two across tokens, and
 // there the two waves that share a weight-row half fetch the same lines, the
 // second mostly from L1.
-// Weight fragments are prefetched one stage ahead into the idle one of two
-// register sets, activations two stages ahead into the free one of three
-// LDS buffers; the stage loop is unrolled by six so both rotations run
-// without copies, which requires an even number of stages.
+// Weight fragments and activations are loaded kWAhead and kXAhead stages
+// ahead, into a rotation of register sets and one of LDS buffers; the stage
+// loop is unrolled by whole turns of both, so neither needs copies.
 namespace wdx {
 
-constexpr int BN = 256, BM = 256, BK = 64;
+constexpr int BM = 256, BK = 64;  // most tokens of a block, K of a stage
 // Wave tile: A 32-row weight tiles x TB 32-token tiles.  The 4 waves of a
-// workgroup are TB/2 across N and 8/TB across the 256 tokens, so a block
-// has 16*A*TB weight rows.  Built: (A, TB) = (2, 8) -> 256 rows, every wave
-// over all tokens; (3, 4) -> 192 rows (QKV at 2048 tokens: 256 blocks in
-// one round instead of 192 blocks of 256 rows); (1, 8) -> 128 rows, every
-// wave over all tokens (small token counts, see choose_tiles).
-template <int A, int TB>
-constexpr int kBN = 16 * A * TB;
-constexpr int kRowsWide = kBN<2, 8>;  // 256
-constexpr int kRows192 = kBN<3, 4>;
-constexpr int kRows128 = kBN<1, 8>;   // every wave 32 rows over all 256 tokens
+// workgroup are WN across N and 4/WN across the tokens, so a block has
+// 32*A*WN weight rows and 32*TB*4/WN tokens.  Built: (A, TB, WN) = (2, TB, 4)
+// -> 256 rows and (1, TB, 4) -> 128 rows (small token counts, see
+// choose_tiles), every wave over all 32 TB tokens, TB = 5..8 by the tokens a
+// block really has (see launch_gemm_linear); (3, 4, 2) -> 192 rows x 256
+// tokens (QKV at 2048 tokens: 256 blocks in one round instead of 192 blocks
+// of 256 rows).
+constexpr int kRowsWide = 256, kRows192 = 192, kRows128 = 128;
 constexpr int kThreads = 256;
-constexpr int kXStageBytes = BM * BK * 2;  // 32 KB of activation fragments per stage
+template <int A, int WN>
+constexpr int kBN = 32 * A * WN;
+template <int TB, int WN>
+constexpr int kBM = 32 * TB * (4 / WN);
+template <int TB, int WN>
+constexpr int kXStageBytes = kBM<TB, WN> * BK * 2;  // activation fragments of a stage
+
+// Stages loaded ahead: weights into registers kWAhead stages ahead, activations
+// into LDS kXAhead.  Loads retire in order, so a stage's wait for its
+// activations is also a wait for every weight load issued before them; both
+// run equally far ahead where the weights come from HBM, i.e. where few token
+// blocks share a weight block: 128-row blocks, and 256-row blocks of up to 192
+// tokens.  Against one stage ahead: QKV / o / gate_up + SiLU*up / down at 129
+// tokens 19.8 / 19.4 / 37.6 / 32.9 -> 18.6 / 18.4 / 35.9 / 32.3 us, at 301
+// 23.4 / 21.2 / 47.0 / 36.5 -> 22.5 / 20.5 / 47.0 / 35.7; what is left is the
+// bytes each CU pulls through L2 (55-75 bytes/ns) and the split's exchange.
+// At more tokens the weights are L2 hits and the registers of (2, 8) allow
+// one.
+template <int A, int TB>
+constexpr int kWAhead = A > 2 ? 1 : TB <= 6 ? 4 : A == 1 ? 3 : 1;
+template <int A, int TB>
+constexpr int kXAhead = kWAhead<A, TB> > 2 ? kWAhead<A, TB> : 2;
+constexpr int kMaxBuffers = 5;
+struct XBuffers {
+  unsigned char* p[kMaxBuffers];
+};
 
 using big::f32x16_t;
 using big::mfma32;
@@ -517,12 +539,17 @@ struct WFrags {
 
 // A fragment (32 rows x 16 K) of tile a, step q: lane (li, kg) takes row li of
 // the two 16-row packed tiles 2a, 2a+1 and K chunk 2(q&1)+kg of k-tile q/2.
+// voff: the lane's byte offset in the block's first tiles (an offset beyond
+// the buffer's range moves no data).
 template <int A>
-__device__ __forceinline__ void load_w(WFrags<A>& f, const bf16x8_t* __restrict__ wl, int KT, int s) {
+__device__ __forceinline__ void load_w(WFrags<A>& f, __amdgpu_buffer_rsrc_t wbuf, unsigned voff, int KT, int s) {
 #pragma unroll
   for (int q = 0; q < 4; ++q)
 #pragma unroll
-    for (int a = 0; a < A; ++a) f.v[q][a] = wl[((size_t)(2 * a) * KT + 2 * s + (q >> 1)) * 64 + (q & 1) * 32];
+    for (int a = 0; a < A; ++a)
+      f.v[q][a] = __builtin_bit_cast(
+          bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(wbuf, voff + (q >> 1) * 1024 + (q & 1) * 512,
+                                                          (unsigned)(2 * a * KT + 2 * s) * 1024u, 0));
 }
 
 struct Args {
@@ -548,30 +575,30 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 // buffer covers exactly the block's rows.
 // MUBUF, not FLAT: a FLAT load that writes LDS makes the compiler drain
 // every counter before the next dependent use.
+template <int ND>
 __device__ __forceinline__ void dma_x(unsigned char* buf, __amdgpu_buffer_rsrc_t rsrc, int ldx, int rmax, int s,
-                                      int wave, int lane) {
+                                      int wave, int lane, unsigned out) {
   const int r = lane >> 3;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int j = wave * 8 + i;  // 1 KB block: tokens 8j .. 8j+7 (j & 7 == i)
-    const int c = (lane & 7) ^ r ^ i;
+  for (int i = 0; i < ND; ++i) {
+    const int j = wave * ND + i;  // 1 KB block: tokens 8j .. 8j+7
+    const int c = (lane & 7) ^ r ^ (j & 7);
     const int row = min(8 * j + r, rmax);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t*)(buf + j * 1024), 16, (row * ldx + c * 8) * 2,
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t*)(buf + j * 1024), 16, ((unsigned)(row * ldx + c * 8) * 2u) | out,
                                              s * BK * 2, 0, 0);
   }
 }
 
-// The stage barrier: s_waitcnt vmcnt(4A + 8) lgkmcnt(0), then s_barrier.
-// Only the current stage's 4A weight loads and 8 activation DMAs may still
-// be in flight after it, so the previous stage's DMA has landed in every
-// wave.  Not __syncthreads: its release fence waits for vmcnt(0), i.e. for
-// the loads just issued too.  The builtins (not inline asm) let the
-// compiler's wait-counter model see these waits; the empty asm statements
-// keep memory accesses from moving across them.
-template <int A>
+// The stage barrier: s_waitcnt vmcnt(VM) lgkmcnt(0), then s_barrier.  VM: the
+// loads issued after the next stage's activation DMA, which has therefore
+// landed in every wave after it.  Not __syncthreads: its release fence waits
+// for vmcnt(0), i.e. for the loads just issued too.  The builtins (not inline
+// asm) let the compiler's wait-counter model see these waits; the empty asm
+// statements keep memory accesses from moving across them.
+template <int VM>
 __device__ __forceinline__ void stage_sync() {
-  constexpr int vm = 4 * A + 8;
-  constexpr int imm = (vm & 15) | ((vm >> 4) << 14) | (7 << 4);
+  static_assert(VM < 64, "the load counter has 6 bits");
+  constexpr int imm = (VM & 15) | ((VM >> 4) << 14) | (7 << 4);
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(imm);
   __builtin_amdgcn_s_barrier();
@@ -579,17 +606,17 @@ __device__ __forceinline__ void stage_sync() {
 }
 
 // acc[a][b] += W rows of 32-row tiles (wn*A + a) x tokens of 32-token tiles
-// (wm*TB + b) over stages [s0, s1) (s1 - s0 even) of block (nb, mb).
+// (wm*TB + b) over stages [s0, s1) of block (nb, mb).
 //
-// Software pipeline over 64-K stages with three LDS activation buffers.
-// While the MFMAs of stage s run on buffer cur with weight fragments wc, the
-// same instruction stream reads the activation fragments of the next 16-K
-// step, loads stage s+1's weight fragments into the idle register set and
-// DMAs stage s+2's activations into the buffer stage s-1 read.  The barrier
-// before the last 16-K step publishes stage s+1's buffer (its DMA was issued
-// one stage earlier) and retires every read of this stage's.  Stage indices
-// past s1 are clamped: those loads stay in bounds and the data they stage is
-// never multiplied.
+// Software pipeline over 64-K stages with X + 1 LDS activation buffers and
+// P + 1 weight register sets (X = kXAhead, P = kWAhead).  While the MFMAs of
+// stage s run on its buffer and weight set, the same instruction stream reads
+// the activation fragments of the next 16-K step, loads stage s + P's weight
+// fragments into the set stage s - 1 used and DMAs stage s + X's activations
+// into the buffer stage s - 1 read.  The barrier before the last 16-K step
+// publishes stage s + 1's buffer and retires every read of this stage's.
+// Loads of stages past s1 go beyond the buffers' range: they move no data and
+// keep the count of loads in flight the same for every stage's wait.
 template <int kM, int ND, int VO, int NV>
 __device__ __forceinline__ void sched_step() {
   // kM MFMAs of one 16-K step, each followed by one of the step's ND LDS
@@ -602,10 +629,14 @@ __device__ __forceinline__ void sched_step() {
   }
 }
 
-template <int A, int TB>
-__device__ __forceinline__ void mainloop(f32x16_t (&acc)[A][TB], const Args& g, unsigned char* xa, unsigned char* xb,
-                                         unsigned char* xc, int nb, int mb, int s0, int s1) {
-  constexpr int WN = TB / 2;  // waves across N
+template <int A, int TB, int WN>
+__device__ __forceinline__ void mainloop(f32x16_t (&acc)[A][TB], const Args& g, const XBuffers& xs, int nb, int mb,
+                                         int s0, int s1) {
+  constexpr int P = kWAhead<A, TB>, X = kXAhead<A, TB>;
+  static_assert(X + 1 <= kMaxBuffers && (P == 1 || P == X), "stage order of the loads");
+  constexpr int kTokens = kBM<TB, WN>;
+  constexpr int ND = kTokens / 32;  // activation DMAs of a stage per wave
+  constexpr int kInFlight = (X - 1) * (4 * A + ND);  // loads issued after the next stage's DMA
   // Opaque per call: keeps the per-lane offsets below from being hoisted out
   // of a caller's loop over blocks, where they would stay live (and spill)
   // across the epilogues.
@@ -615,17 +646,19 @@ __device__ __forceinline__ void mainloop(f32x16_t (&acc)[A][TB], const Args& g, 
   const int wave = tid >> 6;
   const int wn = wave % WN;
   const int wm = wave / WN;
-  const int m0 = mb * BM;
+  const int m0 = mb * kTokens;
   const int li = lane & 31;
   const int kg = lane >> 5;
   const int KT = g.KT;
-  const int rmax = min(g.M - m0, BM) - 1;
+  const int rmax = min(g.M - m0, kTokens) - 1;
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(g.x + (size_t)m0 * g.ldx), (short)0, (int)((unsigned)(rmax + 1) * (unsigned)g.ldx * 2u), 0x00020000);
-
-  // This lane's element of weight fragment (a=0, q=0) at stage 0.
-  const bf16x8_t* wl =
-      g.w + ((size_t)(nb * (kBN<A, TB> / kTileRows) + wn * 2 * A + (li >> 4)) * KT) * 64 + (li & 15) + kg * 16;
+  // The block's weight rows, and this lane's element of weight fragment
+  // (a=0, q=0) at stage 0 in them.
+  constexpr int kRb = kBN<A, WN> / kTileRows;
+  const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(g.w + (size_t)nb * kRb * KT * 64), (short)0, (int)((unsigned)(kRb * KT) * 1024u), 0x00020000);
+  const unsigned wl = (unsigned)((wn * 2 * A + (li >> 4)) * KT) * 1024u + ((li & 15) + kg * 16) * 16u;
   // Chunk 2q + kg of token t = wm*TB*32 + b*32 + li sits at position
   // (2q + kg) ^ (li & 7) ^ (li >> 3) ^ 4(b & 1): x_lane[q] holds it for
   // even b, odd b flip bit 6 of the byte offset.
@@ -645,91 +678,94 @@ __device__ __forceinline__ void mainloop(f32x16_t (&acc)[A][TB], const Args& g, 
 #pragma unroll
       for (int b = 0; b < TB; ++b) acc[a][b] = mfma32(fa[a], fb[b], acc[a][b]);
   };
+  auto past = [&](int s) { return s < s1 ? 0u : 0x80000000u; };
+  auto at = [&](int s) { return s < s1 ? s : 0; };
 
-  WFrags<A> wf0, wf1;
+  WFrags<A> wf[P + 1];
   bf16x8_t fb0[TB], fb1[TB];
 
   // Interleave groups per 16-K step: A*TB MFMAs with the step's TB LDS
-  // reads and its global traffic (4A weight loads in step 0, 8 DMA in
+  // reads and its global traffic (4A weight loads in step 0, ND DMA in
   // step 1).
   constexpr int kM = A * TB;
-  // Step 1's 8 DMAs go after the MFMAs that follow its TB LDS reads, as far
-  // as the step has MFMAs there: for A = 1 (kM = TB = 8) from the first one.
-  constexpr int kDmaSlot = kM - 8 >= TB ? TB : (kM > 8 ? kM - 8 : 0);
-  // Stage s multiplies buffer cur, DMAs the activations of stage s + 2 into
-  // dst (the buffer stage s - 1 read) and, before its barrier, waits for the
-  // DMA of stage s + 1 (issued one stage earlier; only the 4A weight loads
-  // and 8 DMA of this stage may still be in flight).
-  auto stage = [&](int s, const WFrags<A>& wc, WFrags<A>& wn_, const unsigned char* cur, unsigned char* dst,
-                   const unsigned char* nxt) {
-    const int sw = min(s + 1, s1 - 1);
-    const int sx = min(s + 2, s1 - 1);
+  // Step 1's DMAs go after the MFMAs that follow its TB LDS reads, as far as
+  // the step has MFMAs there: for A = 1 (kM = TB = ND) from the first one.
+  constexpr int kDmaSlot = kM - ND >= TB ? TB : (kM > ND ? kM - ND : 0);
+  // Stage s, the i-th of a round of the rotation.
+  auto stage = [&](int s, auto i_tag) {
+    constexpr int i = decltype(i_tag)::value;
+    const WFrags<A>& wc = wf[i % (P + 1)];
+    const unsigned char* cur = xs.p[i % (X + 1)];
 
     __builtin_amdgcn_sched_barrier(0);
     read_b(fb1, cur, 1);
-    load_w(wn_, wl, KT, sw);
+    load_w(wf[(i + P) % (P + 1)], wbuf, wl | past(s + P), KT, at(s + P));
     mfma_step(wc.v[0], fb0);
     sched_step<kM, TB, 0, 4 * A>();
 
     __builtin_amdgcn_sched_barrier(0);
     read_b(fb0, cur, 2);
-    dma_x(dst, xr, g.ldx, rmax, sx, wave, lane);
+    dma_x<ND>(xs.p[(i + X) % (X + 1)], xr, g.ldx, rmax, at(s + X), wave, lane, past(s + X));
     mfma_step(wc.v[1], fb1);
-    sched_step<kM, TB, kDmaSlot, 8>();
+    sched_step<kM, TB, kDmaSlot, ND>();
 
     __builtin_amdgcn_sched_barrier(0);
     read_b(fb1, cur, 3);
     mfma_step(wc.v[2], fb0);
     sched_step<kM, TB, 0, 0>();
 
-    // Publishes nxt (stage s + 1's DMA) and retires every read of cur.
-    stage_sync<A>();
-    read_b(fb0, nxt, 0);
+    // Publishes stage s + 1's buffer and retires every read of cur.
+    stage_sync<kInFlight>();
+    read_b(fb0, xs.p[(i + 1) % (X + 1)], 0);
     mfma_step(wc.v[3], fb1);
     sched_step<kM, TB, 0, 0>();
     __builtin_amdgcn_sched_barrier(0);
   };
 
   // Every wave is past its last read of the buffers (a previous call's
-  // stages) before the prologue overwrites xa and xb.
+  // stages) before the prologue overwrites them.
   __syncthreads();
-  dma_x(xa, xr, g.ldx, rmax, s0, wave, lane);
-  dma_x(xb, xr, g.ldx, rmax, min(s0 + 1, s1 - 1), wave, lane);
-  load_w(wf0, wl, KT, s0);
-  stage_sync<A>();
-  read_b(fb0, xa, 0);
+#pragma unroll
+  for (int i = 0; i < X; ++i) {
+    dma_x<ND>(xs.p[i], xr, g.ldx, rmax, at(s0 + i), wave, lane, past(s0 + i));
+    if (i < P) load_w(wf[i], wbuf, wl | past(s0 + i), KT, at(s0 + i));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // Stage 0's DMA is the first of the loads above.
+  stage_sync<kInFlight>();
+  read_b(fb0, xs.p[0], 0);
+  constexpr int U = P == X ? P + 1 : 6;  // stages until both rotations repeat
+  static_assert(U % (P + 1) == 0 && U % (X + 1) == 0, "whole rotations");
+  auto run = [&](int s, int count) {
+    if (count > 0) stage(s, std::integral_constant<int, 0>{});
+    if (count > 1) stage(s + 1, std::integral_constant<int, 1>{});
+    if constexpr (U > 2)
+      if (count > 2) stage(s + 2, std::integral_constant<int, 2>{});
+    if constexpr (U > 3)
+      if (count > 3) stage(s + 3, std::integral_constant<int, 3>{});
+    if constexpr (U > 4)
+      if (count > 4) stage(s + 4, std::integral_constant<int, 4>{});
+    if constexpr (U > 5)
+      if (count > 5) stage(s + 5, std::integral_constant<int, 5>{});
+  };
   int s = s0;
-  for (; s + 6 <= s1; s += 6) {
-    stage(s, wf0, wf1, xa, xc, xb);
-    stage(s + 1, wf1, wf0, xb, xa, xc);
-    stage(s + 2, wf0, wf1, xc, xb, xa);
-    stage(s + 3, wf1, wf0, xa, xc, xb);
-    stage(s + 4, wf0, wf1, xb, xa, xc);
-    stage(s + 5, wf1, wf0, xc, xb, xa);
-  }
-  if (s + 2 <= s1) {
-    stage(s, wf0, wf1, xa, xc, xb);
-    stage(s + 1, wf1, wf0, xb, xa, xc);
-    if (s + 4 <= s1) {
-      stage(s + 2, wf0, wf1, xc, xb, xa);
-      stage(s + 3, wf1, wf0, xa, xc, xb);
-    }
-  }
+  for (; s + U <= s1; s += U) run(s, U);
+  run(s, s1 - s);
 }
 
 // Epilogue of this lane's 32x32 tile (a, b) of block (nb, mb).  src(p)
 // returns elements 2p, 2p+1 of the lane's 16 fp32 results of the tile.
 // Lane l of tile (a, b) holds D[8*(j/4) + 4*(l/32) + j%4][l%32], j = 0..15.
-template <int EPI, int A, int TB, typename Src>
+template <int EPI, int A, int TB, int WN, typename Src>
 __device__ __forceinline__ void store_one_tile(Src src, const Args& g, int nb, int mb, int a, int b) {
-  constexpr int WN = TB / 2;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wn = wave % WN;
   const int wm = wave / WN;
   const int li = lane & 31;
   const int kg = lane >> 5;
-  const int m = mb * BM + (wm * TB + b) * 32 + li;
+  const int m = mb * kBM<TB, WN> + (wm * TB + b) * 32 + li;
   if (m >= g.M) return;
   const int an = (nb * WN + wn) * A + a;  // global 32-row tile index
   if constexpr (EPI == static_cast<int>(Epilogue::kSiluMul)) {
@@ -762,26 +798,14 @@ __device__ __forceinline__ void store_one_tile(Src src, const Args& g, int nb, i
   }
 }
 
-// Epilogue of the whole block straight from the accumulators.
-template <int EPI, int A, int TB>
-__device__ __forceinline__ void store_tile(const f32x16_t (&acc)[A][TB], const Args& g, int nb, int mb) {
-#pragma unroll
-  for (int b = 0; b < TB; ++b)
-#pragma unroll
-    for (int a = 0; a < A; ++a)
-      store_one_tile<EPI, A, TB>([&](int p) { return make_float2(acc[a][b][2 * p], acc[a][b][2 * p + 1]); }, g, nb,
-                                 mb, a, b);
-}
-
 // Epilogue of a whole block through LDS.  Stored straight from the
-// accumulators (store_tile), each store instruction writes 8 bytes per lane
+// accumulators, each store instruction writes 8 bytes per lane
 // into 32 different token rows; every CU does that at the same moment at
 // the end of a round, and it cost 14-19 us of a 2048 x 8192 output.  Here
-// each wave rounds its results to bf16 into its own 16 KB of the (free)
-// activation buffers, token-major, then reads them back 16 bytes per lane
+// each wave rounds its results to bf16 into its own half of a (free)
+// activation buffer, token-major, then reads them back 16 bytes per lane
 // in row order, so one store instruction covers whole row segments (8 rows
-// of 128 bytes for the 2x8 wave tile).  Two passes of half the wave's
-// tokens each.  Needs every wave past its last activation read and no DMA
+// of 128 bytes for A = 2), in passes of as many token tiles as fit.  Needs every wave past its last activation read and no DMA
 // in flight (the caller's barrier).  Rounding is that of store_one_tile:
 // bf16 products, then the residual added in fp32 and rounded again.
 //
@@ -796,33 +820,33 @@ __device__ __forceinline__ int epi_pos(int r, int c) {
   return r * C + ((c ^ ((r ^ (r >> 3)) & kMask)) << 4);
 }
 
-template <int EPI, int A, int TB>
+template <int EPI, int A, int TB, int WN>
 __device__ __forceinline__ void store_tile_lds(const f32x16_t (&acc)[A][TB], const Args& g, int nb, int mb,
                                                unsigned char* xa, unsigned char* xb) {
-  constexpr int WN = TB / 2;
   constexpr bool kSilu = EPI == static_cast<int>(Epilogue::kSiluMul);
   constexpr int C = kSilu ? 32 * A : 64 * A;  // output bytes per token of this wave
-  constexpr int HB = TB / 2;                  // token tiles per pass
-  constexpr int kChunks = HB * 32 * C / 16;   // 16-byte chunks per pass
-  static_assert(HB * 32 * C <= 16384, "a pass must fit the wave's 16 KB region");
-  static_assert(kChunks % 64 == 0, "whole chunks per lane");
+  constexpr int kRegion = kXStageBytes<TB, WN> / 2;  // of each wave
+  constexpr int HB = kRegion / (32 * C) < TB ? kRegion / (32 * C) : TB;  // token tiles per pass
+  static_assert(HB >= 1 && 32 * C / 16 % 64 == 0, "a pass fits the wave's region, in whole chunks per lane");
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wn = wave % WN;
   const int wm = wave / WN;
   const int li = lane & 31;
   const int kg = lane >> 5;
-  unsigned char* reg = (wave < 2 ? xa : xb) + (wave & 1) * 16384;
+  unsigned char* reg = (wave < 2 ? xa : xb) + (wave & 1) * kRegion;
   // First output column of this wave and its first token.
   const int n0 = (nb * WN + wn) * A * (kSilu ? 16 : 32);
-  const int t0 = mb * BM + wm * TB * 32;
+  const int t0 = mb * kBM<TB, WN> + wm * TB * 32;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int b0 = 0; b0 < TB; b0 += HB) {
+    constexpr int kTileChunks = 32 * C / 16;  // 16-byte chunks of one token tile
+    const int tiles = TB - b0 < HB ? TB - b0 : HB;
 #pragma unroll
-    for (int b = 0; b < HB; ++b)
+    for (int b = 0; b < HB && b0 + b < TB; ++b)
 #pragma unroll
       for (int a = 0; a < A; ++a) {
-        const f32x16_t& v = acc[a][h * HB + b];
+        const f32x16_t& v = acc[a][b0 + b];
         const int r = b * 32 + li;
         if constexpr (kSilu) {
           // rows 8jj + 4kg + e of the tile are gate, 16 + the same are up
@@ -848,11 +872,11 @@ __device__ __forceinline__ void store_tile_lds(const f32x16_t (&acc)[A][TB], con
     // The same wave reads back what it wrote: LDS executes one wave's
     // accesses in order.
 #pragma unroll
-    for (int i = 0; i < kChunks / 64; ++i) {
+    for (int i = 0; i < tiles * kTileChunks / 64; ++i) {
       const int k = i * 64 + lane;
       const int r = k / (C / 16);
       const int c = k % (C / 16);
-      const int m = t0 + h * HB * 32 + r;
+      const int m = t0 + b0 * 32 + r;
       const u32x4_t q = *reinterpret_cast<const u32x4_t*>(reg + epi_pos<C>(r, c));
       if (m >= g.M) continue;
       const int n = n0 + c * 8;
@@ -959,11 +983,17 @@ struct Split {
   unsigned spin_limit;      // polls of the arrival word before a wait gives up
 };
 
-template <int EPI, int A, int TB>
+template <int EPI, int A, int TB, int WN>
 __global__ __launch_bounds__(kThreads, 1) void gemm_wdx_kernel(Args g, Split k) {
-  __shared__ __attribute__((aligned(1024))) unsigned char xa[kXStageBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char xb[kXStageBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char xc[kXStageBytes];
+  constexpr int kStage = kXStageBytes<TB, WN>, kBuffers = kXAhead<A, TB> + 1;
+  // One array per buffer: in one array the compiler could not tell the DMA
+  // targets and the fragment reads apart and would drain every load.
+  __shared__ __attribute__((aligned(1024))) unsigned char xa[kStage];
+  __shared__ __attribute__((aligned(1024))) unsigned char xb[kStage];
+  __shared__ __attribute__((aligned(1024))) unsigned char xc[kStage];
+  __shared__ __attribute__((aligned(1024))) unsigned char xd[kBuffers > 3 ? kStage : 16];
+  __shared__ __attribute__((aligned(1024))) unsigned char xe[kBuffers > 4 ? kStage : 16];
+  const XBuffers xs{{xa, xb, xc, xd, xe}};
   const int tid = threadIdx.x;
   const int b = blockIdx.x;
   f32x16_t acc[A][TB];
@@ -975,13 +1005,13 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wdx_kernel(Args g, Split k) 
     const int t = k.dp % 8 == 0 ? (b % 8) * (k.dp / 8) + b / 8 : b;
     int nb, mb;
     tile_coords(t, g.n_blocks, g.m_blocks, nb, mb);
-    mainloop(acc, g, xa, xb, xc, nb, mb, 0, g.KT / 2);
+    mainloop<A, TB, WN>(acc, g, xs, nb, mb, 0, g.KT / 2);
     // The last stages' activation DMAs (clamped, never read) may still be
     // writing the buffers and other waves may still read them: both end
     // before the epilogue reuses them.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    store_tile_lds<EPI, A, TB>(acc, g, nb, mb, xa, xb);
+    store_tile_lds<EPI, A, TB, WN>(acc, g, nb, mb, xa, xb);
     return;
   }
   // Chunk-major order: all split blocks' chunk 0, then chunk 1, ...
@@ -1004,7 +1034,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wdx_kernel(Args g, Split k) 
     tile_coords(k.dp + i, g.n_blocks, g.m_blocks, nb, mb);
   }
   const int u0 = chunk * k.units / k.S, u1 = (chunk + 1) * k.units / k.S;
-  mainloop(acc, g, xa, xb, xc, nb, mb, 2 * u0, 2 * u1);
+  mainloop<A, TB, WN>(acc, g, xs, nb, mb, 2 * u0, 2 * u1);
 
   // This workgroup sums tiles [ab0, ab1) of the block (each thread its own
   // quads of them); it keeps its partial of those in its accumulators and
@@ -1095,7 +1125,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wdx_kernel(Args g, Split k) 
         for (int q = 0; q < 4; ++q) sum[q] = f32x4_t{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""),
                                                      __builtin_nanf("")};
       }
-      store_one_tile<EPI, A, TB>(
+      store_one_tile<EPI, A, TB, WN>(
           [&](int p) { return make_float2(sum[p >> 1][2 * (p & 1)], sum[p >> 1][2 * (p & 1) + 1]); }, g, nb, mb, a,
           bb);
     }
@@ -1197,10 +1227,10 @@ inline int choose_tiles(int N, int m_blocks, int grid, int units, int split_grid
 }
 
 // `grid` = CUs available to the split (0: no split, no workspace needed).
-template <int EPI, int A, int TB>
+template <int EPI, int A, int TB, int WN>
 hipError_t launch(const void* w, int N, int K, const void* x, int M, int ldx, void* y, int ldy,
                   const void* residual, int ldr, void* workspace, int grid, hipStream_t stream) {
-  const Args g = make_args(kBN<A, TB>, w, N, K, x, M, ldx, y, ldy, residual, ldr);
+  const Args g = make_args(kBN<A, WN>, w, N, K, x, M, ldx, y, ldy, residual, ldr);
   const int T = g.n_blocks * g.m_blocks;
   Split k;
   k.units = g.KT / 4;
@@ -1212,7 +1242,7 @@ hipError_t launch(const void* w, int N, int K, const void* x, int M, int ldx, vo
   k.partials = ws != nullptr ? ws + kSkPartialsOffset : nullptr;
   k.partial_bytes = (unsigned)((size_t)k.R * k.S * kSkPartialBytes);
   k.spin_limit = g_wait_limit.load(std::memory_order_relaxed);
-  launch_kernel(gemm_wdx_kernel<EPI, A, TB>, dim3(k.dp + k.R * k.S), dim3(kThreads), 0, stream, g, k);
+  launch_kernel(gemm_wdx_kernel<EPI, A, TB, WN>, dim3(k.dp + k.R * k.S), dim3(kThreads), 0, stream, g, k);
   return hipGetLastError();
 }
 
@@ -1250,7 +1280,7 @@ hipError_t sk_grid(int device, int* grid_out) {
     hipError_t err = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
     if (err != hipSuccess) return err;
     err = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, reinterpret_cast<const void*>(&wdx::gemm_wdx_kernel<0, 2, 8>), wdx::kThreads, 0);
+        &per_cu, reinterpret_cast<const void*>(&wdx::gemm_wdx_kernel<0, 2, 8, 4>), wdx::kThreads, 0);
     if (err != hipSuccess) return err;
     int grid = cus * (per_cu > 0 ? per_cu : 1);
     cache[device] = grid < kSkMaxGrid ? grid : kSkMaxGrid;
@@ -1319,25 +1349,39 @@ hipError_t launch_gemm_linear(const void* w, int N, int K, const void* x, int M,
     const hipError_t err = wdx_plan(M, N, K, workspace != nullptr, &grid, &tiles);
     if (err != hipSuccess) return err;
     void* ws = grid > 0 ? workspace : nullptr;
-    auto go = [&](auto a_tag, auto tb_tag) -> hipError_t {
+    auto go = [&](auto a_tag, auto tb_tag, auto wn_tag) -> hipError_t {
       constexpr int A = decltype(a_tag)::value;
       constexpr int TB = decltype(tb_tag)::value;
+      constexpr int WN = decltype(wn_tag)::value;
       switch (epi) {
         case Epilogue::kSiluMul:
-          return wdx::launch<1, A, TB>(w, N, K, x, M, ldx, y, ldy, residual, ldr, ws, grid, stream);
+          return wdx::launch<1, A, TB, WN>(w, N, K, x, M, ldx, y, ldy, residual, ldr, ws, grid, stream);
         case Epilogue::kResidualAdd:
-          return wdx::launch<2, A, TB>(w, N, K, x, M, ldx, y, ldy, residual, ldr, ws, grid, stream);
+          return wdx::launch<2, A, TB, WN>(w, N, K, x, M, ldx, y, ldy, residual, ldr, ws, grid, stream);
         case Epilogue::kNone:
         default:
-          return wdx::launch<0, A, TB>(w, N, K, x, M, ldx, y, ldy, residual, ldr, ws, grid, stream);
+          return wdx::launch<0, A, TB, WN>(w, N, K, x, M, ldx, y, ldy, residual, ldr, ws, grid, stream);
       }
     };
-    // 256-row blocks run the (2, 8) wave tile: every wave over all 256
-    // tokens, so each weight fragment is fetched by one wave only (4-9 %
-    // faster than (4, 4), whose wave pairs fetched every weight line twice).
-    if (tiles == 3) return go(std::integral_constant<int, 3>{}, std::integral_constant<int, 4>{});
-    if (tiles == 1) return go(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{});
-    return go(std::integral_constant<int, 2>{}, std::integral_constant<int, 8>{});
+    using std::integral_constant;
+    if (tiles == 3) return go(integral_constant<int, 3>{}, integral_constant<int, 4>{}, integral_constant<int, 2>{});
+    // 256- and 128-row blocks: every wave over all of the block's tokens, so
+    // each weight fragment is fetched by one wave only (4-9 % faster than a
+    // (4, 4) wave tile, whose wave pairs fetched every weight line twice).
+    // ceil(M / 256) token blocks of equal size, in 32-token tiles: 301 tokens
+    // run as 2 x 160 instead of 2 x 256 (gate_up + SiLU*up 57.5 -> 47.0 us, QKV
+    // 25.4 -> 22.5; at 129 tokens 40.7 -> 35.9 and 21.7 -> 18.6).
+    const int m_blocks = (M + wdx::BM - 1) / wdx::BM;
+    const int tb = ((M + m_blocks - 1) / m_blocks + 31) / 32;
+    auto by_tokens = [&](auto a_tag) -> hipError_t {
+      constexpr integral_constant<int, 4> wn{};
+      if (tb <= 5) return go(a_tag, integral_constant<int, 5>{}, wn);
+      if (tb == 6) return go(a_tag, integral_constant<int, 6>{}, wn);
+      if (tb == 7) return go(a_tag, integral_constant<int, 7>{}, wn);
+      return go(a_tag, integral_constant<int, 8>{}, wn);
+    };
+    if (tiles == 1) return by_tokens(integral_constant<int, 1>{});
+    return by_tokens(integral_constant<int, 2>{});
   }
   if (M > kGemmBM && N % big::BN == 0 && K % big::BK == 0) {
     switch (epi) {
