@@ -47,16 +47,18 @@ def _plain_eager(*tensors: torch.Tensor) -> bool:
     for: bfloat16 GPU tensors of one device at 16-byte aligned addresses, and
     nothing around the call that follows torch ops one by one (autograd, forward-mode
     AD, functorch transforms, tracing, compilation, autocast, torch modes)."""
-    device = tensors[0].device
-    if device.type != "cuda" or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda"):
-        return False
+    device = tensors[0].get_device()  # -1 off the GPU
     c = torch._C
-    if (c._get_tracing_state() is not None or c._len_torch_dispatch_stack() or c._len_torch_function_stack()
+    if (device < 0 or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")
+            or c._get_tracing_state() is not None or c._len_torch_dispatch_stack() or c._len_torch_function_stack()
             or c._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0):
         return False
     grad = torch.is_grad_enabled()
-    return all(type(t) in _PLAIN_TYPES and t.dtype is torch.bfloat16 and t.device == device
-               and not (grad and t.requires_grad) and t.data_ptr() % 16 == 0 for t in tensors)
+    for t in tensors:
+        if (type(t) not in _PLAIN_TYPES or t.dtype is not torch.bfloat16 or t.get_device() != device
+                or (grad and t.requires_grad) or t.data_ptr() % 16):
+            return False
+    return True
 
 
 def qwen_rmsnorm(hidden_states: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
@@ -65,7 +67,7 @@ def qwen_rmsnorm(hidden_states: torch.Tensor, weight: torch.Tensor, eps: float) 
     if (k % 512 == 0 and 0 < k <= kernels.RMSNORM_MAX_K and weight.shape == (k,) and isinstance(eps, float)
             and 0.0 <= eps < math.inf and _plain_eager(hidden_states, weight) and hidden_states.is_contiguous()
             and weight.is_contiguous()):
-        return kernels.rmsnorm_rows(hidden_states, weight, eps)
+        return kernels._rmsnorm_rows(hidden_states, weight, eps)
     return F.rms_norm(hidden_states, normalized_shape=(hidden_states.shape[-1],), weight=weight, eps=eps)
 
 
@@ -115,7 +117,8 @@ def _attend_row(query_states, key_states, value_states, attention_scale, num_key
             and (n_kv == 1 or key_states.stride(1) >= rows * d)
             and isinstance(attention_scale, float) and math.isfinite(attention_scale)
             and query_states.is_contiguous() and _plain_eager(query_states, key_states, value_states)):
-        return kernels.gqa_attention(query_states[0, :, 0], key_states[0], value_states[0], attention_scale)
+        return kernels._gqa_attention(query_states.view(n_q, d), key_states.select(0, 0), value_states.select(0, 0),
+                                     attention_scale)
     return None
 
 
@@ -170,9 +173,9 @@ def _semantic_attention_qkv(hidden_states, qkv_proj_weight, q_proj_out_dim, k_pr
     qkv_states = kernels.linear(hidden_states, w)
     if _qk_kernel_serves(qkv_states, q_proj_out_dim, k_proj_out_dim, num_attention_heads, num_key_value_heads, head_dim,
                          q_norm_weight, k_norm_weight, cos, sin, rms_norm_eps):
-        query_states, key_states = kernels.qk_norm_rope(
-            qkv_states, q_norm_weight, k_norm_weight, rms_norm_eps, cos, sin,
-            num_attention_heads=num_attention_heads, num_key_value_heads=num_key_value_heads)
+        query_states, key_states = kernels._qk_norm_rope(
+            qkv_states, q_norm_weight, k_norm_weight, rms_norm_eps, cos, sin, num_attention_heads,
+            num_key_value_heads)
         value_states = qkv_states[..., q_proj_out_dim + k_proj_out_dim :].view(
             batch_size, query_len, num_key_value_heads, head_dim).transpose(1, 2)
         return query_states, key_states, value_states
@@ -202,11 +205,11 @@ def _semantic_attention_qkv_vector(hidden_states, qkv_proj_weight, q_proj_out_di
 def _qkv_heads_vector(qkv_states, q_proj_out_dim, k_proj_out_dim, num_attention_heads, num_key_value_heads,
                       head_dim, q_norm_weight, k_norm_weight, cos, sin, rms_norm_eps):
     """Split a [qkv] row into heads, q/k norm and RoPE (qwen_explicit.py:788-806)."""
-    if _qk_kernel_serves(qkv_states.view(1, 1, -1), q_proj_out_dim, k_proj_out_dim, num_attention_heads,
+    rows = qkv_states.view(1, 1, -1)
+    if _qk_kernel_serves(rows, q_proj_out_dim, k_proj_out_dim, num_attention_heads,
                          num_key_value_heads, head_dim, q_norm_weight, k_norm_weight, cos, sin, rms_norm_eps):
-        query_states, key_states = kernels.qk_norm_rope(
-            qkv_states.view(1, 1, -1), q_norm_weight, k_norm_weight, rms_norm_eps, cos, sin,
-            num_attention_heads=num_attention_heads, num_key_value_heads=num_key_value_heads)
+        query_states, key_states = kernels._qk_norm_rope(
+            rows, q_norm_weight, k_norm_weight, rms_norm_eps, cos, sin, num_attention_heads, num_key_value_heads)
         return query_states, key_states, qkv_states[q_proj_out_dim + k_proj_out_dim :].view(
             1, num_key_value_heads, 1, head_dim)
     query_states, key_states, value_states = torch.split(

@@ -9,7 +9,9 @@ another implementation: a missing library or a rejected argument raises.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import functools
 
 import torch
 
@@ -17,8 +19,22 @@ from . import _lib
 from .layout import PackedWeight
 
 
+# The wrappers run for every projection of every token, so their host time is
+# kept below the kernels': tensor attributes that need no Python object
+# (is_cuda, get_device), the raw stream handle and device index straight from
+# torch's bindings, a device switch only where the call's device is not the
+# current one, and sizes that depend on the shape alone looked up once.  One
+# decode layer of five calls: 89 -> 52 us, the kernels' own time.
+_NO_SWITCH = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """Context in which a GPU tensor's `device` is current."""
+    return _NO_SWITCH if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
+
+
 def _require_device(t: torch.Tensor, what: str) -> None:
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{what} must be a GPU tensor, got device {t.device}")
 
 
@@ -26,21 +42,24 @@ def _one_device(first: torch.Tensor, *named: tuple[torch.Tensor | None, str]) ->
     """The device of `first`, after checking that every other tensor given
     (None skipped) lives on it: the C layer launches on one device and sees
     only pointers."""
-    dev = first.device
+    index, dev = first.get_device(), first.device
     for t, what in named:
-        if t is not None and t.device != dev:
+        if t is not None and (t.get_device() != index or (index < 0 and t.device != dev)):
             raise ValueError(f"{what} is on {t.device}, the call's tensors are on {dev}")
     return dev
 
 
 def _rows(x: torch.Tensor, k: int, what: str) -> tuple[torch.Tensor, int, int]:
-    """View x as [M, k] rows with unit column stride; returns (x2d, M, ld).
-    Rows the kernels cannot read in place (column stride, row stride not a
-    multiple of 8 or above the library's largest, misalignment) are copied."""
-    if x.dtype != torch.bfloat16:
+    """x as [M, k] rows with unit column stride: the tensor whose data_ptr()
+    they start at, M, and the row stride.  Rows the kernels cannot read in
+    place (column stride, row stride not a multiple of 8 or above the
+    library's largest, misalignment) are copied."""
+    if x.dtype is not torch.bfloat16:
         raise ValueError(f"{what} must be bfloat16, got {x.dtype}")
     if x.shape[-1] != k:
         raise ValueError(f"{what} last dim {x.shape[-1]} != K={k}")
+    if x.is_contiguous() and k % 8 == 0 and k <= _lib.MAX_ACTIVATION_STRIDE and x.data_ptr() % 16 == 0:
+        return x, x.numel() // k, k
     x2 = x.reshape(-1, k)
     if (x2.stride(-1) != 1 or (x2.shape[0] > 1 and (x2.stride(0) % 8 or x2.stride(0) > _lib.MAX_ACTIVATION_STRIDE))
             or x2.data_ptr() % 16):
@@ -50,7 +69,7 @@ def _rows(x: torch.Tensor, k: int, what: str) -> tuple[torch.Tensor, int, int]:
 
 
 def stream_handle() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _check_out(out: torch.Tensor, m: int, n_out: int, dtype: torch.dtype, what: str = "out") -> None:
@@ -76,7 +95,8 @@ def _device_workspace(cache: dict[tuple[int, int], torch.Tensor], device: torch.
     zero fill (run the same launch once on the capture stream before the
     capture); a graph keeps using the workspace of the stream it was captured
     on, so eager calls on that stream must not overlap its replays."""
-    key = (_device_index(device), torch.cuda.current_stream(device).cuda_stream)
+    index = _device_index(device)
+    key = (index, torch._C._cuda_getCurrentRawStream(index))
     ws = cache.get(key)
     if ws is None or ws.numel() < nbytes:
         if torch.cuda.is_current_stream_capturing():
@@ -90,11 +110,18 @@ def _device_workspace(cache: dict[tuple[int, int], torch.Tensor], device: torch.
 _prefill_workspaces: dict[tuple[int, int], torch.Tensor] = {}
 
 
+@functools.lru_cache(maxsize=4096)
+def _linear_workspace_bytes(current_device: int, m: int, n: int, k: int) -> int:
+    """lsk_workspace_bytes of a projection: a function of the shape and the
+    current device's CU count."""
+    return _lib.load().lsk_workspace_bytes(_lib.OP_LINEAR, m, n, k)
+
+
 def prefill_workspace(device: torch.device, m: int, n: int, k: int) -> torch.Tensor | None:
     """The split-K workspace of the prefill GEMM on `device` for the current
     stream (zero-filled once, left zero-filled by every call), or None when
     the shape does not use one."""
-    nbytes = _lib.load().lsk_workspace_bytes(_lib.OP_LINEAR, m, n, k)
+    nbytes = _linear_workspace_bytes(torch._C._cuda_getDevice(), m, n, k)
     if nbytes == 0:
         return None
     return _device_workspace(_prefill_workspaces, device, nbytes, "prefill")
@@ -166,7 +193,7 @@ def linear(x: torch.Tensor, weight: PackedWeight, *, epilogue: int = _lib.EPI_NO
     _require_device(x, "x")
     _require_device(weight.data, "weight")
     if out is None:
-        out = torch.empty((*x.shape[:-1], n_out), device=x.device, dtype=torch.bfloat16)
+        out = x.new_empty((*x.shape[:-1], n_out))
     _require_device(out, "out")
     res_ptr, ldr = (None, 0) if r2 is None else (r2.data_ptr(), ldr)
     if r2 is not None:
@@ -182,7 +209,7 @@ def linear(x: torch.Tensor, weight: PackedWeight, *, epilogue: int = _lib.EPI_NO
         _require_device(workspace, "workspace")
         ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
     dev = _one_device(x, (weight.data, "weight"), (out, "out"), (r2, "residual"), (workspace, "workspace"))
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = lib.lsk_linear_bf16(
             weight.data.data_ptr(), weight.layout, weight.n, weight.k,
             x2.data_ptr(), m, ldx,
@@ -221,7 +248,7 @@ def rmsnorm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, weigh
     if nw.stride(0) != 1 or nw.data_ptr() % 16:
         nw = nw.contiguous() if nw.stride(0) != 1 else nw.clone()
     if out is None:
-        out = torch.empty((*x.shape[:-1], n_out), device=x.device, dtype=torch.bfloat16)
+        out = x.new_empty((*x.shape[:-1], n_out))
     _require_device(out, "out")
     res_ptr, ldr = (None, 0) if r2 is None else (r2.data_ptr(), ldr)
     if r2 is not None:
@@ -229,7 +256,7 @@ def rmsnorm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, weigh
     if m == 0:
         return out
     dev = _one_device(x, (weight.data, "weight"), (nw, "norm_weight"), (out, "out"), (r2, "residual"))
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = lib.lsk_rmsnorm_linear_bf16(
             weight.data.data_ptr(), weight.layout, weight.n, weight.k,
             x2.data_ptr(), m, ldx,
@@ -255,12 +282,18 @@ def rmsnorm_rows(x: torch.Tensor, norm_weight: torch.Tensor, eps: float) -> torc
         raise ValueError("x and norm_weight must be contiguous")
     _require_device(x, "x")
     _require_device(norm_weight, "norm_weight")
-    dev = _one_device(x, (norm_weight, "norm_weight"))
-    out = torch.empty_like(x)
+    _one_device(x, (norm_weight, "norm_weight"))
+    return _rmsnorm_rows(x, norm_weight, eps)
+
+
+def _rmsnorm_rows(x: torch.Tensor, norm_weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """rmsnorm_rows of tensors already known to fit it."""
+    k = x.shape[-1]
+    out = x.new_empty(x.shape)
     m = x.numel() // k if k else 0
     if m == 0:
         return out
-    with torch.cuda.device(dev):
+    with _on(x.device):
         status = _lib.load().lsk_rmsnorm_bf16(x.data_ptr(), m, k, k, norm_weight.data_ptr(), float(eps),
                                               out.data_ptr(), stream_handle())
     _lib.check(status, "lsk_rmsnorm_bf16")
@@ -291,13 +324,20 @@ def qk_norm_rope(qkv: torch.Tensor, q_norm_weight: torch.Tensor, k_norm_weight: 
             or cos.shape[1] not in (1, t) or cos.shape[2] != d // 2 or cos.stride(2) != 1):
         raise ValueError(f"cos / sin must be [{b} or 1, {t} or 1, {d // 2}] with equal strides and contiguous rows, got "
                          f"{tuple(cos.shape)} / {tuple(sin.shape)}")
-    dev = _one_device(qkv, (q_norm_weight, "q_norm_weight"), (k_norm_weight, "k_norm_weight"), (cos, "cos"),
-                      (sin, "sin"))
-    q = torch.empty((b, n_q, t, d), device=qkv.device, dtype=torch.bfloat16)
-    k = torch.empty((b, n_kv, t, d), device=qkv.device, dtype=torch.bfloat16)
+    _one_device(qkv, (q_norm_weight, "q_norm_weight"), (k_norm_weight, "k_norm_weight"), (cos, "cos"), (sin, "sin"))
+    return _qk_norm_rope(qkv, q_norm_weight, k_norm_weight, eps, cos, sin, n_q, n_kv)
+
+
+def _qk_norm_rope(qkv: torch.Tensor, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, eps: float,
+                  cos: torch.Tensor, sin: torch.Tensor, n_q: int, n_kv: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """qk_norm_rope of tensors already known to fit it."""
+    b, t, n = qkv.shape
+    d = n // (n_q + 2 * n_kv)
+    q = qkv.new_empty((b, n_q, t, d))
+    k = qkv.new_empty((b, n_kv, t, d))
     if b * t == 0:
         return q, k
-    with torch.cuda.device(dev):
+    with _on(qkv.device):
         status = _lib.load().lsk_qk_norm_rope_bf16(
             qkv.data_ptr(), b, t, n, n_q, n_kv, d, q_norm_weight.data_ptr(), k_norm_weight.data_ptr(), float(eps),
             cos.data_ptr(), sin.data_ptr(), cos.stride(0) if cos.shape[0] > 1 else 0,
@@ -309,12 +349,17 @@ def qk_norm_rope(qkv: torch.Tensor, q_norm_weight: torch.Tensor, k_norm_weight: 
 _attention_workspaces: dict[tuple[int, int], torch.Tensor] = {}
 
 
+@functools.lru_cache(maxsize=1024)
+def _attention_workspace_bytes(n_q: int, n_kv: int, head_dim: int, max_seq_len: int) -> int:
+    return _lib.load().lsk_attention_workspace_bytes(n_q, n_kv, head_dim, max_seq_len)
+
+
 def attention_workspace(device: torch.device, n_q: int, n_kv: int, head_dim: int,
                         max_seq_len: int) -> torch.Tensor:
     """The decode attention workspace of `device` for the current stream
     (zero-filled once, left zero-filled by every call), large enough for this
     geometry.  Calls on other streams get their own."""
-    nbytes = _lib.load().lsk_attention_workspace_bytes(n_q, n_kv, head_dim, max_seq_len)
+    nbytes = _attention_workspace_bytes(n_q, n_kv, head_dim, max_seq_len)
     if nbytes == 0:
         raise ValueError(f"no attention workspace for n_q={n_q}, n_kv={n_kv}, head_dim={head_dim}, "
                          f"max_seq_len={max_seq_len}")
@@ -362,9 +407,9 @@ def decode_attention(qkv: torch.Tensor, q_norm_weight: torch.Tensor, k_norm_weig
         _require_device(pos, "pos")
         if pos.dtype != torch.int32 or pos.numel() != 1:
             raise ValueError("a device pos must be a one-element int32 tensor")
-    flat = [t.reshape(-1).contiguous() for t in (qkv, q_norm_weight, k_norm_weight, cos, sin)]
+    flat = [t if t.is_contiguous() else t.reshape(-1).contiguous() for t in (qkv, q_norm_weight, k_norm_weight, cos, sin)]
     if out is None:
-        out = torch.empty((n_q * d,), device=qkv.device, dtype=torch.bfloat16)
+        out = qkv.new_empty((n_q * d,))
     if out.dtype != torch.bfloat16 or out.numel() != n_q * d or not out.is_contiguous():
         raise ValueError(f"out must be a contiguous bfloat16 tensor of {n_q * d} values")
     if isinstance(workspace, str):
@@ -378,7 +423,7 @@ def decode_attention(qkv: torch.Tensor, q_norm_weight: torch.Tensor, k_norm_weig
     common = (flat[0].data_ptr(), n_q, n_kv, d, flat[1].data_ptr(), flat[2].data_ptr(), float(eps),
               flat[3].data_ptr(), flat[4].data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), s_max)
     tail = (float(scale), out.data_ptr(), workspace.data_ptr(), workspace.numel() * workspace.element_size())
-    with torch.cuda.device(dev):
+    with _on(dev):
         tail += (stream_handle(),)
         if on_device:
             status = lib.lsk_decode_attention_at_bf16(*common, pos.data_ptr(), *tail)
@@ -424,13 +469,20 @@ def gqa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: floa
             or not q.is_contiguous():
         raise ValueError(f"q must be contiguous [n_q, {d}] and k / v [n_kv, rows, {d}] with equal strides and "
                          f"contiguous rows, got {tuple(q.shape)}, {tuple(k.shape)} / {tuple(v.shape)}")
-    dev = _one_device(q, (k, "k"), (v, "v"))
+    _one_device(q, (k, "k"), (v, "v"))
+    return _gqa_attention(q, k, v, scale)
+
+
+def _gqa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float) -> torch.Tensor:
+    """gqa_attention of tensors already known to fit it."""
+    n_q, d = q.shape
+    n_kv, rows, _ = k.shape
     lib = _lib.load()
-    out = torch.empty((n_q * d,), device=q.device, dtype=torch.bfloat16)
-    with torch.cuda.device(dev):
+    out = q.new_empty((n_q * d,))
+    with _on(q.device):
         workspace = None
         if rows > 128:  # sized for the longest cache: one workspace as a sequence grows
-            workspace = _gqa_workspace(dev, lib.lsk_attention_workspace_bytes(n_q, n_kv, d, ATTENTION_MAX_ROWS))
+            workspace = _gqa_workspace(q.device, _attention_workspace_bytes(n_q, n_kv, d, ATTENTION_MAX_ROWS))
         status = lib.lsk_gqa_attention_bf16(
             q.data_ptr(), n_q, n_kv, d, k.data_ptr(), v.data_ptr(), max(k.stride(0), rows * d), rows, float(scale),
             out.data_ptr(), None if workspace is None else workspace.data_ptr(),
@@ -500,7 +552,7 @@ def lm_head_argmax(hidden: torch.Tensor, weight: PackedWeight, *, logits_mode: i
     if norm_weight is not None:
         _require_device(norm_weight, "norm_weight")
         nw = norm_weight.reshape(-1).contiguous()
-        with torch.cuda.device(dev):
+        with _on(dev):
             status = lib.lsk_rmsnorm_lm_head_argmax_bf16(
                 weight.data.data_ptr(), weight.layout, v, weight.k, h2.data_ptr(), m, ldx, nw.data_ptr(), float(eps),
                 logits_ptr, logits_mode, out.data_ptr(), workspace.buffer.data_ptr(), workspace.buffer.numel(),
@@ -508,7 +560,7 @@ def lm_head_argmax(hidden: torch.Tensor, weight: PackedWeight, *, logits_mode: i
             )
         _lib.check(status, "lsk_rmsnorm_lm_head_argmax_bf16")
         return out
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = lib.lsk_lm_head_argmax_bf16(
             weight.data.data_ptr(), weight.layout, v, weight.k,
             h2.data_ptr(), m, ldx,
@@ -543,7 +595,7 @@ def lm_head_argmax_noalloc(hidden: torch.Tensor, weight: PackedWeight, out: torc
     if m == 0:
         return out
     dev = _one_device(hidden, (weight.data, "weight"), (out, "out"), (logits_out, "logits_out"))
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = _lib.load().lsk_lm_head_argmax_noalloc_bf16(
             weight.data.data_ptr(), weight.layout, weight.n, weight.k, hidden.data_ptr(), m, weight.k,
             logits_out.data_ptr() if logits_out is not None else None, logits_mode, out.data_ptr(), stream_handle())

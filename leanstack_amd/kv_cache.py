@@ -61,7 +61,8 @@ class ArenaKVCache:
 
     def layer_tensors(self, layer: int) -> tuple[torch.Tensor, torch.Tensor]:
         """The layer's whole key and value blocks, [n_kv, capacity, d] each."""
-        return self.storage[layer, 0], self.storage[layer, 1]
+        blocks = self.storage.select(0, layer)
+        return blocks.select(0, 0), blocks.select(0, 1)
 
     def advance(self, layer: int, rows: int) -> None:
         """Count `rows` rows written after the layer's cursor (by the decode
@@ -103,8 +104,8 @@ class ArenaKVCache:
                              f"[{k_block.shape[0]}, rows, {k_block.shape[2]}]")
         start = self.layer_seq_lens[layer]
         self.advance(layer, keys.shape[1])
-        k_block[:, start : start + keys.shape[1]].copy_(keys)
-        v_block[:, start : start + keys.shape[1]].copy_(values)
+        k_block.narrow(1, start, keys.shape[1]).copy_(keys)
+        v_block.narrow(1, start, keys.shape[1]).copy_(values)
 
     def attended(self, layer: int) -> tuple[torch.Tensor, torch.Tensor]:
         """The layer's written rows as [1, n_kv, rows, d] views (what the
