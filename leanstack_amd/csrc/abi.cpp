@@ -168,18 +168,20 @@ int lsk_linear_bf16(const void* w_packed, int layout_id, int N, int K, const voi
   const auto epi = static_cast<lsk::Epilogue>(epilogue);
   hipError_t err;
   const bool gemm_shape = N % lsk::kGemmBN == 0 && K % lsk::kGemmBK == 0;
-  if (M <= lsk::kDecodeMaxM) {
-    err = lsk::launch_decode_linear(w_packed, N, K, x, M, ldx, y, ldy, epi, residual, ldr, stream);
-  } else if (lsk::skinny_route(M, N, K, epi == lsk::Epilogue::kSiluMul)) {
+  const bool silu = epi == lsk::Epilogue::kSiluMul;
+  if (lsk::skinny_route(M, N, K, silu)) {
+    if (M <= lsk::kDecodeMaxM) workspace = nullptr;  // ignored there
     int cus = 0;
     err = lsk::current_device_cus(&cus);
     if (err != hipSuccess) return hip_fail(err, "device CU count");
-    const lsk::SkinnyPlan p = lsk::skinny_plan(M, N, K, epi == lsk::Epilogue::kSiluMul, cus, workspace != nullptr);
+    const lsk::SkinnyPlan p = lsk::skinny_plan(M, N, K, silu, cus, workspace != nullptr);
     if (p.S > 1 && (ws_bytes < p.bytes || !aligned(workspace, 256)))
       return fail(LSK_ERR_WORKSPACE, "projection workspace needs %zu bytes, 256-byte aligned (got %zu)", p.bytes,
                   ws_bytes);
     err = lsk::launch_skinny_linear(w_packed, N, K, x, M, ldx, y, ldy, epi, residual, ldr,
                                     p.S > 1 ? workspace : nullptr, ws_bytes, cus, stream);
+  } else if (M <= lsk::kDecodeMaxM) {
+    err = lsk::launch_decode_linear(w_packed, N, K, x, M, ldx, y, ldy, epi, residual, ldr, stream);
   } else if (gemm_shape) {
     if (workspace != nullptr) {
       int device = 0;

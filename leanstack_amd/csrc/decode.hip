@@ -54,59 +54,36 @@ __device__ __forceinline__ f32x4_t mfma16(bf16x8_t a, bf16x8_t b, f32x4_t c) {
 
 __device__ __forceinline__ float bf16_to_f32(__bf16 v) { return static_cast<float>(v); }
 
-// Accumulate RBW row-blocks over this wave's K range into acc.
+// Accumulate RBW row-blocks over this wave's K range into acc, in rounds of
+// 8 / RBW k-tiles plus a remainder (any K without a single-round form).
 //   wt   : tile (rb0, 0) of the workgroup, already offset by `lane`
 //   xrow : x row (m, or row 0 for padding lanes), as 16-byte units, + g
-// U > 0: the range is exactly U k-tiles and every weight load of the wave is
-// issued in one round (one memory latency per wave).  U == 0: any length,
-// in rounds of 8 / RBW k-tiles plus a remainder.
-template <int RBW, int U>
+template <int RBW>
 __device__ __forceinline__ void accumulate_rows(f32x4_t (&acc)[RBW], const bf16x8_t* __restrict__ wt,
                                                 const bf16x8_t* __restrict__ xrow, bool m_active,
                                                 int KT, int kb, int ke) {
   const unsigned keep = m_active ? 0xffffffffu : 0u;
-  if constexpr (U > 0) {
-    // One round: every weight load of the wave goes out first (the HBM
-    // latency is paid once), then the activation fragments -- L2 hits --
-    // are fetched next to the multiplies that use them, which keeps the
-    // register footprint at the weights plus a short window.
-    bf16x8_t wv[U][RBW];
+  constexpr int R = 8 / RBW;
+  int kt = kb;
+  for (; kt + R <= ke; kt += R) {
+    bf16x8_t xv[R];
+    bf16x8_t wv[R][RBW];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < R; ++u) {
+      xv[u] = load_x_frag(xrow + (kt + u) * 4, keep);
 #pragma unroll
-      for (int r = 0; r < RBW; ++r) wv[u][r] = load_weight_tile(wt + ((size_t)r * KT + kb + u) * 64);
+      for (int r = 0; r < RBW; ++r) wv[u][r] = load_weight_tile(wt + ((size_t)r * KT + kt + u) * 64);
     }
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bf16x8_t xv = load_x_frag(xrow + (kb + u) * 4, keep);
+    for (int u = 0; u < R; ++u) {
 #pragma unroll
-      for (int r = 0; r < RBW; ++r) acc[r] = mfma16(wv[u][r], xv, acc[r]);
+      for (int r = 0; r < RBW; ++r) acc[r] = mfma16(wv[u][r], xv[u], acc[r]);
     }
-    (void)ke;
-  } else {
-    constexpr int R = 8 / RBW;
-    int kt = kb;
-    for (; kt + R <= ke; kt += R) {
-      bf16x8_t xv[R];
-      bf16x8_t wv[R][RBW];
+  }
+  for (; kt < ke; ++kt) {
+    const bf16x8_t xv = load_x_frag(xrow + kt * 4, keep);
 #pragma unroll
-      for (int u = 0; u < R; ++u) {
-        xv[u] = load_x_frag(xrow + (kt + u) * 4, keep);
-#pragma unroll
-        for (int r = 0; r < RBW; ++r) wv[u][r] = load_weight_tile(wt + ((size_t)r * KT + kt + u) * 64);
-      }
-#pragma unroll
-      for (int u = 0; u < R; ++u) {
-#pragma unroll
-        for (int r = 0; r < RBW; ++r) acc[r] = mfma16(wv[u][r], xv[u], acc[r]);
-      }
-    }
-    for (; kt < ke; ++kt) {
-      const bf16x8_t xv = load_x_frag(xrow + kt * 4, keep);
-#pragma unroll
-      for (int r = 0; r < RBW; ++r) acc[r] = mfma16(load_weight_tile(wt + ((size_t)r * KT + kt) * 64), xv, acc[r]);
-    }
+    for (int r = 0; r < RBW; ++r) acc[r] = mfma16(load_weight_tile(wt + ((size_t)r * KT + kt) * 64), xv, acc[r]);
   }
 }
 
@@ -292,19 +269,21 @@ __device__ __forceinline__ void accumulate_rows_rms_dense(f32x4_t (&acc)[RBW], c
   }
 }
 
-// Bytes of one wave's area when its slice of x is staged: the M rows of the
-// slice (row stride U*32+8 bf16), and at least the RBW partial tiles of the
-// cross-wave sum that reuse the area.
-__host__ __device__ constexpr int staged_wave_bytes(int U, int M, int RBW) {
-  return M * (U * 32 + 8) * 2 > RBW * 1024 ? M * (U * 32 + 8) * 2 : RBW * 1024;
+// Bytes of one wave's area when its slice of x is staged in PH phases: the M
+// rows of a phase's k-tiles (at most ceil(U / PH); row stride 32 per tile + 8
+// bf16), and at least the RBW partial tiles of the cross-wave sum that reuse
+// the area.
+__host__ __device__ constexpr int staged_wave_bytes(int U, int M, int RBW, int PH = 1) {
+  const int rows = M * ((U + PH - 1) / PH * 32 + 8) * 2;
+  return rows > RBW * 1024 ? rows : RBW * 1024;
 }
 
 // NORM value of the kernels' staged-activation form with NC chunks per lane
-// (NORM = 0: fragments loaded per tile; > 0 and -1: the RMSNorm prologues).
-constexpr int staged_x(int nc) { return -1 - nc; }
-// The same with the wave's x slice staged in two phases (NC chunks per lane
-// per phase): decode_linear_kernel only.
-constexpr int staged_x2(int nc) { return -101 - nc; }
+// and phase, PH phases (NORM = 0: fragments loaded per tile; > 0 and -1: the
+// RMSNorm prologues); more than one phase: the 16-row form only.
+constexpr int staged_x(int nc, int ph = 1) { return -1 - nc - 100 * (ph - 1); }
+constexpr int staged_chunks(int norm) { return (-1 - norm) % 100; }
+constexpr int staged_phases(int norm) { return (-1 - norm) / 100 + 1; }
 
 // Single-round accumulate_rows with the wave's slice of x -- M rows x U*32
 // values, M*U*4 chunks of 8 -- loaded densely (NC chunks per lane, one
@@ -318,13 +297,15 @@ template <int NW, int RBW, int U, int NC, bool HALF, int PH = 1>
 __device__ __forceinline__ void accumulate_rows_staged(f32x4_t (&acc)[RBW], const bf16x8_t* __restrict__ wt,
                                                        const __bf16* __restrict__ x, int ldx, int M, int KT, int kb,
                                                        int wave, int lane) {
-  static_assert(PH == 1 || (PH == 2 && !HALF), "two-phase staging is for the 16-row form");
-  constexpr int kRowStride = U * 32 + 8;
-  __bf16* xs = reinterpret_cast<__bf16*>(rms_lds + (size_t)wave * staged_wave_bytes(U, M, RBW));
+  static_assert(PH == 1 || !HALF, "staging in phases is for the 16-row form");
+  constexpr int kRowStride = (U + PH - 1) / PH * 32 + 8;
+  __bf16* xs = reinterpret_cast<__bf16*>(rms_lds + (size_t)wave * staged_wave_bytes(U, M, RBW, PH));
   const int m = lane & 15;
   const int g = lane >> 4;
   // Phase p stages k-tiles [kt0(p), kt0(p + 1)) of the wave's slice: M rows
-  // of (kt1 - kt0) * 4 chunks of 8 values, NC chunks per lane.
+  // of (kt1 - kt0) * 4 chunks of 8 values, NC chunks per lane, in the same
+  // LDS area (a wave's LDS accesses run in order, so a phase's stores follow
+  // the last one's reads).
   auto kt0 = [](int p) { return p * U / PH; };
   bf16x8_t xd[NC];
   auto load_phase = [&](int p) {
@@ -345,7 +326,7 @@ __device__ __forceinline__ void accumulate_rows_staged(f32x4_t (&acc)[RBW], cons
     for (int i = 0; i < NC; ++i) {
       const int c = min(lane + 64 * i, C - 1);
       const int mc = c / pc;
-      const int j = kt0(p) * 4 + c - mc * pc;
+      const int j = c - mc * pc;
       *reinterpret_cast<bf16x8_t*>(xs + mc * kRowStride + j * 8) = xd[i];
     }
   };
@@ -372,15 +353,15 @@ __device__ __forceinline__ void accumulate_rows_staged(f32x4_t (&acc)[RBW], cons
     }
   } else {
     const int mr = m < M ? m : M - 1;  // padding columns: finite, never stored
-    // The second phase's chunks load while the first phase multiplies (they
+    // The next phase's chunks load while a phase multiplies (the second's
     // queue behind the weight loads, which the first multiplies wait for).
-    if constexpr (PH == 2) load_phase(1);
 #pragma unroll
     for (int p = 0; p < PH; ++p) {
-      if (p == 1) store_phase(1);
+      if (p > 0) store_phase(p);
+      if (p + 1 < PH) load_phase(p + 1);
 #pragma unroll
       for (int u = kt0(p); u < kt0(p + 1); ++u) {
-        const bf16x8_t xn = *reinterpret_cast<const bf16x8_t*>(xs + mr * kRowStride + u * 32 + g * 8);
+        const bf16x8_t xn = *reinterpret_cast<const bf16x8_t*>(xs + mr * kRowStride + (u - kt0(p)) * 32 + g * 8);
 #pragma unroll
         for (int r = 0; r < RBW; ++r) acc[r] = mfma16(wv[u][r], xn, acc[r]);
       }
@@ -526,24 +507,21 @@ __global__ __launch_bounds__(NW * 64) void decode_linear_kernel(
   } else if constexpr (NORM == -1) {
     const bf16x8_t* nrow = reinterpret_cast<const bf16x8_t*>(norm_w) + g;
     accumulate_rows_rms<NW, RBW>(acc, wt, xrow, nrow, m_active, KT, kb, ke, wave, lane, eps);
-  } else if constexpr (NORM < -100) {
-    (void)norm_w;
-    (void)eps;
-    accumulate_rows_staged<NW, RBW, U, -101 - NORM, false, 2>(acc, wt, x, ldx, M, KT, kb, wave, lane);
   } else if constexpr (NORM < -1) {
     (void)norm_w;
     (void)eps;
-    accumulate_rows_staged<NW, RBW, U, -1 - NORM, false>(acc, wt, x, ldx, M, KT, kb, wave, lane);
+    accumulate_rows_staged<NW, RBW, U, staged_chunks(NORM), false, staged_phases(NORM)>(acc, wt, x, ldx, M, KT, kb,
+                                                                                        wave, lane);
   } else {
     (void)norm_w;
     (void)eps;
-    accumulate_rows<RBW, U>(acc, wt, xrow, m_active, KT, kb, ke);
+    accumulate_rows<RBW>(acc, wt, xrow, m_active, KT, kb, ke);
   }
 
   if constexpr (NORM > 0) {
     if (!reduce_waves_at<NW, RBW>(acc, wave, lane, rms_lds, rms_wave_bytes(U, NORM, M, RBW))) return;
   } else if constexpr (NORM < -1) {
-    if (!reduce_waves_at<NW, RBW>(acc, wave, lane, rms_lds, staged_wave_bytes(U, M, RBW))) return;
+    if (!reduce_waves_at<NW, RBW>(acc, wave, lane, rms_lds, staged_wave_bytes(U, M, RBW, staged_phases(NORM)))) return;
   } else {
     if (!reduce_waves<NW, RBW>(acc, wave, lane)) return;
   }
@@ -685,7 +663,7 @@ __device__ __forceinline__ void reduce_row_partials(ArgmaxPartial* __restrict__ 
 // best (score, index) per activation row stored as partial[m * P + slot].
 // NC > 0: the activations staged through LDS (NC chunks per lane), or with
 // NORM their RMSNorm (norm_w, eps) applied on the way (the dense prologue).
-template <int NW, int RB, int U, int NC, bool NORM>
+template <int NW, int RB, int U, int NC, bool NORM, int PH>
 __device__ __forceinline__ void lm_head_score(const bf16x8_t* __restrict__ w, const __bf16* __restrict__ x, int ldx,
                                               float* __restrict__ logits, int V, int logits_bf16,
                                               ArgmaxPartial* __restrict__ partial, int P, int M, int KT,
@@ -715,12 +693,12 @@ __device__ __forceinline__ void lm_head_score(const bf16x8_t* __restrict__ w, co
     (void)ke;
     (void)norm_w;
     (void)eps;
-    accumulate_rows_staged<NW, RB, U, NC, false>(acc, wt, x, ldx, M, KT, kb, wave, lane);
-    leader = reduce_waves_at<NW, RB>(acc, wave, lane, rms_lds, staged_wave_bytes(U, M, RB));
+    accumulate_rows_staged<NW, RB, U, NC, false, PH>(acc, wt, x, ldx, M, KT, kb, wave, lane);
+    leader = reduce_waves_at<NW, RB>(acc, wave, lane, rms_lds, staged_wave_bytes(U, M, RB, PH));
   } else {
     (void)norm_w;
     (void)eps;
-    accumulate_rows<RB, U>(acc, wt, xrow, m_active, KT, kb, ke);
+    accumulate_rows<RB>(acc, wt, xrow, m_active, KT, kb, ke);
     leader = reduce_waves<NW, RB>(acc, wave, lane);
   }
 
@@ -763,7 +741,7 @@ __device__ __forceinline__ void lm_head_score(const bf16x8_t* __restrict__ w, co
 // into out_idx[m] while the last scoring workgroups finish
 // (reduce_row_partials).  The workspace must be zero when a call starts, and
 // every call leaves it zero.
-template <int NW, int RBW, int U, int NC = 0, bool NORM = false>
+template <int NW, int RBW, int U, int NC = 0, bool NORM = false, int PH = 1>
 __global__ __launch_bounds__(NW * 64) void lm_head_kernel(
     const bf16x8_t* __restrict__ w, const __bf16* __restrict__ x, int ldx, float* __restrict__ logits,
     int V, int logits_bf16, ArgmaxPartial* __restrict__ partial, unsigned* __restrict__ status,
@@ -777,14 +755,14 @@ __global__ __launch_bounds__(NW * 64) void lm_head_kernel(
     return;
   }
   if constexpr (RBW == 1) {
-    lm_head_score<NW, 1, U, NC, NORM>(w, x, ldx, logits, V, logits_bf16, partial, P, M, KT, norm_w, eps, b, b);
+    lm_head_score<NW, 1, U, NC, NORM, PH>(w, x, ldx, logits, V, logits_bf16, partial, P, M, KT, norm_w, eps, b, b);
   } else {
     const int P2 = (V / kTileRows - P) / (RBW - 1);
     if (b < P2)
-      lm_head_score<NW, RBW, U, NC, NORM>(w, x, ldx, logits, V, logits_bf16, partial, P, M, KT, norm_w, eps,
+      lm_head_score<NW, RBW, U, NC, NORM, PH>(w, x, ldx, logits, V, logits_bf16, partial, P, M, KT, norm_w, eps,
                                           b * RBW, b);
     else
-      lm_head_score<NW, 1, U, NC, NORM>(w, x, ldx, logits, V, logits_bf16, partial, P, M, KT, norm_w, eps,
+      lm_head_score<NW, 1, U, NC, NORM, PH>(w, x, ldx, logits, V, logits_bf16, partial, P, M, KT, norm_w, eps,
                                         P2 * RBW + (b - P2), b);
   }
 }
@@ -812,15 +790,19 @@ constexpr size_t kDefaultDynamicLds = 64 * 1024;
 template <int NW, int RBW, int EPI, int U, int NORM>
 hipError_t launch_decode_cfg(const DecodeArgs& a, hipStream_t stream) {
   auto* kernel = decode_linear_kernel<NW, RBW, EPI, U, NORM>;
-  size_t lds = NORM < -1 ? (size_t)NW * staged_wave_bytes(U, a.M, RBW) : 0;
+  size_t lds = NORM < -1 ? (size_t)NW * staged_wave_bytes(U, a.M, RBW, staged_phases(NORM)) : 0;
   if constexpr (NORM < -1) {
     if (lds > kDefaultDynamicLds) {
-      // Raised once per kernel, to what M = 8 (the largest staged M) needs.
+      // Raised once per kernel, to what the most rows it is launched with
+      // (NC chunks per lane of a phase's rows) need.
       static std::once_flag once;
       static hipError_t raised = hipSuccess;
       std::call_once(once, [&] {
+        constexpr int kTiles = (U + staged_phases(NORM) - 1) / staged_phases(NORM);
+        constexpr int kRows = staged_chunks(NORM) * 64 / (4 * kTiles);
         raised = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     NW * staged_wave_bytes(U, 8, RBW));
+                                     NW * staged_wave_bytes(U, kRows < kDecodeMaxM ? kRows : kDecodeMaxM, RBW,
+                                                            staged_phases(NORM)));
       });
       if (raised != hipSuccess) return raised;
     }
@@ -869,45 +851,20 @@ __global__ __launch_bounds__(NW * 64) void decode_half_kernel(
   const int h = blockIdx.x & 1;
   const int rb0 = (blockIdx.x >> 1) * RBW;
   const bf16x8_t* wt = w + (size_t)rb0 * KT * 64 + (c >> 3) * 64 + g * 16 + 8 * h + (c & 7);
-  const bool b_lo = c < M;
-  const bool b_hi = c >= M && c < 2 * M;
-  const unsigned keep = (b_lo || b_hi) ? 0xffffffffu : 0u;
-  const int xr = b_lo ? c : (b_hi ? c - M : 0);
-  const bf16x8_t* xrow = reinterpret_cast<const bf16x8_t*>(x + (size_t)xr * ldx) + (b_hi ? 4 : 0) + g;
   f32x4_t acc[RBW];
 #pragma unroll
   for (int r = 0; r < RBW; ++r) acc[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int pb = wave * U;
+  static_assert(NORM > 0 || NORM < -1, "halves take the RMSNorm prologue or staged activations");
   if constexpr (NORM > 0) {
-    (void)xrow;
-    (void)keep;
     accumulate_rows_rms_dense<NW, RBW, 2 * U, NORM, true>(acc, wt, x, ldx, reinterpret_cast<const bf16x8_t*>(norm_w),
                                                           M, KT, 2 * pb, wave, lane, eps);
     if (!reduce_waves_at<NW, RBW>(acc, wave, lane, rms_lds, rms_wave_bytes(2 * U, NORM, M, RBW))) return;
-  } else if constexpr (NORM < -1) {
-    (void)xrow;
-    (void)keep;
-    (void)norm_w;
-    (void)eps;
-    accumulate_rows_staged<NW, RBW, 2 * U, -1 - NORM, true>(acc, wt, x, ldx, M, KT, 2 * pb, wave, lane);
-    if (!reduce_waves_at<NW, RBW>(acc, wave, lane, rms_lds, staged_wave_bytes(2 * U, M, RBW))) return;
   } else {
     (void)norm_w;
     (void)eps;
-    bf16x8_t wv[U][RBW];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-#pragma unroll
-      for (int r = 0; r < RBW; ++r) wv[u][r] = load_weight_tile(wt + ((size_t)r * KT + 2 * (pb + u)) * 64);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bf16x8_t xv = load_x_frag(xrow + (pb + u) * 8, keep);
-#pragma unroll
-      for (int r = 0; r < RBW; ++r) acc[r] = mfma16(wv[u][r], xv, acc[r]);
-    }
-    if (!reduce_waves<NW, RBW>(acc, wave, lane)) return;
+    accumulate_rows_staged<NW, RBW, 2 * U, staged_chunks(NORM), true>(acc, wt, x, ldx, M, KT, 2 * pb, wave, lane);
+    if (!reduce_waves_at<NW, RBW>(acc, wave, lane, rms_lds, staged_wave_bytes(2 * U, M, RBW))) return;
   }
   const int partner = lane + 32 + M;  // only read where g < 2 and c < M (partner < 64)
 #pragma unroll
@@ -942,11 +899,10 @@ __global__ __launch_bounds__(NW * 64) void decode_half_kernel(
   }
 }
 
-template <int NW, int RBW, int EPI, int U, int NORM = 0>
+template <int NW, int RBW, int EPI, int U, int NORM>
 hipError_t launch_half_cfg(const DecodeArgs& a, hipStream_t stream) {
-  const size_t lds = NORM > 0    ? (size_t)NW * rms_wave_bytes(2 * U, NORM, a.M, RBW)
-                     : NORM < -1 ? (size_t)NW * staged_wave_bytes(2 * U, a.M, RBW)
-                                 : 0;
+  const size_t lds = NORM > 0 ? (size_t)NW * rms_wave_bytes(2 * U, NORM, a.M, RBW)
+                              : (size_t)NW * staged_wave_bytes(2 * U, a.M, RBW);
   launch_kernel(decode_half_kernel<NW, RBW, EPI, U, NORM>, dim3(a.NB / RBW * 2), dim3(NW * 64), lds, stream,
       static_cast<const bf16x8_t*>(a.w), static_cast<const __bf16*>(a.x), a.ldx, static_cast<__bf16*>(a.y), a.ldy,
       static_cast<const __bf16*>(a.residual), a.ldr, a.M, a.KT, static_cast<const __bf16*>(a.norm_w), a.eps);
@@ -984,10 +940,10 @@ hipError_t launch_staged(const DecodeArgs& a, int nc, hipStream_t stream) {
   }
 }
 
-// Shape dispatch: the Qwen3-4B K values get single-round instantiations
-// (K/32 = 80 -> 16 waves x 5 for QKV and the gate/up pairs, 128 -> 8 x 16,
-// 304 -> 16 x 19, each measured faster than the alternatives on MI355X); any
-// other K runs the round-based variant.
+// Shape dispatch: the Qwen3-4B K values get single-round instantiations with
+// staged activations (K/32 = 80, 128 -> 8 x 16, 304 -> 16 x 19, each measured
+// faster than the alternatives on MI355X); any other K runs the round-based
+// variant.
 template <int RBW, int EPI>
 hipError_t launch_decode_shape(const DecodeArgs& a, hipStream_t stream) {
   // K/32 = 80 at M <= 8 (QKV and gate_up, 36-layer step at M = 1):
@@ -1014,28 +970,18 @@ hipError_t launch_decode_shape(const DecodeArgs& a, hipStream_t stream) {
     // so the chunk registers fit beside the 19 weight tiles (8-10 chunks in
     // one phase spill): 13.7-14.3 -> 11.5-11.9 us per launch; at M = 5 the
     // single phase (6 chunks) is 0.3 us faster.
-    if (a.KT == 304 && a.M <= 6) return launch_decode_cfg<16, RBW, EPI, 19, staged_x2(4)>(a, stream);
-    if (a.KT == 304 && a.M <= 8) return launch_decode_cfg<16, RBW, EPI, 19, staged_x2(5)>(a, stream);
+    if (a.KT == 304 && a.M <= 6) return launch_decode_cfg<16, RBW, EPI, 19, staged_x(4, 2)>(a, stream);
+    if (a.KT == 304 && a.M <= 8) return launch_decode_cfg<16, RBW, EPI, 19, staged_x(5, 2)>(a, stream);
   }
-  if (a.KT == 80 && a.M <= 8) {
-    if constexpr (RBW == 1) return launch_half_cfg<8, RBW, EPI, 5>(a, stream);
-    if constexpr (RBW == 2) return launch_half_cfg<4, RBW, EPI, 10>(a, stream);
-  }
-  switch (a.KT) {
-    case 80:
-      // (M > 8) 16 waves x 5 k-tiles, for the single row-block (QKV) and the
-      // gate/up pair alike: measured 4.5 % / 3.2 % faster than 8 waves x 10 (whose
-      // gate/up form needs 96 VGPRs and leaves 96 of 608 workgroups for a
-      // second wave) and than the round-based loop.
-      return launch_decode_cfg<16, RBW, EPI, 5, 0>(a, stream);
-    case 128:
-      if constexpr (RBW == 1) return launch_decode_cfg<8, RBW, EPI, 16, 0>(a, stream);
-      break;
-    case 304:
-      if constexpr (RBW == 1) return launch_decode_cfg<16, RBW, EPI, 19, 0>(a, stream);
-      break;
-    default:
-      break;
+  // M = 9..16: staged in more phases, since 16 rows of a wave's slice beside
+  // its weight tiles take too many registers and too much LDS at once (us per
+  // launch at 12 rows, per-tile fragments before: QKV 9.5 -> 9.0, o_proj 8.0
+  // -> 6.6, down 16.2 -> 13.4, gate_up 22.3 -> 22.0; gate_up as 16 waves x 5
+  // k-tiles 22.3, down_proj in two phases spills).
+  if (a.KT == 80) return launch_decode_cfg<8, RBW, EPI, 10, staged_x(5, 2)>(a, stream);
+  if constexpr (RBW == 1) {
+    if (a.KT == 128) return launch_decode_cfg<8, RBW, EPI, 16, staged_x(8, 2)>(a, stream);
+    if (a.KT == 304) return launch_decode_cfg<16, RBW, EPI, 19, staged_x(5, 4)>(a, stream);
   }
   if (a.KT >= 256) return launch_decode_cfg<16, RBW, EPI, 0, 0>(a, stream);
   return launch_decode_cfg<8, RBW, EPI, 0, 0>(a, stream);
@@ -1150,7 +1096,10 @@ hipError_t launch_lm_head_argmax(const void* w, int V, int K, const void* x, int
   } else if (nw != nullptr) {
     return hipErrorInvalidValue;  // the fused RMSNorm serves K = 2560, M <= 8 (checked by the caller)
   } else if (KT == 80) {
-    launch_kernel(lm_head_kernel<kLmHeadWaves, kLmHeadRBW, 10>, dim3(P + M), dim3(kLmHeadWaves * 64), 0, stream,
+    // M = 9..16: staged in four phases (126.8 -> 122.7 us at 9 rows, 130.6 ->
+    // 124.9 at 12 against per-tile fragments; two phases 127.9 at 12).
+    const size_t lds = (size_t)kLmHeadWaves * staged_wave_bytes(10, M, kLmHeadRBW, 4);
+    launch_kernel(lm_head_kernel<kLmHeadWaves, kLmHeadRBW, 10, 3, false, 4>, dim3(P + M), dim3(kLmHeadWaves * 64), lds, stream,
         static_cast<const bf16x8_t*>(w), static_cast<const __bf16*>(x), ldx, logits, V, logits_bf16, partials, status, out_idx, M,
         KT, nullptr, 0.f);
   } else {

@@ -1,4 +1,4 @@
-// Projections of 17..128 rows on gfx950: y[M][N] = epilogue(x[M][K] . W[N][K]^T).
+// Projections of 17..128 rows (9..16 for a wide SiLU*up) on gfx950: y[M][N] = epilogue(x[M][K] . W[N][K]^T).
 //
 // At these row counts a projection is still bound by the bytes that each CU
 // pulls: the weights from HBM once (the arithmetic intensity is M FLOP per
@@ -366,6 +366,8 @@ template <int RBW, int EPI>
 hipError_t launch_rbw(const SkinnyPlan& p, const void* w, const void* x, int ldx, void* y, int ldy,
                       const void* residual, int ldr, int M, int NB, int KT, void* workspace, hipStream_t stream) {
   switch (skinny_groups(M)) {
+    case 1:
+      return launch_cfg<RBW, 1, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
     case 2:
       return launch_cfg<RBW, 2, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
     case 3:
@@ -438,8 +440,13 @@ int skinny_groups(int M) {
 // activation fragment once per 128 weight rows instead of once per 32 --
 // except with SiLU*up, where units of 8 outputs give every CU 80 weight rows
 // in one round (19456 x 2560 at 128 rows: 37 us, the GEMM 56 us).
+//
+// 9..16 rows with SiLU*up too when every CU gets four units or more (N >=
+// 16384; 19.7 us at 12 rows of 19456 x 2560, the decode kernel 22.0); there a
+// call has no workspace.
 bool skinny_route(int M, int N, int K, bool silu) {
-  if (M <= kDecodeMaxM || M > kSkinnyMaxM || N % kTileRows != 0 || K % kTileK != 0) return false;
+  if (M <= 8 || M > kSkinnyMaxM || N % kTileRows != 0 || K % kTileK != 0) return false;
+  if (M <= kDecodeMaxM) return silu && N >= 16384;
   const bool gemm_grid = N % kGemmBN == 0 && K % kGemmBK == 0;
   return M <= 64 || !gemm_grid || N < 8192 || silu;
 }

@@ -21,8 +21,8 @@ CASES = [  # (N, K, epilogue); the last three take five units per workgroup
 ]
 
 
-@pytest.mark.parametrize("n,k,epi", CASES)
-@pytest.mark.parametrize("m", [17, 33, 64, 81, 128])
+@pytest.mark.parametrize("m,n,k,epi", [(m, *c) for c in CASES for m in (17, 33, 64, 81, 128)]
+                         + [(m, n, k, 1) for m in (9, 16) for n, k in ((16384, 96), (16416, 64), (19456, 2560))])
 def test_skinny_edges(gpu, m, n, k, epi):
     layout = _lib.LAYOUT_MFMA16X32_GATEUP if epi == _lib.EPI_SILU_MUL else _lib.LAYOUT_MFMA16X32
     dev = torch.device("cuda:0")
