@@ -19,14 +19,22 @@
 //
 // Scores run on MFMA: 16 cache rows x 32 dims of K form the A operand
 // (one 16-byte load per lane, straight from the row-major cache) and the G
-// bf16 q heads, padded to 16 columns, the B operand.  P.V runs on the VALU,
-// each wave over its 16-row groups with lane l owning dims 2l, 2l+1, and the
-// waves' partial sums are added in wave order.  A context longer than one
-// chunk leaves each chunk's (max, sum, unnormalised P.V) in the workspace;
-// the workgroup that arrives last for kv head j combines the chunks in chunk
-// order and re-arms the head's counter.  Every sum has a fixed order, so
-// results are bitwise reproducible.  The new row is read from LDS, not back
-// from the cache it was just written to.
+// bf16 q heads, padded to 16 columns, the B operand.  Softmax weights and P.V
+// are fp32 on the VALU, each wave over its 16-row groups, weights through the
+// wave's own LDS; the waves' partial sums are added in wave order.  A context
+// longer than one chunk leaves each chunk's (max, sum, unnormalised P.V) in
+// the workspace; the workgroup that arrives last for kv head j combines the
+// chunks in chunk order and re-arms the head's counter.  Every sum has a fixed
+// order, so results are bitwise reproducible.  The new row is read from LDS,
+// not back from the cache it was just written to.
+//
+// Bound: latency up to some 4096 rows, then the cache bytes (67 MB at 16384
+// rows of 8 kv heads, 9.9 us at the chip's streaming rate) and the steps after
+// the last of them.  Cache rows by buffer loads without branches, half of V
+// after the scores, one barrier around the softmax instead of three, and the
+// combine in 16-byte loads and unrolled LDS reads: 5.77 -> 5.44 us at 128 rows,
+// 9.4 -> 9.1 at 1088, 14.2 -> 12.8 at 4096, 17.5 -> 15.1 at 8192, 24.2 -> 20.8
+// at 16384 (position read from the device, 36 launches per graph).
 
 #include <hip/hip_runtime.h>
 
@@ -74,63 +82,70 @@ __host__ __device__ constexpr unsigned partial_slot_bytes(int G) {
 }
 
 // The last workgroup of kv head j: M_h = max_c m_c and
-// out = sum_c e^(m_c - M) acc_c / sum_c e^(m_c - M) l_c, in chunk order.
-// Every partial value is requested in one round (NB * 8 chunk slots per
-// output; those past the last chunk load from outside the buffer's range,
-// which returns zero and moves no data, and get weight 0), together with the
-// (m, l) pairs, so the combine waits for memory once.
-template <int G, int NB>
+// out = sum_c e^(m_c - M) acc_c / sum_c e^(m_c - M) l_c.  The workgroup's
+// threads are up to 8 groups of 32 G; a group takes its share of up to MAX
+// chunks in chunk order, four values of them per thread (16-byte loads: the 66 KB of 32 chunks come
+// through one CU, and as single values they were four times the requests),
+// and the groups' sums are added in order.  Every partial is requested in one
+// round with the (m, l) pairs, those past the last chunk from outside the
+// buffer's range, which returns zero and moves no data; their weight is 0.
+template <int G, int MAX>
 __device__ __forceinline__ void combine_chunks(const AttnArgs& a, __amdgpu_buffer_rsrc_t parts, unsigned first,
                                                unsigned slot_bytes, int j, float (*mx)[G], float (*lsum)[G],
-                                               float (*wts)[G], float (*wl)[G]) {
-  constexpr int kOut = (G * kHeadDim + kThreads - 1) / kThreads;
-  constexpr int kSlots = NB * 8;
-  float v[kOut][kSlots];
-#pragma unroll
-  for (int o = 0; o < kOut; ++o) {
-    const int e = min((int)threadIdx.x + o * kThreads, G * kHeadDim - 1);
-#pragma unroll
-    for (int k = 0; k < kSlots; ++k) {
-      // Out of range goes in the vector offset: the range check covers the
-      // vector and instruction offsets, not the scalar one.
-      const bool real = k < a.chunks;
-      const unsigned voff = (real ? 0u : kOutOfRange) + (unsigned)(2 * G + e) * 4u;
-      const unsigned base = real ? first + (unsigned)k * slot_bytes : 0u;
-      v[o][k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(parts, voff, base, kCoherent));
-    }
-  }
-  // (m, l) of chunk k, head h, to thread kG + h; weights past the last
-  // chunk are 0.
+                                               float (*wts)[G], float* sums) {
+  constexpr int kQuads = G * kHeadDim / 4;
+  // As many groups as `sums`, the memory of the waves' sums, has rows.
+  constexpr int kGroups = kThreads / kQuads < kWaves ? kThreads / kQuads : kWaves;
+  constexpr int kSlots = MAX / kGroups;
+  const int quad = threadIdx.x % kQuads;
+  const int grp = threadIdx.x / kQuads;
+  // (m, l) of chunk k, head h, to thread kG + h.
   const int wk = threadIdx.x / G;
   const int wh = threadIdx.x - wk * G;
-  if (wk < a.chunks) {
-    const unsigned base = first + wk * slot_bytes;
-    mx[wk][wh] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(parts, (unsigned)wh * 4u, base,
-                                                                                  kCoherent));
-    lsum[wk][wh] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(parts, (unsigned)(G + wh) * 4u,
-                                                                                    base, kCoherent));
+  const unsigned wbase = wk < a.chunks ? first + wk * slot_bytes : 0u;
+  const unsigned wout = wk < a.chunks ? 0u : kOutOfRange;
+  const float cm = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(parts, wout + (unsigned)wh * 4u,
+                                                                                  wbase, kCoherent));
+  const float cl = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                 parts, wout + (unsigned)(G + wh) * 4u, wbase, kCoherent));
+  f32x4_t v[kSlots];
+#pragma unroll
+  for (int i = 0; i < kSlots; ++i) {
+    // Out of range goes in the vector offset: the range check covers the
+    // vector and instruction offsets, not the scalar one.
+    const int k = grp * kSlots + i;
+    const unsigned off = (k < a.chunks && grp < kGroups ? first + (unsigned)k * slot_bytes : kOutOfRange) + (unsigned)(2 * G + 4 * quad) * 4u;
+    v[i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(parts, off, 0, kCoherent));
+  }
+  if (wk < MAX) {
+    mx[wk][wh] = wk < a.chunks ? cm : -__builtin_huge_valf();
   }
   __syncthreads();
-  if (wk < kSlots) {
+  // (Over all chunk slots, so that the LDS reads are issued together: a loop
+  // over a.chunks pays an LDS access per chunk, 1.5 us of 32.)
+  if (wk < MAX) {
     float m = -__builtin_huge_valf();
-    for (int k = 0; k < a.chunks; ++k) m = fmaxf(m, mx[k][wh]);
-    const float w = wk < a.chunks ? expf(mx[wk][wh] - m) : 0.f;
+#pragma unroll
+    for (int k = 0; k < MAX; ++k) m = fmaxf(m, mx[k][wh]);
+    const float w = mx[wk][wh] != -__builtin_huge_valf() ? expf(mx[wk][wh] - m) : 0.f;
     wts[wk][wh] = w;
-    wl[wk][wh] = wk < a.chunks ? w * lsum[wk][wh] : 0.f;
+    lsum[wk][wh] = wk < a.chunks ? w * cl : 0.f;
   }
   __syncthreads();
+  f32x4_t num = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int o = 0; o < kOut; ++o) {
-    const int e = threadIdx.x + o * kThreads;
-    if (e >= G * kHeadDim) break;
+  for (int i = 0; i < kSlots; ++i)
+    num += wts[min(grp * kSlots + i, MAX - 1)][quad / (kHeadDim / 4)] * v[i];
+  if (grp < kGroups) *reinterpret_cast<f32x4_t*>(sums + grp * G * kHeadDim + 4 * quad) = num;
+  __syncthreads();
+  for (int e = threadIdx.x; e < G * kHeadDim; e += kThreads) {
     const int h = e / kHeadDim;
-    float num = 0.f, den = 0.f;
+    float s = sums[e], den = 0.f;
 #pragma unroll
-    for (int k = 0; k < kSlots; ++k) {
-      num += wts[k][h] * v[o][k];
-      den += wl[k][h];
-    }
-    a.out[(size_t)(j * G) * kHeadDim + e] = static_cast<__bf16>(num / den);
+    for (int q = 1; q < kGroups; ++q) s += sums[q * G * kHeadDim + e];
+#pragma unroll
+    for (int k = 0; k < MAX; ++k) den += lsum[k][h];
+    a.out[(size_t)(j * G) * kHeadDim + e] = static_cast<__bf16>(s / den);
   }
 }
 
@@ -151,7 +166,6 @@ template <int G, int NU, AttnMode MODE>
 __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs args) {
   static_assert(G >= 1 && G <= 16, "q heads per kv head are the MFMA B columns");
   constexpr int kGroups = NU;              // 16-row groups per wave
-  constexpr int kRows = 16 * kWaves * NU;  // rows per workgroup at most: 128 NU
   constexpr int kMaxChunks = kAttnMaxChunks;
   AttnArgs a = args;
   if constexpr (MODE == kDevicePos) {
@@ -161,7 +175,7 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
     a.cos += (size_t)pos * (kHeadDim / 2);
     a.sin += (size_t)pos * (kHeadDim / 2);
   }
-  // Rows per chunk (at most kRows: the launch picks NU for the largest chunk
+  // Rows per chunk (at most 16 kWaves NU: the launch picks NU for the largest chunk
   // it can meet) and the chunk count, as the host computes them.
   const int rows = attention_rows_per_chunk(a.pos + 1);
   a.chunks = (a.pos + rows) / rows;  // ceil((pos + 1) / rows)
@@ -184,13 +198,13 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
 
   __shared__ __align__(16) __bf16 qs[16][kHeadDim];     // rotated q heads; rows >= G are zero
   __shared__ __align__(16) __bf16 kv_new[2][kHeadDim];  // this token's rotated k and its v
-  __shared__ __align__(16) float sc[G][kRows];          // scores, then exp(s - m)
+  // A wave's softmax weights e^(s - m) of its group u, row 4i + g: [g][i][head]
+  __shared__ __align__(16) float pw[kWaves][kGroups][4][4][G];
   __shared__ __align__(16) float part[kWaves][G][kHeadDim];
-  __shared__ float stat[2][G];                          // chunk max, chunk sum
+  __shared__ float stat[2][kWaves][G];                  // each wave's max and sum
   __shared__ float cmax[kMaxChunks][G];                 // combine: chunk maxima m_c
-  __shared__ float lsum[kMaxChunks][G];                 // combine: chunk sums l_c
+  __shared__ float lsum[kMaxChunks][G];                 // combine: e^(m_c - M) l_c
   __shared__ float wts[kMaxChunks][G];                  // combine: e^(m_c - M)
-  __shared__ float wl[kMaxChunks][G];                   // combine: e^(m_c - M) l_c
   __shared__ int last;
 
   // ---- inputs of this wave's prologue items, loaded before the cache rows
@@ -200,30 +214,30 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   // read a q head again and store nothing): a load used only under a branch
   // may be sunk into it, behind the cache-row loads.  Lane l: dims l, l + 64.
   constexpr int kItems = (G + kWaves) / kWaves;  // ceil((G + 1) / kWaves)
-  float px0[kItems], px1[kItems], pw0[kItems], pw1[kItems];
+  __bf16 px0[kItems], px1[kItems], pw0[kItems], pw1[kItems];
 #pragma unroll
   for (int u = 0; u < kItems; ++u) {
     const int i = wave + kWaves * u;
     if constexpr (MODE == kGiven) {
       const __bf16* src = a.qkv + (size_t)(j * G + (i < G ? i : G - 1)) * kHeadDim;
-      px0[u] = static_cast<float>(src[lane]);
-      px1[u] = static_cast<float>(src[lane + 64]);
+      px0[u] = src[lane];
+      px1[u] = src[lane + 64];
       continue;
     }
     const bool is_k = i == G;
     const int src_head = is_k ? a.n_q + j : j * G + (i < G ? i : G - 1);
     const __bf16* src = a.qkv + (size_t)src_head * kHeadDim;
     const __bf16* nw = is_k ? a.k_norm_w : a.q_norm_w;
-    px0[u] = static_cast<float>(src[lane]);
-    px1[u] = static_cast<float>(src[lane + 64]);
-    pw0[u] = static_cast<float>(nw[lane]);
-    pw1[u] = static_cast<float>(nw[lane + 64]);
+    px0[u] = src[lane];
+    px1[u] = src[lane + 64];
+    pw0[u] = nw[lane];
+    pw1[u] = nw[lane + 64];
   }
-  float cs = 0.f, sn = 0.f;
+  __bf16 cs = __bf16(0.f), sn = __bf16(0.f);
   __bf16 v_new0 = __bf16(0.f), v_new1 = __bf16(0.f);
   if constexpr (MODE != kGiven) {
-    cs = static_cast<float>(a.cos[lane]);
-    sn = static_cast<float>(a.sin[lane]);
+    cs = a.cos[lane];
+    sn = a.sin[lane];
     const __bf16* vsrc = a.qkv + ((size_t)a.n_q + a.n_kv + j) * kHeadDim;
     v_new0 = vsrc[lane];
     v_new1 = vsrc[lane + 64];
@@ -234,28 +248,39 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   // fragments: group u, lane (g, c) = row lb(u) + c, dims 32kt + 8g .. +7.
   // V: lane (g, c) = dims 8c .. 8c+7 of rows lb(u) + 4i + g.  Row pos is this
   // token's (from LDS below); rows past it are not read.
-  const __bf16* kbase = a.k_cache + (size_t)j * a.kv_stride;
-  const __bf16* vbase = a.v_cache + (size_t)j * a.kv_stride;
+  // Buffer loads over the cached rows: a row past them, or past the chunk,
+  // lies beyond the buffer's range and reads as zero without a branch (with
+  // one, the compiler cannot count the loads in flight and the prologue waits
+  // for every row).  All K first, then V of the first half of the groups: a CU
+  // takes only some 60 KB of loads at a time, so a wave with more than that to
+  // issue gets to its prologue when the last one is accepted; the other half
+  // goes out after the scores, while the first is multiplied.
+  constexpr int kEarly = kGroups > 1 ? kGroups / 2 : 1;
+  const unsigned cached_bytes = (unsigned)cached * (kHeadDim * 2);
+  const __amdgpu_buffer_rsrc_t kbuf = __builtin_amdgcn_make_buffer_rsrc(
+      a.k_cache + (size_t)j * a.kv_stride, (short)0, (int)cached_bytes, (int)kRawBufferDword3);
+  const __amdgpu_buffer_rsrc_t vbuf = __builtin_amdgcn_make_buffer_rsrc(
+      a.v_cache + (size_t)j * a.kv_stride, (short)0, (int)cached_bytes, (int)kRawBufferDword3);
+  auto row_at = [&](int u, int r) {  // byte offset of row r of the wave's group u
+    return (lb(u) < rows ? 0u : kOutOfRange) + (unsigned)(row0 + lb(u) + r) * (kHeadDim * 2);
+  };
   bf16x8_t kf[kGroups][4];
   bf16x8_t vf[kGroups][4];
 #pragma unroll
-  for (int u = 0; u < kGroups; ++u) {
-    const int t = row0 + lb(u) + c;
+  for (int u = 0; u < kGroups; ++u)
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
-      bf16x8_t v = {};
-      if (t < cached && lb(u) < rows)
-        v = *reinterpret_cast<const bf16x8_t*>(kbase + (size_t)t * kHeadDim + 32 * kt + 8 * g);
-      kf[u][kt] = v;
-    }
+    for (int kt = 0; kt < 4; ++kt)
+      kf[u][kt] = __builtin_bit_cast(
+          bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(kbuf, row_at(u, c) + 64 * kt + 16 * g, 0, 0));
+  __builtin_amdgcn_sched_barrier(0);
+  auto load_v = [&](int u) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tv = row0 + lb(u) + 4 * i + g;
-      bf16x8_t v = {};
-      if (tv < cached && lb(u) < rows) v = *reinterpret_cast<const bf16x8_t*>(vbase + (size_t)tv * kHeadDim + 8 * c);
-      vf[u][i] = v;
-    }
-  }
+    for (int i = 0; i < 4; ++i)
+      vf[u][i] = __builtin_bit_cast(
+          bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(vbuf, row_at(u, 4 * i + g) + 16 * c, 0, 0));
+  };
+#pragma unroll
+  for (int u = 0; u < kEarly; ++u) load_v(u);
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- the prologue items: RMSNorm, RoPE; k and v appended to the caches.
@@ -264,16 +289,18 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
     const int i = wave + kWaves * u;
     if constexpr (MODE == kGiven) {
       if (i < G) {
-        qs[i][lane] = static_cast<__bf16>(px0[u]);
-        qs[i][lane + 64] = static_cast<__bf16>(px1[u]);
+        qs[i][lane] = px0[u];
+        qs[i][lane + 64] = px1[u];
       }
       continue;
     }
-    const float r = inv_rms(wave_sum(px0[u] * px0[u] + px1[u] * px1[u]), kHeadDim, a.eps);
-    const float n0 = bf16_round((px0[u] * r) * pw0[u]);
-    const float n1 = bf16_round((px1[u] * r) * pw1[u]);
-    const __bf16 o0 = rope_half(n0, n1, cs, sn, -1.f);
-    const __bf16 o1 = rope_half(n1, n0, cs, sn, 1.f);
+    const float x0 = static_cast<float>(px0[u]), x1 = static_cast<float>(px1[u]);
+    const float cf = static_cast<float>(cs), sf = static_cast<float>(sn);
+    const float r = inv_rms(wave_sum(x0 * x0 + x1 * x1), kHeadDim, a.eps);
+    const float n0 = bf16_round((x0 * r) * static_cast<float>(pw0[u]));
+    const float n1 = bf16_round((x1 * r) * static_cast<float>(pw1[u]));
+    const __bf16 o0 = rope_half(n0, n1, cf, sf, -1.f);
+    const __bf16 o1 = rope_half(n1, n0, cf, sf, 1.f);
     if (i < G) {
       qs[i][lane] = o0;
       qs[i][lane + 64] = o1;
@@ -293,73 +320,68 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   for (int e = threadIdx.x; e < (16 - G) * kHeadDim; e += kThreads) qs[G + e / kHeadDim][e % kHeadDim] = __bf16(0.f);
   __syncthreads();
 
-  // ---- this token's row pos, if it falls in one of this wave's groups.
-  // (Unrolled selects: a runtime index would put kf / vf in scratch memory.)
-  if (has_new) {
-    const bf16x8_t vn = *reinterpret_cast<const bf16x8_t*>(&kv_new[1][8 * c]);
-#pragma unroll
-    for (int u = 0; u < kGroups; ++u) {
-      const int d = a.pos - row0 - lb(u);
-      if (d < 0 || d >= 16) continue;
-      if (c == d) {
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) kf[u][kt] = *reinterpret_cast<const bf16x8_t*>(&kv_new[0][32 * kt + 8 * g]);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (d == 4 * i + g) vf[u][i] = vn;
-    }
-  }
-
   // ---- scores: output lane (g, c) holds rows lb(u) + 4g .. +3 of head c.
+  // This token's row pos, if it falls in one of the wave's groups, comes from
+  // LDS.  (Unrolled selects: a runtime index would put kf / vf in scratch
+  // memory.)
+  const float kNegInf = -__builtin_huge_valf();
+  const int n = min(rows, L - row0);  // filled rows of the chunk
   bf16x8_t qf[4];
 #pragma unroll
   for (int kt = 0; kt < 4; ++kt) qf[kt] = *reinterpret_cast<const bf16x8_t*>(&qs[c][32 * kt + 8 * g]);
+  f32x4_t sv[kGroups];
+  float mx = kNegInf;
 #pragma unroll
   for (int u = 0; u < kGroups; ++u) {
-    if (lb(u) >= rows || row0 + lb(u) >= L) break;
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    sv[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (lb(u) >= n) continue;
+    if (has_new && c == a.pos - row0 - lb(u)) {
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[u][kt], qf[kt], acc, 0, 0, 0);
-    if (c < G) {
+      for (int kt = 0; kt < 4; ++kt) kf[u][kt] = *reinterpret_cast<const bf16x8_t*>(&kv_new[0][32 * kt + 8 * g]);
+    }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sc[c][lb(u) + 4 * g + i] = acc[i] * a.scale;
+    for (int kt = 0; kt < 4; ++kt) sv[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[u][kt], qf[kt], sv[u], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      sv[u][i] *= a.scale;
+      if (lb(u) + 4 * g + i < n) mx = fmaxf(mx, sv[u][i]);
     }
   }
-  __syncthreads();
 
-  // ---- chunk softmax state per head over its filled rows n (up to
-  // kRows / 64 per lane, summed in row order within a lane, then across
-  // lanes); the rows past the last are never read again.
-  const int n = min(rows, L - row0);
-  for (int h = wave; h < G; h += kWaves) {
-    float sv[kRows / 64];
-    float mx = -__builtin_huge_valf();
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < kRows / 64; ++u) {
-      if (64 * u >= n) break;
-      sv[u] = lane + 64 * u < n ? sc[h][lane + 64 * u] : -__builtin_huge_valf();
-      mx = fmaxf(mx, sv[u]);
-    }
-    const float m = wave_max(mx);
-    float sum = 0.f;
+  for (int u = kEarly; u < kGroups; ++u) load_v(u);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- the chunk's maximum m per head, the weights e^(s - m) (to the wave's
+  // own LDS, no barrier) and each wave's sum of them.  Rows that score -inf
+  // weigh nothing, also in a chunk without others (m = -inf; a NaN beside them
+  // stays NaN); a context of such rows alone gives 0 / 0 in the end, as
+  // torch's softmax.
+  mx = fmaxf(mx, __shfl_xor(mx, 16));
+  mx = fmaxf(mx, __shfl_xor(mx, 32));
+  if (g == 0 && c < G) stat[0][wave][c] = mx;
+  __syncthreads();
+  float m = kNegInf;
 #pragma unroll
-    for (int u = 0; u < kRows / 64; ++u) {
-      if (64 * u >= n) break;
-      // A chunk of -inf scores only has weight 0 beside other chunks (given
-      // rows may hold any values), not the NaN of -inf - -inf.
-      const bool live = lane + 64 * u < n && !(MODE == kGiven && m == -__builtin_huge_valf());
-      const float e = live ? expf(sv[u] - m) : 0.f;
-      sc[h][lane + 64 * u] = e;
+  for (int w = 0; w < kWaves; ++w) m = fmaxf(m, stat[0][w][c < G ? c : 0]);
+  float sum = 0.f;
+#pragma unroll
+  for (int u = 0; u < kGroups; ++u) {
+    if (lb(u) >= n) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool live = lb(u) + 4 * g + i < n && sv[u][i] != kNegInf;
+      const float e = live ? expf(sv[u][i] - m) : 0.f;
       sum += e;
-    }
-    const float l = wave_sum(sum);
-    if (lane == 0) {
-      stat[0][h] = m;
-      stat[1][h] = l;
+      // P.V lane (g', c') takes rows 4i' + g' of every head: row 4g + i is
+      // i' = g, g' = i.
+      if (c < G) pw[wave][u][i][g][c] = e;
     }
   }
-  __syncthreads();
+  sum += __shfl_xor(sum, 16);
+  sum += __shfl_xor(sum, 32);
+  if (g == 0 && c < G) stat[1][wave][c] = sum;
 
   // ---- P.V over this wave's groups: lane (g, c) sums rows lb(u) + 4i + g
   // for dims 8c .. 8c+7, then the four row phases g are added as
@@ -373,17 +395,24 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
     for (int e = 0; e < 8; ++e) acc8[h][e] = 0.f;
 #pragma unroll
   for (int u = 0; u < kGroups; ++u) {
-    if (lb(u) >= rows || row0 + lb(u) >= L) break;
+    if (lb(u) >= n) continue;
+    float pr[4][G];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tl = lb(u) + 4 * i + g;  // row within the chunk
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int h = 0; h < G; ++h) {
-        const float pr = sc[h][tl];
+      for (int h = 0; h < G; ++h) pr[i][h] = pw[wave][u][g][i][h];
+    if (has_new) {
+      const int d = a.pos - row0 - lb(u);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc8[h][e] += pr * static_cast<float>(vf[u][i][e]);
-      }
+      for (int i = 0; i < 4; ++i)
+        if (d == 4 * i + g) vf[u][i] = *reinterpret_cast<const bf16x8_t*>(&kv_new[1][8 * c]);
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int h = 0; h < G; ++h)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc8[h][e] += pr[i][h] * static_cast<float>(vf[u][i][e]);
   }
   constexpr int kHalf = 4 * G;  // of the 8G values (flat index q = 8h + e)
   const bool odd = g & 1, high = g >> 1;
@@ -405,14 +434,26 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   for (int q = 0; q < kHalf / 2; ++q) part[wave][(q0 + q) / 8][8 * c + (q0 + q) % 8] = quarter[q];
   __syncthreads();
 
+  // Sums over the waves, in wave order: the chunk's P.V of head h, dim d, and
+  // its sum of weights.
+  auto chunk_sum = [&](int h, int d) {
+    float s = part[0][h][d];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) s += part[w][h][d];
+    return s;
+  };
+  auto weight_sum = [&](int h) {
+    float l = stat[1][0][h];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) l += stat[1][w][h];
+    return l;
+  };
+
   if (a.chunks == 1) {
     for (int e = threadIdx.x; e < G * kHeadDim; e += kThreads) {
       const int h = e / kHeadDim;
       const int d = e - h * kHeadDim;
-      float s = part[0][h][d];
-#pragma unroll
-      for (int w = 1; w < kWaves; ++w) s += part[w][h][d];
-      a.out[(size_t)(j * G + h) * kHeadDim + d] = static_cast<__bf16>(s / stat[1][h]);
+      a.out[(size_t)(j * G + h) * kHeadDim + d] = static_cast<__bf16>(chunk_sum(h, d) / weight_sum(h));
     }
     return;
   }
@@ -428,15 +469,14 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   for (int e = threadIdx.x; e < G * kHeadDim; e += kThreads) {
     const int h = e / kHeadDim;
     const int d = e - h * kHeadDim;
-    float s = part[0][h][d];
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) s += part[w][h][d];
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s), parts, (unsigned)(2 * G + e) * 4u, slot,
-                                          kCoherent);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, chunk_sum(h, d)), parts,
+                                          (unsigned)(2 * G + e) * 4u, slot, kCoherent);
   }
-  if (threadIdx.x < 2 * G) {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, stat[threadIdx.x / G][threadIdx.x % G]), parts,
-                                          threadIdx.x * 4u, slot, kCoherent);
+  // Lanes c < G of every wave hold the chunk's maximum of head c.
+  if (threadIdx.x < G) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, m), parts, threadIdx.x * 4u, slot, kCoherent);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, weight_sum(threadIdx.x)), parts,
+                                          (unsigned)(G + threadIdx.x) * 4u, slot, kCoherent);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -448,15 +488,12 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   if (!last) return;
 
   const unsigned first = (unsigned)(j * a.chunks) * slot_bytes;
-  if (a.chunks <= 8) {
-    combine_chunks<G, 1>(a, parts, first, slot_bytes, j, cmax, lsum, wts, wl);
-  } else if (a.chunks <= 16) {
-    combine_chunks<G, 2>(a, parts, first, slot_bytes, j, cmax, lsum, wts, wl);
-  } else if (a.chunks <= 24) {
-    combine_chunks<G, 3>(a, parts, first, slot_bytes, j, cmax, lsum, wts, wl);
-  } else {
-    combine_chunks<G, 4>(a, parts, first, slot_bytes, j, cmax, lsum, wts, wl);
-  }
+  // (The waves' sums in `part` have been published: its memory takes the
+  // groups' sums.)
+  if (a.chunks <= 8)
+    combine_chunks<G, 8>(a, parts, first, slot_bytes, j, cmax, lsum, wts, &part[0][0][0]);
+  else
+    combine_chunks<G, kMaxChunks>(a, parts, first, slot_bytes, j, cmax, lsum, wts, &part[0][0][0]);
   if (threadIdx.x == 0) __hip_atomic_store(a.counters + j, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
