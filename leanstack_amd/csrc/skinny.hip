@@ -16,7 +16,7 @@
 // 16 bytes of it another cache access), they cost four times the accesses and
 // the weights waited behind them.  17.5 / 14.0 / 45.0 / 24.5 -> 12.9 / 10.8 /
 // 24.8 / 17.6 us for QKV / o / gate_up + SiLU*up / down at 64 rows, 32 / 24 /
-// 56 / 42 -> 18.5 / 15.4 / 37 / 25 at 128; per CU about 33 bytes/ns of weights
+// 56 / 42 -> 18.5 / 15.4 / 32.6 / 25 at 128; per CU about 33 bytes/ns of weights
 // and activations together, against 27 of weights alone in the decode kernels.
 //
 // When the row-blocks alone would leave CUs idle (kv/o/down-sized N), the call's
@@ -115,7 +115,13 @@ struct Shape {
   static constexpr int kSlot = kLoads * 1024;
   static constexpr int kFit = kLdsBytes / (kNW * kSlot);
   static constexpr int kDepth = kFit < 1 ? 1 : kFit > 4 ? 4 : kFit;  // steps in flight per wave
-  static constexpr int kRing = kNW * kDepth * kSlot;
+  // Where only one step fits (RBW 5 from 6 token groups), the weights of the
+  // step after it still fit beside it, and they are what comes from HBM: a
+  // wave then waits for activations from L2 alone (19456 x 2560 with SiLU*up:
+  // 36.0 -> 32.6 us at 128 rows, 29.5 -> 28.8 at 96).
+  static constexpr bool kAhead = kDepth == 1 && kNW * (kSlot + 2 * RBW * 1024) <= kLdsBytes;
+  static constexpr int kWaveRing = kDepth * kSlot + (kAhead ? 2 * RBW * 1024 : 0);
+  static constexpr int kRing = kNW * kWaveRing;
   // Row-blocks whose partial tiles of all waves fit the ring at once.
   static constexpr int kSumRows = kRing / (kNW * MG * 1024) < RBW ? kRing / (kNW * MG * 1024) : RBW;
   static_assert(kFit >= 1 && kSumRows >= 1, "one step per wave fits the LDS");
@@ -170,9 +176,12 @@ __global__ __launch_bounds__(kNW * 64) void skinny_kernel(
 #pragma unroll
   for (int i = 0; i < 2 * MG; ++i) xrow[i] = (unsigned)min(8 * i + xr, M - 1) * ldx * 2u;
   const unsigned ring0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)ring +
-                         wave * D * Sh::kSlot;
+                         wave * Sh::kWaveRing;
 
-  auto issue = [&](int step, int slot) {
+  // A wave's ring: D slots of weights, then activations; kAhead: one slot of
+  // activations between two of weights.
+  constexpr unsigned kXSlot = Sh::kAhead ? 0 : Sh::kSlot;
+  auto issue_w = [&](int step, int slot) {
     const int u = ub + wave + kNW * step;
     const bool half = 2 * u + 1 >= KT;  // odd KT: the last step has one k-tile
     const unsigned lds = ring0 + slot * Sh::kSlot;
@@ -181,11 +190,16 @@ __global__ __launch_bounds__(kNW * 64) void skinny_kernel(
 #pragma unroll
       for (int h = 0; h < 2; ++h)
         dma_1k<true>(wrsrc, wvoff[r], (unsigned)(2 * u + (half ? 0 : h)) * 1024u, lds + (2 * r + h) * 1024);
+  };
+  auto issue_x = [&](int step, int slot) {
+    const int u = ub + wave + kNW * step;
+    const bool half = 2 * u + 1 >= KT;
+    const unsigned lds = ring0 + 2 * RBW * 1024 + slot * kXSlot;
 #pragma unroll
     for (int i = 0; i < 2 * MG; ++i) {
       int c = (lane & 7) ^ (((i & 1) << 2) | (xr >> 1));
       if (half) c &= 3;
-      dma_1k<false>(xrsrc, xrow[i] + c * 16u, (unsigned)u * 128u, lds + (2 * RBW + i) * 1024);
+      dma_1k<false>(xrsrc, xrow[i] + c * 16u, (unsigned)u * 128u, lds + i * 1024);
     }
   };
 
@@ -197,11 +211,19 @@ __global__ __launch_bounds__(kNW * 64) void skinny_kernel(
 
 #pragma unroll
   for (int d = 0; d < D; ++d)
-    if (d < n) issue(d, d);
+    if (d < n) {
+      issue_w(d, d);
+      issue_x(d, d);
+    }
+  if (Sh::kAhead && n > 1) issue_w(1, 1);
   int slot = 0;
   for (int i = 0; i < n; ++i) {
-    wait_steps<Sh::kLoads, D>(min(D - 1, n - 1 - i));
-    const unsigned char* buf = ring + (wave * D + slot) * Sh::kSlot;
+    if constexpr (Sh::kAhead)
+      wait_steps<2 * RBW, 2>(min(1, n - 1 - i));  // all but the next step's weights
+    else
+      wait_steps<Sh::kLoads, D>(min(D - 1, n - 1 - i));
+    const unsigned char* buf = ring + wave * Sh::kWaveRing + slot * Sh::kSlot;
+    const unsigned char* xbuf = ring + wave * Sh::kWaveRing + 2 * RBW * 1024 + slot * kXSlot;
     bf16x8_t wv[2][RBW], xv[2][MG];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -209,12 +231,17 @@ __global__ __launch_bounds__(kNW * 64) void skinny_kernel(
       for (int r = 0; r < RBW; ++r) wv[h][r] = *reinterpret_cast<const bf16x8_t*>(buf + (2 * r + h) * 1024 + lane * 16);
 #pragma unroll
       for (int q = 0; q < MG; ++q)
-        xv[h][q] = *reinterpret_cast<const bf16x8_t*>(buf + 2 * RBW * 1024 + (16 * q + m) * 128 +
-                                                      (((4 * h + g) ^ (m >> 1)) << 4));
+        xv[h][q] = *reinterpret_cast<const bf16x8_t*>(xbuf + (16 * q + m) * 128 + (((4 * h + g) ^ (m >> 1)) << 4));
     }
     // The slot's values are in registers before its next loads may land.
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (i + D < n) issue(i + D, slot);
+    if constexpr (Sh::kAhead) {
+      if (i + 1 < n) issue_x(i + 1, 0);
+      if (i + 2 < n) issue_w(i + 2, slot);
+    } else if (i + D < n) {
+      issue_w(i + D, slot);
+      issue_x(i + D, slot);
+    }
     const bool half = 2 * (ub + wave + kNW * i) + 1 >= KT;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -224,7 +251,7 @@ __global__ __launch_bounds__(kNW * 64) void skinny_kernel(
 #pragma unroll
         for (int q = 0; q < MG; ++q) acc[r][q] = mfma16(wv[h][r], xv[h][q], acc[r][q]);
     }
-    slot = slot + 1 == D ? 0 : slot + 1;
+    slot = slot + 1 == (Sh::kAhead ? 2 : D) ? 0 : slot + 1;
   }
 
   // Cross-wave sum in wave order through the drained ring, kSumRows row-blocks
@@ -439,7 +466,7 @@ int skinny_groups(int M) {
 // the 128 x 128 GEMM's grid, whose blocks then fill the chip and read each
 // activation fragment once per 128 weight rows instead of once per 32 --
 // except with SiLU*up, where units of 8 outputs give every CU 80 weight rows
-// in one round (19456 x 2560 at 128 rows: 37 us, the GEMM 56 us).
+// in one round (19456 x 2560 at 128 rows: 32.6 us, the GEMM 56 us).
 //
 // 9..16 rows with SiLU*up too when every CU gets four units or more (N >=
 // 16384; 19.7 us at 12 rows of 19456 x 2560, the decode kernel 22.0); there a

@@ -15,9 +15,10 @@ from tests.helpers import activations, assert_parity, weight
 
 pytestmark = pytest.mark.gpu
 
-CASES = [  # (N, K, epilogue); the last three take five units per workgroup
+CASES = [  # (N, K, epilogue); the last four take five units per workgroup
     (16, 32, 0), (48, 64, 0), (2560, 96, 2), (16, 2560, 2), (80, 544, 0), (4096, 1056, 0), (32, 32, 1), (96, 160, 1),
     (2592, 608, 1), (16416, 96, 1), (19456, 288, 1), (20512, 64, 1),
+    (16416, 800, 1),
 ]
 
 
