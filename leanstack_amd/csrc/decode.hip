@@ -1073,8 +1073,8 @@ hipError_t launch_lm_head_argmax(const void* w, int V, int K, const void* x, int
           KT, nullptr, 0.f);
     }
   };
-  // K/32 = 80: 8 waves x 10 k-tiles; for M <= 8 the activations are staged
-  // through LDS (the wave's 40 M chunks over 64 lanes).
+  // K/32 = 80: 8 waves x 10 k-tiles; the activations are staged through LDS
+  // (the wave's 40 M chunks over 64 lanes), for M > 8 in four phases.
   if (KT == 80 && M <= 8) {
     switch ((40 * M + 63) / 64) {
       case 1:

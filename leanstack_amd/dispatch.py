@@ -3,10 +3,11 @@
 leanstack's semantic runtime calls these module-level names once per layer
 per step (src/leanstack/runtime/qwen_explicit.py:963-971, call sites :1117,
 :1155, :1170, :1235, :1264, :1293).  Here every projection inside them runs
-on the gfx950 kernels through the C ABI; the work around the projections
-that is not part of this path (RMSNorm, q/k norm, RoPE, attention) stays
-torch code with the reference's semantics (attention is computed explicitly
-in fp32 with contiguous operands, see _sdpa).  The weight arguments are PackedWeight objects
+on the gfx950 kernels through the C ABI, and so does the row work between
+them (RMSNorm, q/k norm and RoPE, attention of one query row) for plain eager
+bfloat16 calls (_plain_eager); any other call of it, and attention over
+several query rows (in fp32 with contiguous operands, see _sdpa), is torch
+code with the reference's semantics.  The weight arguments are PackedWeight objects
 from the resident arena (leanstack_amd.leanserve) instead of row-major
 tensors; a row-major tensor is rejected with ValueError.
 
