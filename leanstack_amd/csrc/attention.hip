@@ -30,11 +30,11 @@
 //
 // Bound: latency up to some 4096 rows, then the cache bytes (67 MB at 16384
 // rows of 8 kv heads, 9.9 us at the chip's streaming rate) and the steps after
-// the last of them.  Cache rows by buffer loads without branches, half of V
+// the last of them.  Cache rows by counted buffer loads, half of V
 // after the scores, one barrier around the softmax instead of three, and the
-// combine in 16-byte loads and unrolled LDS reads: 5.8 -> 5.7 us at 128 rows,
-// 9.2 -> 9.1 at 1088, 14.1 -> 12.9 at 4000, 24.1 -> 21.0 at 16384 (position
-// read from the device, 36 launches per graph).
+// combine in 16-byte loads and unrolled LDS reads: 5.77 -> 5.44 us at 128 rows,
+// 9.4 -> 9.1 at 1088, 14.2 -> 12.8 at 4096, 17.5 -> 15.1 at 8192, 24.2 -> 20.8
+// at 16384 (position read from the device, 36 launches per graph).
 
 #include <hip/hip_runtime.h>
 
@@ -267,7 +267,25 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   };
   bf16x8_t kf[kGroups][4];
   bf16x8_t vf[kGroups][4];
-  auto load_k = [&]() {
+  auto load_v = [&](int u) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      vf[u][i] = __builtin_bit_cast(
+          bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(vbuf, row_at(u, 4 * i + g) + 16 * c, 0, 0));
+  };
+  // A wave without rows loads none: its loads beyond the range move no data,
+  // but go through the CU's address path in front of other waves' inputs.  The
+  // inputs are waited for first: past the branch the compiler could not tell
+  // them from the rows in flight and would wait for all.  The other side
+  // defines the row registers in place (they are not used there), or each would
+  // be copied, behind a wait, at the join.  Without / with the branch: 4.54 /
+  // 4.35 us at 11 rows of a 576-row cache, 7.40 / 7.22 at 300, 9.05 / 9.15 at
+  // 1088, 12.5 / 12.6 at 4001, 20.65 / 20.85 at 16384, 6.2 / 5.25 at one row of
+  // a 16384-row cache.  A second copy of the prologue, or of the kernel, for
+  // waves with rows instead: as fast on its own, 0.2 us slower between other
+  // kernels (instruction fetch).
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  if (16 * __builtin_amdgcn_readfirstlane(wave) < n) {
 #pragma unroll
     for (int u = 0; u < kGroups; ++u)
 #pragma unroll
@@ -275,65 +293,52 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
         kf[u][kt] = __builtin_bit_cast(
             bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(kbuf, row_at(u, c) + 64 * kt + 16 * g, 0, 0));
     __builtin_amdgcn_sched_barrier(0);
-  };
-  auto load_v = [&](int u) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      vf[u][i] = __builtin_bit_cast(
-          bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(vbuf, row_at(u, 4 * i + g) + 16 * c, 0, 0));
-  };
-  // ---- the prologue items: RMSNorm, RoPE; k and v appended to the caches.
-  auto prologue = [&]() {
-#pragma unroll
-    for (int u = 0; u < kItems; ++u) {
-      const int i = wave + kWaves * u;
-      if constexpr (MODE == kGiven) {
-        if (i < G) {
-          qs[i][lane] = px0[u];
-          qs[i][lane + 64] = px1[u];
-        }
-        continue;
-      }
-      const float x0 = static_cast<float>(px0[u]), x1 = static_cast<float>(px1[u]);
-      const float cf = static_cast<float>(cs), sf = static_cast<float>(sn);
-      const float r = inv_rms(wave_sum(x0 * x0 + x1 * x1), kHeadDim, a.eps);
-      const float n0 = bf16_round((x0 * r) * static_cast<float>(pw0[u]));
-      const float n1 = bf16_round((x1 * r) * static_cast<float>(pw1[u]));
-      const __bf16 o0 = rope_half(n0, n1, cf, sf, -1.f);
-      const __bf16 o1 = rope_half(n1, n0, cf, sf, 1.f);
-      if (i < G) {
-        qs[i][lane] = o0;
-        qs[i][lane + 64] = o1;
-      } else if (i == G && has_new) {
-        kv_new[0][lane] = o0;
-        kv_new[0][lane + 64] = o1;
-        kv_new[1][lane] = v_new0;
-        kv_new[1][lane + 64] = v_new1;
-        __bf16* kc = a.k_cache + (size_t)j * a.kv_stride + (size_t)a.pos * kHeadDim;
-        __bf16* vc = a.v_cache + (size_t)j * a.kv_stride + (size_t)a.pos * kHeadDim;
-        kc[lane] = o0;
-        kc[lane + 64] = o1;
-        vc[lane] = v_new0;
-        vc[lane + 64] = v_new1;
-      }
-    }
-  };
-  // A wave without rows loads none: its loads beyond the range move no data,
-  // but go through the CU's address path in front of other waves' inputs.  Each
-  // side has its own prologue: after a join, the waits for its inputs would
-  // have to count the loads of either side, and wait for every row.  With the
-  // branch 11 rows of a 576-row cache take 4.3 us (4.5 without), 300 rows 7.2
-  // (7.4), one row of a 16384-row cache 5.3 (6.2); full chunks pay for the
-  // second copy: 9.05 -> 9.12 at 1088 rows, 12.4 -> 12.7 at 4001, 20.7 -> 21.0
-  // at 16384.
-  if (16 * __builtin_amdgcn_readfirstlane(wave) < n) {
-    load_k();
 #pragma unroll
     for (int u = 0; u < kEarly; ++u) load_v(u);
-    __builtin_amdgcn_sched_barrier(0);
-    prologue();
   } else {
-    prologue();
+#pragma unroll
+    for (int u = 0; u < kGroups; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        asm volatile("" : "=v"(kf[u][i]));
+        if (u < kEarly) asm volatile("" : "=v"(vf[u][i]));
+      }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- the prologue items: RMSNorm, RoPE; k and v appended to the caches.
+#pragma unroll
+  for (int u = 0; u < kItems; ++u) {
+    const int i = wave + kWaves * u;
+    if constexpr (MODE == kGiven) {
+      if (i < G) {
+        qs[i][lane] = px0[u];
+        qs[i][lane + 64] = px1[u];
+      }
+      continue;
+    }
+    const float x0 = static_cast<float>(px0[u]), x1 = static_cast<float>(px1[u]);
+    const float cf = static_cast<float>(cs), sf = static_cast<float>(sn);
+    const float r = inv_rms(wave_sum(x0 * x0 + x1 * x1), kHeadDim, a.eps);
+    const float n0 = bf16_round((x0 * r) * static_cast<float>(pw0[u]));
+    const float n1 = bf16_round((x1 * r) * static_cast<float>(pw1[u]));
+    const __bf16 o0 = rope_half(n0, n1, cf, sf, -1.f);
+    const __bf16 o1 = rope_half(n1, n0, cf, sf, 1.f);
+    if (i < G) {
+      qs[i][lane] = o0;
+      qs[i][lane + 64] = o1;
+    } else if (i == G && has_new) {
+      kv_new[0][lane] = o0;
+      kv_new[0][lane + 64] = o1;
+      kv_new[1][lane] = v_new0;
+      kv_new[1][lane + 64] = v_new1;
+      __bf16* kc = a.k_cache + (size_t)j * a.kv_stride + (size_t)a.pos * kHeadDim;
+      __bf16* vc = a.v_cache + (size_t)j * a.kv_stride + (size_t)a.pos * kHeadDim;
+      kc[lane] = o0;
+      kc[lane + 64] = o1;
+      vc[lane] = v_new0;
+      vc[lane + 64] = v_new1;
+    }
   }
   for (int e = threadIdx.x; e < (16 - G) * kHeadDim; e += kThreads) qs[G + e / kHeadDim][e % kHeadDim] = __bf16(0.f);
   __syncthreads();
