@@ -32,9 +32,9 @@
 // rows of 8 kv heads, 9.9 us at the chip's streaming rate) and the steps after
 // the last of them.  Cache rows by counted buffer loads, half of V
 // after the scores, one barrier around the softmax instead of three, and the
-// combine in 16-byte loads and unrolled LDS reads: 5.77 -> 5.44 us at 128 rows,
-// 9.4 -> 9.1 at 1088, 14.2 -> 12.8 at 4096, 17.5 -> 15.1 at 8192, 24.2 -> 20.8
-// at 16384 (position read from the device, 36 launches per graph).
+// combine in 16-byte loads and unrolled LDS reads: 5.9 -> 5.7 us at 128 rows,
+// 9.2 -> 9.15 at 1088, 14.1 -> 12.6 at 4001, 24.1 -> 20.85 at 16384 (position
+// read from the device, 36 launches per graph).
 
 #include <hip/hip_runtime.h>
 
