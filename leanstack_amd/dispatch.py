@@ -62,12 +62,17 @@ def _plain_eager(*tensors: torch.Tensor) -> bool:
     return True
 
 
+def _rmsnorm_kernel_serves(hidden_states: torch.Tensor, weight: torch.Tensor, eps: float) -> bool:
+    """Whether the row kernel computes F.rms_norm over the last dim for these arguments."""
+    k = hidden_states.shape[-1]
+    return (k % 512 == 0 and 0 < k <= kernels.RMSNORM_MAX_K and weight.shape == (k,) and isinstance(eps, float)
+            and 0.0 <= eps < math.inf and _plain_eager(hidden_states, weight) and hidden_states.is_contiguous()
+            and weight.is_contiguous())
+
+
 def qwen_rmsnorm(hidden_states: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """F.rms_norm over the last dim (qwen_explicit.py:621-628)."""
-    k = hidden_states.shape[-1]
-    if (k % 512 == 0 and 0 < k <= kernels.RMSNORM_MAX_K and weight.shape == (k,) and isinstance(eps, float)
-            and 0.0 <= eps < math.inf and _plain_eager(hidden_states, weight) and hidden_states.is_contiguous()
-            and weight.is_contiguous()):
+    if _rmsnorm_kernel_serves(hidden_states, weight, eps):
         return kernels._rmsnorm_rows(hidden_states, weight, eps)
     return F.rms_norm(hidden_states, normalized_shape=(hidden_states.shape[-1],), weight=weight, eps=eps)
 
@@ -148,8 +153,12 @@ def _norm_gate_up(hidden_states, norm_weight, eps, gu_w: PackedWeight):
     """SiLU(gate)*up of rms_norm(hidden_states): fused into the gate_up kernel
     for up to 8 rows, a norm kernel in front of it for more (at 12 rows 3.3 +
     19.7 us, fused 25.2: the norm's arithmetic on 16 rows in every workgroup
-    no longer hides behind the weights)."""
-    if hidden_states.numel() // gu_w.k <= _FUSED_NORM_ROWS:
+    no longer hides behind the weights).  9..16 rows that the norm kernel does
+    not serve (a [1, K] norm weight, autocast) stay fused: rmsnorm_linear takes
+    every form that it takes for fewer rows, F.rms_norm does not."""
+    rows = hidden_states.numel() // gu_w.k
+    if rows <= _FUSED_NORM_ROWS or (rows <= _lib.DECODE_MAX_M
+                                    and not _rmsnorm_kernel_serves(hidden_states, norm_weight, eps)):
         return kernels.rmsnorm_linear(hidden_states, norm_weight, eps, gu_w, epilogue=_lib.EPI_SILU_MUL)
     return kernels.linear(qwen_rmsnorm(hidden_states, norm_weight, eps), gu_w, epilogue=_lib.EPI_SILU_MUL)
 

@@ -1,0 +1,43 @@
+"""The MLP names at 9..16 rows: every norm weight form and surrounding that up
+to 8 rows take, against the oracle."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import oracle.projections as ref
+from leanstack_amd import _lib, dispatch
+from leanstack_amd.geometry import QWEN3_4B as G
+from leanstack_amd.layout import PackedWeight
+from tests.helpers import activations, assert_parity, seeded_normal, weight
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+EPS = G.rms_norm_eps
+K = G.hidden_size
+
+
+def _mlp(rows: int, inter: int):
+    """A gate_up / down pair over `rows` rows, and the oracle's result."""
+    wgu, wd = weight(2 * inter, K, seed=inter), weight(K, inter, seed=inter + 1)
+    h, nw = activations(rows, K, seed=rows), seeded_normal((K,), 0.2, 3) + 1
+    expect = h + ref.linear(ref.silu_mul(ref.linear(ref.rmsnorm(h, nw, EPS), wgu), inter), wd)
+    gu = PackedWeight.from_rowmajor(wgu.to(DEV), _lib.LAYOUT_MFMA16X32_GATEUP)
+    down = PackedWeight.from_rowmajor(wd.to(DEV))
+    return h.to(DEV).view(1, rows, K), nw.to(DEV), gu, down, expect
+
+
+@pytest.mark.parametrize("rows", [8, 9, 12, 16])
+def test_norm_weight_forms(gpu, rows):
+    """A [1, K] norm weight, a strided one, and autocast around the call."""
+    h, nw, gu, down, expect = _mlp(rows, 320)
+    plain = dispatch._semantic_mlp_epilogue(h, nw, gu, 320, down, EPS)
+    assert_parity(plain[0].cpu(), expect, f"rows={rows}")
+    assert_parity(dispatch._semantic_mlp_epilogue(h, nw.view(1, K), gu, 320, down, EPS)[0].cpu(), expect, "[1, K]")
+    strided = torch.stack((nw, nw), 1)[:, 0]
+    assert_parity(dispatch._semantic_mlp_epilogue(h, strided, gu, 320, down, EPS)[0].cpu(), expect, "strided")
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert_parity(dispatch._semantic_mlp_epilogue(h, nw, gu, 320, down, EPS)[0].cpu(), expect, "autocast")
+    with pytest.raises(ValueError, match="norm_weight"):
+        dispatch._semantic_mlp_epilogue(h, nw.float(), gu, 320, down, EPS)
