@@ -19,9 +19,10 @@ Differences from the reference, on purpose:
     rejected argument always raises.
   - residual adds that follow a projection (:820, :831, :949) are fused into
     that projection's epilogue, with the same bf16 rounding;
-  - for decode and verify rows (M <= 8) the RMSNorm in front of gate_up
-    (:821-827, :941) runs inside the gate_up kernel (kernels.rmsnorm_linear,
-    one bf16 rounding as F.rms_norm); _semantic_input_norm_attention_qkv_vector
+  - for decode and verify rows (M <= 8, up to 16 where that is faster:
+    _norm_gate_up) the RMSNorm in front of gate_up (:821-827, :941) runs inside
+    the gate_up kernel (kernels.rmsnorm_linear, one bf16 rounding as
+    F.rms_norm); _semantic_input_norm_attention_qkv_vector
     offers the same for input_layernorm + QKV (:1255 then :787).
 """
 
@@ -150,15 +151,25 @@ _FUSED_NORM_ROWS = 8
 
 
 def _norm_gate_up(hidden_states, norm_weight, eps, gu_w: PackedWeight):
-    """SiLU(gate)*up of rms_norm(hidden_states): fused into the gate_up kernel
-    for up to 8 rows, a norm kernel in front of it for more (at 12 rows 3.3 +
-    19.7 us, fused 25.2: the norm's arithmetic on 16 rows in every workgroup
-    no longer hides behind the weights).  9..16 rows that the norm kernel does
-    not serve (a [1, K] norm weight, autocast) stay fused: rmsnorm_linear takes
-    every form that it takes for fewer rows, F.rms_norm does not."""
+    """SiLU(gate)*up of rms_norm(hidden_states): fused into the gate_up kernel,
+    or a norm kernel in front of it.
+
+    Up to 8 rows fused, above 16 apart.  Between them by the fused kernel's
+    form: for K = 2560 its workgroups take 32 rows of N, and while they are one
+    round of the CUs (N <= 8192) the norm's arithmetic in each of them hides
+    behind the weights (us at 9 / 12 / 16 rows, fused | apart: N = 2432 8.2 / 8.9
+    / 8.9 | 8.7 / 8.9 / 8.9, 4864 8.9 / 9.5 / 9.7 | 9.5 / 9.6 / 9.8, 8192 11.4 /
+    11.3 / 11.6 | 12.3 / 12.0 / 12.1); in a second round it does not (8704 16.0 /
+    16.7 / 17.9 | 16.0 / 16.1 / 16.5, 19456 24.2 / 25.7 / 27.7 | 21.9 / 22.1 /
+    22.1).  Any other K runs the fused kernel in rounds, slower than two kernels
+    from K = 1024 on (12 rows: 4096 x 1024 9.8 | 7.1, 16384 x 2048 23.8 | 16.7,
+    28672 x 4096 58 | 48; 2048 x 512 4.4 | 5.2).  Calls that the norm kernel does
+    not serve (a [1, K] norm weight, autocast) stay fused up to 16 rows:
+    rmsnorm_linear takes every form that it takes for fewer rows, F.rms_norm
+    does not."""
     rows = hidden_states.numel() // gu_w.k
-    if rows <= _FUSED_NORM_ROWS or (rows <= _lib.DECODE_MAX_M
-                                    and not _rmsnorm_kernel_serves(hidden_states, norm_weight, eps)):
+    apart = rows > _FUSED_NORM_ROWS and (gu_w.n > 8192 if gu_w.k == 2560 else gu_w.k > 512)
+    if rows <= _lib.DECODE_MAX_M and not (apart and _rmsnorm_kernel_serves(hidden_states, norm_weight, eps)):
         return kernels.rmsnorm_linear(hidden_states, norm_weight, eps, gu_w, epilogue=_lib.EPI_SILU_MUL)
     return kernels.linear(qwen_rmsnorm(hidden_states, norm_weight, eps), gu_w, epilogue=_lib.EPI_SILU_MUL)
 

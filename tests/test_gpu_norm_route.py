@@ -41,3 +41,15 @@ def test_norm_weight_forms(gpu, rows):
         assert_parity(dispatch._semantic_mlp_epilogue(h, nw, gu, 320, down, EPS)[0].cpu(), expect, "autocast")
     with pytest.raises(ValueError, match="norm_weight"):
         dispatch._semantic_mlp_epilogue(h, nw.float(), gu, 320, down, EPS)
+
+
+@pytest.mark.parametrize("rows", [9, 12, 16])
+@pytest.mark.parametrize("inter", [1216, 4096, 4128, G.intermediate_size])
+def test_mlp_names(gpu, rows, inter):
+    """Both routes on either side of the width where they meet, through both
+    MLP names (o_proj in front: an identity o_proj adds the attention rows)."""
+    h, nw, gu, down, expect = _mlp(rows, inter)
+    assert_parity(dispatch._semantic_mlp_epilogue(h, nw, gu, inter, down, EPS)[0].cpu(), expect, f"{rows} x {inter}")
+    eye = PackedWeight.from_rowmajor(torch.eye(K, dtype=torch.bfloat16, device=DEV))
+    out = dispatch._semantic_post_attention_mlp(h, torch.zeros_like(h), eye, nw, gu, inter, down, EPS)
+    assert_parity(out[0].cpu(), expect, f"post attention {rows} x {inter}")

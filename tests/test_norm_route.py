@@ -37,3 +37,18 @@ def test_more_rows_take_a_norm_of_their_own(calls):
     hidden = torch.ones(1, 17, 2560, dtype=torch.bfloat16)
     dispatch._norm_gate_up(hidden, torch.ones(2560, dtype=torch.bfloat16), 1e-6, _gate_up(19456, 2560))
     assert calls == ["linear"]
+
+
+@pytest.mark.parametrize("rows,n,k,route", [
+    (8, 19456, 2560, ["fused"]), (9, 2432, 2560, ["fused"]), (16, 8192, 2560, ["fused"]),
+    (9, 8224, 2560, ["norm", "linear"]), (16, 19456, 2560, ["norm", "linear"]), (12, 2048, 512, ["fused"]),
+    (12, 2048, 1024, ["norm", "linear"]), (8, 2048, 1024, ["fused"]), (17, 2432, 2560, ["norm", "linear"]),
+])
+def test_route_by_width(calls, monkeypatch, rows, n, k, route):
+    """9..16 rows that the row kernel serves: fused where the fused kernel was
+    measured faster."""
+    monkeypatch.setattr(dispatch, "_plain_eager", lambda *tensors: True)
+    monkeypatch.setattr(kernels, "_rmsnorm_rows", lambda *a: calls.append("norm"))
+    hidden = torch.ones(rows, k, dtype=torch.bfloat16)
+    dispatch._norm_gate_up(hidden, torch.ones(k, dtype=torch.bfloat16), 1e-6, _gate_up(n, k))
+    assert calls == route
