@@ -33,6 +33,7 @@ import os
 
 import torch
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from . import _lib, kernels
 from .layout import PackedWeight
@@ -44,15 +45,25 @@ from .layout import PackedWeight
 _PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
+def _follows_ops() -> bool:
+    """Whether a torch function mode sees every torch op of this thread.  A
+    default device (torch.set_default_device, with torch.device(...)) is such a
+    mode too, but changes only where new tensors are made by default."""
+    c = torch._C
+    return any(type(c._get_function_stack_at(i)) is not DeviceContext for i in range(c._len_torch_function_stack()))
+
+
 def _plain_eager(*tensors: torch.Tensor) -> bool:
     """Whether a call on these tensors is one that a HIP kernel may stand in
     for: bfloat16 GPU tensors of one device at 16-byte aligned addresses, and
     nothing around the call that follows torch ops one by one (autograd, forward-mode
-    AD, functorch transforms, tracing, compilation, autocast, torch modes)."""
+    AD, functorch transforms, tracing, compilation, autocast, torch modes other
+    than a default device)."""
     device = tensors[0].get_device()  # -1 off the GPU
     c = torch._C
     if (device < 0 or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")
-            or c._get_tracing_state() is not None or c._len_torch_dispatch_stack() or c._len_torch_function_stack()
+            or c._get_tracing_state() is not None or c._len_torch_dispatch_stack()
+            or (c._len_torch_function_stack() and _follows_ops())
             or c._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0):
         return False
     grad = torch.is_grad_enabled()
