@@ -67,7 +67,8 @@ __device__ __forceinline__ u32x4_t buffer_words(const void* base, size_t bytes) 
 // land at lds + 16 l.  In assembly, with no result register, so that the
 // compiler neither counts it nor waits for it before unrelated LDS reads (one
 // ring in one LDS array would otherwise be drained before every read); each
-// use waits for its own data (wait_steps).
+// use waits for its own data (wait_steps).  m0, the LDS address of such a load,
+// is written here and named as clobbered.
 template <bool STREAM>
 __device__ __forceinline__ void dma_1k(u32x4_t rsrc, unsigned voff, unsigned soff, unsigned lds) {
   soff = __builtin_amdgcn_readfirstlane(soff);  // wave-uniform; says so to the compiler
@@ -75,11 +76,11 @@ __device__ __forceinline__ void dma_1k(u32x4_t rsrc, unsigned voff, unsigned sof
   if constexpr (STREAM)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds), "v"(voff),
                  "s"(rsrc), "s"(soff)
-                 : "memory");
+                 : "m0", "memory");
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
                  "s"(rsrc), "s"(soff)
-                 : "memory");
+                 : "m0", "memory");
 }
 
 // Wait until at most `steps` (0..D-1, wave-uniform) steps of NL loads are in
