@@ -404,6 +404,7 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   sum += __shfl_xor(sum, 16);
   sum += __shfl_xor(sum, 32);
   if (g == 0 && c < G) stat[1][wave][c] = sum;
+  wave_lds_order();
 
   // ---- P.V over this wave's groups: lane (g, c) sums rows lb(u) + 4i + g
   // for dims 8c .. 8c+7, then the four row phases g are added as

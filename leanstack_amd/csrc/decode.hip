@@ -304,8 +304,7 @@ __device__ __forceinline__ void accumulate_rows_staged(f32x4_t (&acc)[RBW], cons
   const int g = lane >> 4;
   // Phase p stages k-tiles [kt0(p), kt0(p + 1)) of the wave's slice: M rows
   // of (kt1 - kt0) * 4 chunks of 8 values, NC chunks per lane, in the same
-  // LDS area (a wave's LDS accesses run in order, so a phase's stores follow
-  // the last one's reads).
+  // LDS area: a phase's stores follow the last one's reads.
   auto kt0 = [](int p) { return p * U / PH; };
   bf16x8_t xd[NC];
   auto load_phase = [&](int p) {
@@ -342,6 +341,7 @@ __device__ __forceinline__ void accumulate_rows_staged(f32x4_t (&acc)[RBW], cons
   }
   __builtin_amdgcn_sched_barrier(0);
   store_phase(0);
+  wave_lds_order();
   if constexpr (HALF) {
     const int hi = m >= M && m < 2 * M ? 1 : 0;
     const int row = m < M ? m : (hi ? m - M : M - 1);
@@ -357,7 +357,11 @@ __device__ __forceinline__ void accumulate_rows_staged(f32x4_t (&acc)[RBW], cons
     // queue behind the weight loads, which the first multiplies wait for).
 #pragma unroll
     for (int p = 0; p < PH; ++p) {
-      if (p > 0) store_phase(p);
+      if (p > 0) {
+        wave_lds_order();
+        store_phase(p);
+        wave_lds_order();
+      }
       if (p + 1 < PH) load_phase(p + 1);
 #pragma unroll
       for (int u = kt0(p); u < kt0(p + 1); ++u) {

@@ -842,6 +842,7 @@ __device__ __forceinline__ void store_tile_lds(const f32x16_t (&acc)[A][TB], con
   for (int b0 = 0; b0 < TB; b0 += HB) {
     constexpr int kTileChunks = 32 * C / 16;  // 16-byte chunks of one token tile
     const int tiles = TB - b0 < HB ? TB - b0 : HB;
+    if (b0 > 0) wave_lds_order();
 #pragma unroll
     for (int b = 0; b < HB && b0 + b < TB; ++b)
 #pragma unroll
@@ -869,8 +870,8 @@ __device__ __forceinline__ void store_tile_lds(const f32x16_t (&acc)[A][TB], con
           }
         }
       }
-    // The same wave reads back what it wrote: LDS executes one wave's
-    // accesses in order.
+    // The same wave reads back what it wrote.
+    wave_lds_order();
 #pragma unroll
     for (int i = 0; i < tiles * kTileChunks / 64; ++i) {
       const int k = i * 64 + lane;

@@ -132,6 +132,16 @@ __device__ __forceinline__ float wave_max(float v) {
   return fmaxf(fmaxf(row_lane(v, 0), row_lane(v, 16)), fmaxf(row_lane(v, 32), row_lane(v, 48)));
 }
 
+// What the lanes of a wave stored in LDS before this is what any of them reads
+// after it, and what they read before it is not yet overwritten.  The hardware
+// runs one wave's LDS accesses in issue order; the compiler sees one lane's
+// code and is kept from moving an access across.  No instruction, no wait.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // One projection of a stack program, as the kernel reads it (64 bytes).
 struct StackDesc {
   const bf16x8_t* w;
