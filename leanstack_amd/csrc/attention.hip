@@ -157,57 +157,27 @@ __device__ __forceinline__ void combine_chunks(const AttnArgs& a, __amdgpu_buffe
 // kernels (and 13 launches) at 700 rows.
 enum AttnMode { kHostPos, kDevicePos, kGiven };
 
-// kDevicePos: pos is read from device memory (a.pos_ptr), cos / sin are the whole
-// position tables ([s_max][d/2]), and the chunk size and count follow from
-// pos here; the grid holds the most chunks max_seq_len can need and the
-// workgroups past this pos's count leave at once.  A pos outside
-// [0, s_max) leaves every buffer untouched.
+// One chunk, rows row0 .. row0 + n - 1 of kv head j, of a chunk size that NU
+// 16-row groups per wave cover: prologue items, scores, softmax weights and
+// P.V.  Leaves each wave's P.V and weight sums in part and stat[1] (behind a
+// barrier) and returns the chunk's maximum of head c (lanes c < G).
 template <int G, int NU, AttnMode MODE>
-__global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs args) {
-  static_assert(G >= 1 && G <= 16, "q heads per kv head are the MFMA B columns");
-  constexpr int kGroups = NU;              // 16-row groups per wave
-  constexpr int kMaxChunks = kAttnMaxChunks;
-  AttnArgs a = args;
-  if constexpr (MODE == kDevicePos) {
-    const int pos = *args.pos_ptr;
-    if (pos < 0 || pos >= a.s_max) return;
-    a.pos = pos;
-    a.cos += (size_t)pos * (kHeadDim / 2);
-    a.sin += (size_t)pos * (kHeadDim / 2);
-  }
-  // Rows per chunk (at most 16 kWaves NU: the launch picks NU for the largest chunk
-  // it can meet) and the chunk count, as the host computes them.
-  const int rows = attention_rows_per_chunk(a.pos + 1);
-  a.chunks = (a.pos + rows) / rows;  // ceil((pos + 1) / rows)
-  const int j = blockIdx.x / a.grid_chunks;
-  const int ci = blockIdx.x - j * a.grid_chunks;
-  if (ci >= a.chunks) return;
+__device__ __forceinline__ float attend_chunk(const AttnArgs& a, int j, int row0, int rows, int n,
+                                              __bf16 (&qs)[16][kHeadDim], __bf16 (&kv_new)[2][kHeadDim],
+                                              float (&pw)[kWaves][NU][4][4][G], float (&part)[kWaves][G][kHeadDim],
+                                              float (&stat)[2][kWaves][G]) {
+  constexpr int kGroups = NU;  // 16-row groups per wave
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int g = lane >> 4;
   const int c = lane & 15;
-  const int L = a.pos + 1;
-  const int row0 = ci * rows;
-  const int n = min(rows, L - row0);  // filled rows of the chunk
   // Wave w owns the chunk's 16-row groups w, w + 8, w + 16, ...: group u of
   // the wave starts at chunk row lb(u) = 16 (w + 8u).  Groups past the last
   // row are skipped, so short contexts cost little and the waves share the
   // rows evenly.
   auto lb = [&](int u) { return 16 * (wave + kWaves * u); };
   const bool has_new = MODE != kGiven && a.pos >= row0 && a.pos < row0 + rows;
-  const int cached = MODE == kGiven ? L : a.pos;  // rows read from the caches
-
-  __shared__ __align__(16) __bf16 qs[16][kHeadDim];     // rotated q heads; rows >= G are zero
-  __shared__ __align__(16) __bf16 kv_new[2][kHeadDim];  // this token's rotated k and its v
-  // A wave's softmax weights e^(s - m) of its group u, row 4i + g: [g][i][head]
-  __shared__ __align__(16) float pw[kWaves][kGroups][4][4][G];
-  __shared__ __align__(16) float part[kWaves][G][kHeadDim];
-  __shared__ float stat[2][kWaves][G];                  // each wave's max and sum
-  __shared__ float cmax[kMaxChunks][G];                 // combine: chunk maxima m_c
-  __shared__ float lsum[kMaxChunks][G];                 // combine: e^(m_c - M) l_c
-  __shared__ float wts[kMaxChunks][G];                  // combine: e^(m_c - M)
-  __shared__ int last;
-
+  const int cached = MODE == kGiven ? a.pos + 1 : a.pos;  // rows read from the caches
   // ---- inputs of this wave's prologue items, loaded before the cache rows
   // so that the norms and rotations run while the rows stream in.  Item
   // i = wave + 8u: i < G is q head jG+i, i == G the k head j (only in the
@@ -280,10 +250,9 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
   // defines the row registers in place (they are not used there), or each would
   // be copied, behind a wait, at the join.  Without / with the branch: 4.54 /
   // 4.35 us at 11 rows of a 576-row cache, 7.40 / 7.22 at 300, 9.05 / 9.15 at
-  // 1088, 12.5 / 12.6 at 4001, 20.65 / 20.85 at 16384, 6.2 / 5.25 at one row of
-  // a 16384-row cache.  A second copy of the prologue, or of the kernel, for
-  // waves with rows instead: as fast on its own, 0.2 us slower between other
-  // kernels (instruction fetch).
+  // 1088, 12.5 / 12.6 at 4001, 20.65 / 20.85 at 16384.  A second copy of the
+  // prologue, or of the kernel, for waves with rows instead: as fast on its
+  // own, 0.2 us slower between other kernels (instruction fetch).
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   if (16 * __builtin_amdgcn_readfirstlane(wave) < n) {
 #pragma unroll
@@ -456,6 +425,72 @@ __global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs arg
 #pragma unroll
   for (int q = 0; q < kHalf / 2; ++q) part[wave][(q0 + q) / 8][8 * c + (q0 + q) % 8] = quarter[q];
   __syncthreads();
+  return m;
+}
+
+// attend_chunk for the groups per wave that chunks of `rows` rows take, LO..NU.
+template <int G, int U, int LO, int NU, AttnMode MODE>
+__device__ __forceinline__ float attend_chunk_of(const AttnArgs& a, int j, int row0, int rows, int n,
+                                                 __bf16 (&qs)[16][kHeadDim], __bf16 (&kv_new)[2][kHeadDim],
+                                                 float (&pw)[kWaves][NU][4][4][G], float (&part)[kWaves][G][kHeadDim],
+                                                 float (&stat)[2][kWaves][G]) {
+  if constexpr (U > LO) {
+    if (rows <= 16 * kWaves * (U - 1))
+      return attend_chunk_of<G, U - 1, LO, NU, MODE>(a, j, row0, rows, n, qs, kv_new, pw, part, stat);
+  }
+  return attend_chunk<G, U, MODE>(a, j, row0, rows, n, qs, kv_new,
+                                  reinterpret_cast<float (&)[kWaves][U][4][4][G]>(pw), part, stat);
+}
+
+// kDevicePos: pos is read from device memory (a.pos_ptr), cos / sin are the whole
+// position tables ([s_max][d/2]), and the chunk size and count follow from
+// pos here; the grid holds the most chunks max_seq_len can need and the
+// workgroups past this pos's count leave at once.  A pos outside
+// [0, s_max) leaves every buffer untouched.
+//
+// NU: groups per wave of the largest chunk that the launch can meet.  With the
+// position on the device the chunk may be smaller, and the code for its own
+// size runs (every workgroup of the launch the same; the largest, nearest in
+// memory, first): the code for the largest would issue a load for every row that the chunk does not have, which moves
+// no data but goes through the CU's address path (a 16384-row cache of 8 kv
+// heads of 4 q heads, NU = 4: 7.5 -> 6.4 us at 128 rows, 9.9 -> 8.8 at 700, 10.8
+// -> 9.6 at 1088, 12.1 -> 10.8 at 2000, 13.8 -> 12.7 at 4001).
+template <int G, int NU, AttnMode MODE>
+__global__ __launch_bounds__(kThreads) void decode_attention_kernel(AttnArgs args) {
+  static_assert(G >= 1 && G <= 16, "q heads per kv head are the MFMA B columns");
+  constexpr int kMaxChunks = kAttnMaxChunks;
+  AttnArgs a = args;
+  if constexpr (MODE == kDevicePos) {
+    const int pos = *args.pos_ptr;
+    if (pos < 0 || pos >= a.s_max) return;
+    a.pos = pos;
+    a.cos += (size_t)pos * (kHeadDim / 2);
+    a.sin += (size_t)pos * (kHeadDim / 2);
+  }
+  // Rows per chunk (at most 16 kWaves NU: the launch picks NU for the largest chunk
+  // it can meet) and the chunk count, as the host computes them.
+  const int rows = attention_rows_per_chunk(a.pos + 1);
+  a.chunks = (a.pos + rows) / rows;  // ceil((pos + 1) / rows)
+  const int j = blockIdx.x / a.grid_chunks;
+  const int ci = blockIdx.x - j * a.grid_chunks;
+  if (ci >= a.chunks) return;
+  const int L = a.pos + 1;
+  const int row0 = ci * rows;
+  const int n = min(rows, L - row0);  // filled rows of the chunk
+
+  __shared__ __align__(16) __bf16 qs[16][kHeadDim];     // rotated q heads; rows >= G are zero
+  __shared__ __align__(16) __bf16 kv_new[2][kHeadDim];  // this token's rotated k and its v
+  // A wave's softmax weights e^(s - m) of its group u, row 4i + g: [g][i][head]
+  __shared__ __align__(16) float pw[kWaves][NU][4][4][G];
+  __shared__ __align__(16) float part[kWaves][G][kHeadDim];
+  __shared__ float stat[2][kWaves][G];                  // each wave's max and sum
+  __shared__ float cmax[kMaxChunks][G];                 // combine: chunk maxima m_c
+  __shared__ float lsum[kMaxChunks][G];                 // combine: e^(m_c - M) l_c
+  __shared__ float wts[kMaxChunks][G];                  // combine: e^(m_c - M)
+  __shared__ int last;
+
+  const float m = attend_chunk_of<G, NU, MODE == kDevicePos ? 1 : NU, NU, MODE>(a, j, row0, rows, n, qs, kv_new, pw,
+                                                                           part, stat);
 
   // Sums over the waves, in wave order: the chunk's P.V of head h, dim d, and
   // its sum of weights.
