@@ -7,8 +7,8 @@
 //    128 or 192, K of 128: every Qwen3-4B projection).  Up to 256 tokens x 256,
 //    192 or 128 weight rows x 64 K per stage and workgroup on
 //    v_mfma_f32_32x32x16_bf16: weight fragments from HBM/L2 straight into
-//    registers one to four stages ahead, activations DMA'd into an LDS ring two
-//    to four stages ahead, a counted stage barrier, the epilogue through LDS in
+//    registers one or two stages ahead, activations DMA'd into a three-buffer LDS
+//    ring two stages ahead, a counted stage barrier, the epilogue through LDS in
 //    row order, and, with a workspace, the last partial round split along K
 //    over the idle CUs ("Split-K of the last round" below).
 //  * big::gemm256_kernel, 256 x 256 blocks with both operands staged in LDS,
@@ -483,8 +483,8 @@ hipError_t launch(const void* w, int N, int K, const void* x, int M, int ldx, vo
 // rows the same way; the 192-row blocks keep two waves across N and two across tokens, and
 // there the two waves that share a weight-row half fetch the same lines, the
 // second mostly from L1.
-// Weight fragments and activations are loaded kWAhead and kXAhead stages
-// ahead, into a rotation of register sets and one of LDS buffers; the stage
+// Weight fragments are loaded kWAhead stages ahead into a rotation of register
+// sets, activations kXAhead stages ahead into one of LDS buffers; the stage
 // loop is unrolled by whole turns of both, so neither needs copies.
 namespace wdx {
 
@@ -508,22 +508,21 @@ constexpr int kXStageBytes = kBM<TB, WN> * BK * 2;  // activation fragments of a
 
 // Stages loaded ahead: weights into registers kWAhead stages ahead, activations
 // into LDS kXAhead.  Loads retire in order, so a stage's wait for its
-// activations is also a wait for every weight load issued before them; both
-// run equally far ahead where the weights come from HBM, i.e. where few token
-// blocks share a weight block: 128-row blocks, and 256-row blocks of up to 192
-// tokens.  Against one stage ahead: QKV / o / gate_up + SiLU*up / down at 129
-// tokens 19.8 / 19.4 / 37.6 / 32.9 -> 18.6 / 18.4 / 35.9 / 32.3 us, at 301
-// 23.4 / 21.2 / 47.0 / 36.5 -> 22.5 / 20.5 / 47.0 / 35.7; what is left is the
-// bytes each CU pulls through L2 (55-75 bytes/ns) and the split's exchange.
-// At more tokens the weights are L2 hits and the registers of (2, 8) allow
-// one.
+// activations is also a wait for every weight load issued before them; where
+// the registers allow it both run two stages ahead.  Against weights one stage
+// ahead, QKV / o / gate_up + SiLU*up / down in us at 129 tokens 19.3 / 18.4 / 34.0
+// / 30.0 -> 18.0 / 17.9 / 32.4 / 29.7, at 384 24.8 / 22.2 / 50.2 / 39.3 -> 23.6 /
+// 21.6 / 50.5 / 38.0; at 512 and more tokens up to 2 % for 128-row blocks.
+// Further ahead costs a longer first wait and more buffers: with four stages up
+// to 192 tokens a block and three for 128-row blocks of more, 4096 x 4096 took
+// 31.4 us at 256 tokens and 35.8 at 512 (two: 27.9 and 32.1), 2560 x 2048 19.2
+// at 512 (18.1).  256-row blocks of more than 192 tokens and the 192-row ones
+// have registers for one.
 template <int A, int TB>
-constexpr int kWAhead = A > 2 ? 1 : TB <= 6 ? 4 : A == 1 ? 3 : 1;
-template <int A, int TB>
-constexpr int kXAhead = kWAhead<A, TB> > 2 ? kWAhead<A, TB> : 2;
-constexpr int kMaxBuffers = 5;
+constexpr int kWAhead = A == 1 || (A == 2 && TB <= 6) ? 2 : 1;
+constexpr int kXAhead = 2;
 struct XBuffers {
-  unsigned char* p[kMaxBuffers];
+  unsigned char* p[kXAhead + 1];
 };
 
 using big::f32x16_t;
@@ -632,8 +631,8 @@ __device__ __forceinline__ void sched_step() {
 template <int A, int TB, int WN>
 __device__ __forceinline__ void mainloop(f32x16_t (&acc)[A][TB], const Args& g, const XBuffers& xs, int nb, int mb,
                                          int s0, int s1) {
-  constexpr int P = kWAhead<A, TB>, X = kXAhead<A, TB>;
-  static_assert(X + 1 <= kMaxBuffers && (P == 1 || P == X), "stage order of the loads");
+  constexpr int P = kWAhead<A, TB>, X = kXAhead;
+  static_assert(P == 1 || P == X, "stage order of the loads");
   constexpr int kTokens = kBM<TB, WN>;
   constexpr int ND = kTokens / 32;  // activation DMAs of a stage per wave
   constexpr int kInFlight = (X - 1) * (4 * A + ND);  // loads issued after the next stage's DMA
@@ -740,14 +739,12 @@ __device__ __forceinline__ void mainloop(f32x16_t (&acc)[A][TB], const Args& g, 
   auto run = [&](int s, int count) {
     if (count > 0) stage(s, std::integral_constant<int, 0>{});
     if (count > 1) stage(s + 1, std::integral_constant<int, 1>{});
-    if constexpr (U > 2)
-      if (count > 2) stage(s + 2, std::integral_constant<int, 2>{});
-    if constexpr (U > 3)
+    if (count > 2) stage(s + 2, std::integral_constant<int, 2>{});
+    if constexpr (U > 3) {
       if (count > 3) stage(s + 3, std::integral_constant<int, 3>{});
-    if constexpr (U > 4)
       if (count > 4) stage(s + 4, std::integral_constant<int, 4>{});
-    if constexpr (U > 5)
       if (count > 5) stage(s + 5, std::integral_constant<int, 5>{});
+    }
   };
   int s = s0;
   for (; s + U <= s1; s += U) run(s, U);
@@ -986,15 +983,13 @@ struct Split {
 
 template <int EPI, int A, int TB, int WN>
 __global__ __launch_bounds__(kThreads, 1) void gemm_wdx_kernel(Args g, Split k) {
-  constexpr int kStage = kXStageBytes<TB, WN>, kBuffers = kXAhead<A, TB> + 1;
+  constexpr int kStage = kXStageBytes<TB, WN>;
   // One array per buffer: in one array the compiler could not tell the DMA
   // targets and the fragment reads apart and would drain every load.
   __shared__ __attribute__((aligned(1024))) unsigned char xa[kStage];
   __shared__ __attribute__((aligned(1024))) unsigned char xb[kStage];
   __shared__ __attribute__((aligned(1024))) unsigned char xc[kStage];
-  __shared__ __attribute__((aligned(1024))) unsigned char xd[kBuffers > 3 ? kStage : 16];
-  __shared__ __attribute__((aligned(1024))) unsigned char xe[kBuffers > 4 ? kStage : 16];
-  const XBuffers xs{{xa, xb, xc, xd, xe}};
+  const XBuffers xs{{xa, xb, xc}};
   const int tid = threadIdx.x;
   const int b = blockIdx.x;
   f32x16_t acc[A][TB];
@@ -1007,9 +1002,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wdx_kernel(Args g, Split k) 
     int nb, mb;
     tile_coords(t, g.n_blocks, g.m_blocks, nb, mb);
     mainloop<A, TB, WN>(acc, g, xs, nb, mb, 0, g.KT / 2);
-    // The last stages' activation DMAs (clamped, never read) may still be
-    // writing the buffers and other waves may still read them: both end
-    // before the epilogue reuses them.
+    // DMAs of stages past the last (out of range) may still be in flight and
+    // other waves may still read the buffers: both end before the epilogue
+    // reuses them.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     store_tile_lds<EPI, A, TB, WN>(acc, g, nb, mb, xa, xb);
