@@ -114,13 +114,19 @@ template <int RBW, int MG>
 struct Shape {
   static constexpr int kLoads = 2 * RBW + 2 * MG;  // 1 KB loads per step
   static constexpr int kSlot = kLoads * 1024;
-  static constexpr int kFit = kLdsBytes / (kNW * kSlot);
+  // Workgroups of two row-blocks are what wide N runs in several rounds: half
+  // of the LDS each, so that a CU holds two and the first loads and last sums of
+  // one hide behind the other's stream (SiLU*up 22016 x 1024 at 17 rows 15.0 ->
+  // 11.3 us, plain 24576 x 2560 at 32 rows 11 % less; calls of one round lose
+  // nothing).
+  static constexpr int kWgLds = RBW == 2 && MG <= 4 ? kLdsBytes / 2 : kLdsBytes;
+  static constexpr int kFit = kWgLds / (kNW * kSlot);
   static constexpr int kDepth = kFit < 1 ? 1 : kFit > 4 ? 4 : kFit;  // steps in flight per wave
-  // Where only one step fits (RBW 5 from 6 token groups), the weights of the
-  // step after it still fit beside it, and they are what comes from HBM: a
+  // Where only one step fits (RBW 5 from 6 token groups, RBW 2 at 4), the weights
+  // of the step after it still fit beside it, and they are what comes from HBM: a
   // wave then waits for activations from L2 alone (19456 x 2560 with SiLU*up:
   // 36.0 -> 32.6 us at 128 rows, 29.5 -> 28.8 at 96).
-  static constexpr bool kAhead = kDepth == 1 && kNW * (kSlot + 2 * RBW * 1024) <= kLdsBytes;
+  static constexpr bool kAhead = kDepth == 1 && kNW * (kSlot + 2 * RBW * 1024) <= kWgLds;
   static constexpr int kWaveRing = kDepth * kSlot + (kAhead ? 2 * RBW * 1024 : 0);
   static constexpr int kRing = kNW * kWaveRing;
   // Row-blocks whose partial tiles of all waves fit the ring at once.
@@ -467,16 +473,25 @@ int skinny_groups(int M) {
 // the 128 x 128 GEMM's grid, whose blocks then fill the chip and read each
 // activation fragment once per 128 weight rows instead of once per 32 --
 // except with SiLU*up, where units of 8 outputs give every CU 80 weight rows
-// in one round (19456 x 2560 at 128 rows: 32.6 us, the GEMM 56 us).
+// in one round (19456 x 2560 at 128 rows: 32.6 us, the GEMM 56 us) and the
+// GEMM catches up as N needs more rounds and K leaves fewer steps in each (at
+// 128 rows 22016 x 1024 29 us, the GEMM 25; 28672 x 2048 50 and 46, x 3072 65
+// and 68; 57344 x 2560 95 and 73; at 96 rows 28672 x 2048 41 and 44, 22016 x 1024
+// 24.4 and 23.5, 19456 x 512 12.0 and 13.3).
 //
 // 9..16 rows with SiLU*up too when every CU gets four units or more (N >=
-// 16384; 19.7 us at 12 rows of 19456 x 2560, the decode kernel 22.0); there a
-// call has no workspace.
+// 16384; 19.7 us at 12 rows of 19456 x 2560, the decode kernel 22.0) and K
+// streams for a while (22016 x 512 7.5 us, the decode kernel 6.5; x 1024 11.0 and
+// 11.4); there a call has no workspace.
 bool skinny_route(int M, int N, int K, bool silu) {
   if (M <= 8 || M > kSkinnyMaxM || N % kTileRows != 0 || K % kTileK != 0) return false;
-  if (M <= kDecodeMaxM) return silu && N >= 16384;
+  if (M <= kDecodeMaxM) return silu && N >= 16384 && K >= 1024;
   const bool gemm_grid = N % kGemmBN == 0 && K % kGemmBK == 0;
-  return M <= 64 || !gemm_grid || N < 8192 || silu;
+  if (M <= 64 || !gemm_grid || N < 8192) return true;
+  if (!silu) return false;
+  if (N <= 20480) return N <= 8192 || K >= 768 || (K >= 512 && (M <= 96 || N < 12288));
+  if (N <= 24576) return K >= 2048;
+  return N <= 40960 && K >= (M <= 96 ? 2048 : 3072);
 }
 
 // Row-blocks per workgroup and the K split, from sweeps of (rows, S) over the
@@ -489,7 +504,12 @@ bool skinny_route(int M, int N, int K, bool silu) {
 // CUs by themselves; four (up to 64 rows) when two would take more than one
 // round of the CUs and four still cover half of them.  SiLU*up takes as many
 // units per workgroup as bring them to one round: five for the 1216 units of
-// 19456 rows (21.3 us at 32 rows; four, in two rounds, 28.6).  With a
+// 19456 rows (21.3 us at 32 rows; four, in two rounds, 28.6).  Past one round of
+// fives: two, which overlap (above), up to 32 rows and up to three rounds of
+// them (22016 x 2560: 22.3 us at 17 rows, fives 32.2, fours 28.4; 33 at 64 rows,
+// 42 and 37), else four or five by the rounds they take (28672 x 2560 at 64 rows
+// 38 us in fours, 43 in twos and fives; 40960 48 in fives, 55 in twos).  Two also
+// for 16384 rows at up to 16 tokens (x 2560 at 12 15.9 us, fours 17.0).  With a
 // workspace the K range is split so that the grid comes to about one
 // workgroup per CU, each split keeping at least 16 k-tiles; a second split
 // that leaves the CUs two rounds costs more than it balances (QKV at 64 rows
@@ -499,9 +519,13 @@ SkinnyPlan skinny_plan(int M, int N, int K, bool silu, int cus, bool has_workspa
   const int KT = K / kTileK;
   const int mg = skinny_groups(M);
   int rbw = 2;
-  if (silu) {
-    // units of 8 outputs: as many per workgroup as bring them to one round
-    if (NB > 2 * cus) rbw = mg <= 4 && NB <= 4 * cus ? 4 : 5;
+  if (silu) {  // NB units of 8 outputs
+    auto rounds = [&](int r) { return ((NB + r - 1) / r + cus - 1) / cus; };
+    if (rounds(5) == 1) {
+      if (NB > 2 * cus && (mg > 1 || NB > 4 * cus)) rbw = mg <= 4 && NB <= 4 * cus ? 4 : 5;
+    } else if (mg > 2 && NB > 6 * cus) {
+      rbw = mg <= 4 && 7 * rounds(4) <= 8 * rounds(5) ? 4 : 5;
+    }
   } else if ((mg <= 2 && NB >= cus && NB <= cus + cus / 8) || NB / 2 < 64 || NB % 2 != 0) {
     rbw = 1;
   } else if (mg <= 4 && NB % 4 == 0 && NB / 2 > cus && NB / 4 <= cus && 2 * (NB / 4) >= cus) {
