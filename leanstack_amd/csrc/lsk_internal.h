@@ -28,7 +28,8 @@ constexpr size_t kSkPartialBytes = 256 * 256 * 4;
 constexpr int kSkMaxGrid = (int)((kSkPartialsOffset - kSkFlagsOffset) / 4);
 constexpr unsigned kSkSpinLimit = 1u << 22;
 
-// Projections of kDecodeMaxM < M <= kSkinnyMaxM rows (skinny.hip).
+// Projections of kDecodeMaxM < M <= kSkinnyMaxM rows, from 9 rows on for a wide
+// SiLU*up (skinny.hip).
 constexpr int kSkinnyMaxM = 128;
 constexpr int kSkinnyWaves = 4;
 // Split-K arrival counters live in the prefill workspace's flag words (each
@@ -100,7 +101,7 @@ __device__ __forceinline__ __bf16 rope_half(float a, float b, float c, float s, 
   return static_cast<__bf16>(bf16_round(a * c) + sign * bf16_round(b * s));
 }
 
-// Wave-wide sum / max with the butterfly's pairing (xor 1, 2, 4, 8 inside a
+// Wave-wide sum with the butterfly's pairing (xor 1, 2, 4, 8 inside a
 // 16-lane row, then (r0 + r1) + (r2 + r3) over the rows).  The in-row steps
 // are DPP moves (quad_perm [1,0,3,2], [2,3,0,1], then row_half_mirror and
 // row_mirror: after the quad steps every lane of a quad holds the quad's
@@ -122,14 +123,6 @@ __device__ __forceinline__ float wave_sum(float v) {
   v += dpp<0x141>(v);
   v += dpp<0x140>(v);
   return (row_lane(v, 0) + row_lane(v, 16)) + (row_lane(v, 32) + row_lane(v, 48));
-}
-
-__device__ __forceinline__ float wave_max(float v) {
-  v = fmaxf(v, dpp<0xb1>(v));
-  v = fmaxf(v, dpp<0x4e>(v));
-  v = fmaxf(v, dpp<0x141>(v));
-  v = fmaxf(v, dpp<0x140>(v));
-  return fmaxf(fmaxf(row_lane(v, 0), row_lane(v, 16)), fmaxf(row_lane(v, 32), row_lane(v, 48)));
 }
 
 // What the lanes of a wave stored in LDS before this is what any of them reads
@@ -265,9 +258,10 @@ hipError_t launch_lm_head_argmax(const void* w, int V, int K, const void* x, int
                                  float* logits, int logits_bf16, long long* out_idx,
                                  void* workspace, const void* norm_w, float eps, hipStream_t stream);
 
-// The skinny kernel's plan: `rows` weight rows per workgroup (16, or 32 for a
-// gate/up pair), `groups` = N / rows, each K range split over S workgroups
-// (S > 1 only with a workspace of `bytes` bytes), for a device of `cus` CUs.
+// The skinny kernel's plan: `rows` weight rows per workgroup (16, 32 or 64;
+// SiLU*up, in units of 8 gate and 8 up rows, 32, 64 or 80), `groups` = N / rows
+// rounded up, each K range split over S workgroups (S > 1 only with a workspace
+// of `bytes` bytes), for a device of `cus` CUs.
 struct SkinnyPlan {
   int rows, groups, S;
   size_t bytes;
@@ -276,7 +270,7 @@ int skinny_groups(int M);
 hipError_t current_device_cus(int* cus_out);
 bool skinny_route(int M, int N, int K, bool silu);
 SkinnyPlan skinny_plan(int M, int N, int K, bool silu, int cus, bool has_workspace);
-// y = epilogue(x . W^T) for kDecodeMaxM < M <= kSkinnyMaxM (N % 16 == 0, or
+// y = epilogue(x . W^T) for the M that skinny_route takes (N % 16 == 0, or
 // N % 32 == 0 for SiLU*up; K % 32 == 0).  `workspace` (NULL: no split) must
 // hold skinny_plan(...).bytes bytes, flags zero (every call leaves them zero).
 hipError_t launch_skinny_linear(const void* w, int N, int K, const void* x, int M, int ldx, void* y, int ldy,

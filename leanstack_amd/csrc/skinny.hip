@@ -400,8 +400,10 @@ template <int RBW, int EPI>
 hipError_t launch_rbw(const SkinnyPlan& p, const void* w, const void* x, int ldx, void* y, int ldy,
                       const void* residual, int ldr, int M, int NB, int KT, void* workspace, hipStream_t stream) {
   switch (skinny_groups(M)) {
-    case 1:
-      return launch_cfg<RBW, 1, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
+    case 1:  // 9..16 rows: SiLU*up only, in twos or fives (skinny_route, skinny_plan)
+      if constexpr (EPI == static_cast<int>(Epilogue::kSiluMul) && RBW != 4)
+        return launch_cfg<RBW, 1, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
+      break;
     case 2:
       return launch_cfg<RBW, 2, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
     case 3:
@@ -425,7 +427,9 @@ hipError_t launch_epi(const SkinnyPlan& p, const void* w, const void* x, int ldx
                       const void* residual, int ldr, int M, int NB, int KT, void* workspace, hipStream_t stream) {
   switch (p.rows / kTileRows) {
     case 1:
-      return launch_rbw<1, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
+      if constexpr (EPI != static_cast<int>(Epilogue::kSiluMul))
+        return launch_rbw<1, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
+      break;
     case 2:
       return launch_rbw<2, EPI>(p, w, x, ldx, y, ldy, residual, ldr, M, NB, KT, workspace, stream);
     case 4:
