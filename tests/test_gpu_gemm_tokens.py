@@ -1,7 +1,8 @@
 """The block GEMM at every token tile count (129..256 tokens per block in
 32-token tiles, part-full last blocks) and every remainder of its stage
-rotation, 128- and 256-row blocks, with and without the K split; against the
-oracle's F.linear."""
+rotation, 128- and 256-row blocks, with a workspace (only K >= 1152 splits, 128-row
+blocks in two chunks; other splits: test_gpu_gemm_split_tiles.py) and without;
+against the oracle's F.linear."""
 
 from __future__ import annotations
 
