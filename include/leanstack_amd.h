@@ -110,8 +110,9 @@ int lsk_unpack_bf16(const void* packed_host, int N, int K, int layout_id, void* 
  *   groups, plan[2] = the groups whose K range is split (all or none),
  *   plan[3] = workgroups per group (1: no split).  This is the plan of the
  *   plain and residual epilogues; a SiLU*up call takes units of 8 gate and 8
- *   up rows, runs this kernel up to 128 rows at any N, and may split
- *   differently.
+ *   up rows, may split differently, and runs this kernel also for 9..16 rows
+ *   of N >= 16384 with K >= 1024 and for most shapes of 65..128 rows on the
+ *   GEMM grid (not for short K or N past some 20000..40000).
  *   M > 128: plan[0] = weight rows per output block of the prefill block GEMM
  *   (256, 192 or 128), plan[1] = output blocks, plan[2] = blocks whose K
  *   range is split over several workgroups, plan[3] = workgroups (K chunks)
@@ -120,7 +121,7 @@ int lsk_unpack_bf16(const void* packed_host, int N, int K, int layout_id, void* 
  * kernels (M <= 16, or M > 128 with N or K off every GEMM tile grid), the
  * 256x256 GEMM with both operands staged in LDS (M > 128, N % 256 == 0,
  * K % 64 == 0 but not a shape the block GEMM takes, e.g. K an odd multiple of
- * 64) or the 128x128 GEMM (65 <= M <= 128 with N >= 8192, and the rest of
+ * 64) or the 128x128 GEMM (65 <= M <= 128 with N >= 8192, as above, and the rest of
  * M > 128 with N % 128 == 0, K % 64 == 0).  A workspace smaller than
  * lsk_workspace_bytes(LSK_OP_LINEAR, M, N, K) is refused with
  * LSK_ERR_WORKSPACE, as lsk_linear_bf16 refuses it.  For tests and tuning; no
@@ -136,11 +137,12 @@ int lsk_linear_plan(int M, int N, int K, size_t ws_bytes, int plan[4]);
  *              SILU_MUL (ldy % 4 == 0, 8-byte aligned)
  *   residual   device bf16 [M][N] at stride ldr, RESIDUAL_ADD only (else NULL)
  *   M          >= 1.  M <= 16 runs the decode/verify kernel (weights streamed
- *              once, activations padded to the 16 MFMA columns); 17..128 the
- *              skinny kernel (weights streamed once, activations in groups
- *              of 16 tokens; 65..128 rows of N >= 8192 without SiLU*up the
- *              128x128 GEMM);
- *              larger M the prefill MFMA GEMM.
+ *              once, activations padded to the 16 MFMA columns; 9..16 rows of
+ *              a SiLU*up with N >= 16384 and K >= 1024 the skinny kernel);
+ *              17..128 the skinny kernel (weights streamed once, activations
+ *              in groups of 16 tokens; 65..128 rows of N >= 8192 on the
+ *              128-row grid the 128x128 GEMM, with SiLU*up only for short K
+ *              or N past some 20000..40000); larger M the prefill MFMA GEMM.
  *   workspace  NULL, or lsk_workspace_bytes(LSK_OP_LINEAR, M, N, K) bytes
  *              (0 bytes: no workspace is used), 256-byte aligned, zero-filled
  *              before its first use.  With it, the prefill GEMM splits the K

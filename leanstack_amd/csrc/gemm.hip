@@ -15,7 +15,8 @@
 //    for the M > 128 shapes with N a multiple of 256 that the wdx kernel does
 //    not take (K an odd multiple of 64).
 //  * gemm_linear_kernel, 128 x 128 blocks for the rest of the 128-row grid
-//    (65..128 rows of N >= 8192 without SiLU*up, or N a multiple of 128 with K an odd
+//    (65..128 rows of N >= 8192, with SiLU*up only the shapes that the skinny
+//    kernel leaves: skinny_route; or N a multiple of 128 with K an odd
 //    multiple of 64 that the 256 x 256 kernel cannot take).  Each packed 1 KB weight
 //    tile already is a v_mfma_f32_16x16x32_bf16 operand in lane order, so the
 //    weight half of every LDS stage is a straight linear copy; the activation
@@ -937,9 +938,9 @@ __device__ __forceinline__ void zero(f32x16_t (&acc)[A][TB]) {
 // share lines the same way.  The S workgroups of a split block each store
 // their fp32 accumulators to a workspace slot and count themselves in the
 // block's arrival word; once all S have arrived, workgroup s sums tiles
-// [16s/S, 16(s+1)/S) of the block, its own partial first and then the other
-// S - 1 slots in chunk order, and stores them with the epilogue, then counts itself out; the last one out
-// clears both words.  R*S <= G, and whole-K blocks never wait, so every
+// [s T/S, (s+1) T/S) of the block's T = A TB accumulator tiles, its own partial
+// first and then the other S - 1 slots in chunk order, and stores them with the
+// epilogue, then counts itself out; the last one out clears both words.  R*S <= G, and whole-K blocks never wait, so every
 // split workgroup gets a CU.  That holds only while no other kernel shares
 // the device, so the waits are bounded: a workgroup that gives up (after
 // Split::spin_limit polls) records it in the error word and stores NaN for
@@ -1154,9 +1155,12 @@ inline Args make_args(int bn, const void* w, int N, int K, const void* x, int M,
 // Blocks split and chunks per split block for T blocks of `units` 128-K
 // units on `grid` CUs (R = 0 or S = 1: no split).  S = the most chunks the
 // grid holds (at least 4 units each), rounded down to 4, 8 or 16 when it is
-// 4 or more: each chunk's workgroup then sums an equal share of the block's
-// 16 partial tiles.  Measured at M = 512 / 1024 (QKV S 5 -> 4: 42.6 -> 35.2
-// us; down S 12 -> 8: 52.9 -> 45.2 us; o_proj S 6 -> 4: 45.1 -> 40.6 us).
+// 4 or more: each chunk's workgroup then sums an equal share of the 16 partial
+// tiles of a 256 x 256 block.  Measured on those at M = 512 / 1024 (QKV S 5 -> 4:
+// 42.6 -> 35.2 us; down S 12 -> 8: 52.9 -> 45.2 us; o_proj S 6 -> 4: 45.1 -> 40.6
+// us).  Blocks of fewer tokens or rows hold 5..14 tiles, which these counts
+// share unevenly (five tiles over eight chunks: three chunks sum none); other
+// counts for them are not measured.
 inline void split_plan(int T, int units, int grid, int* R, int* S) {
   *R = grid > 0 ? T % grid : 0;
   *S = 1;

@@ -1,8 +1,8 @@
 // Row kernels between the projections of verify and prefill rows (M > 1) on
 // gfx950, both HBM-bound streams with a little arithmetic per value:
 //
-//  * rms_rows_kernel: the RMSNorm of [M][K] rows in front of a projection of
-//    more than 16 rows (src/leanstack/runtime/qwen_explicit.py:621-628).
+//  * rms_rows_kernel: the RMSNorm of [M][K] rows that no projection computes in
+//    its own prologue (src/leanstack/runtime/qwen_explicit.py:621-628).
 //  * qk_rope_kernel: the q and k heads of the raw QKV rows -- per-head
 //    RMSNorm, rotate-half RoPE and the [T, heads] -> [heads, T] reorder in one
 //    pass (qwen_explicit.py:748-770, RoPE :690-716; :788-806 for one row).

@@ -6,7 +6,7 @@
 // workgroup owns RBW row-blocks (16 output rows each) and all tokens over one
 // K range, which its 4 wavefronts take in 64-K steps in turn.  Each wave DMAs
 // the weight tiles and activation rows of its steps into a ring of its own in
-// LDS, 2-4 steps deep (up to 160 KB in flight per CU, no registers), and
+// LDS, 1-4 steps deep (up to 160 KB in flight per CU, no registers), and
 // multiplies a step on v_mfma_f32_16x16x32_bf16 as it lands: no barrier and no
 // shared stage until the waves' partial tiles are summed through LDS, in wave
 // order.
